@@ -69,7 +69,7 @@ k_cross_fused(const bf16_t* __restrict__ X, const bf16_t* __restrict__ Wq, gk::E
     // ---- the projection: one GEMM tile, parked in LDS as fp32 ----
     const int KT = static_cast<int>(K / gk::BK);
     if (wave >= gk::kConsumers) {
-        gk::produce<4, false>(smem, gk::Operands{X, Wq, M, N, K, ConvGeom{}, K, e.bias}, KT, 1, tiles_m,
+        gk::produce<4>(smem, gk::Operands{X, Wq, M, N, K, K, e.bias}, KT, 1, tiles_m,
                               tiles_n, group_m, wave - gk::kConsumers, lane);
     } else {
         gk::consume<4, 0, gk::EPI_STORE>(smem, e, nullptr, M, N, KT, 1, tiles_m, tiles_n, group_m, wave,

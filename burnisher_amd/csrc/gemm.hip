@@ -44,10 +44,10 @@ namespace {
 #include "gemm_tile.inc"
 using namespace gk;
 
-template <int ACT, int MODE, bool CONV, int MT = kMaxMT, int NT = kNT>
+template <int ACT, int MODE, int MT = kMaxMT, int NT = kNT>
 __global__ void __launch_bounds__(kWgThreads, 1)
 k_gemm_tn(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, bf16_t* out, int64_t M,
-          int64_t N, int64_t K, Epi e, int tiles_m, int tiles_n, int group_m, ConvGeom cv) {
+          int64_t N, int64_t K, Epi e, int tiles_m, int tiles_n, int group_m) {
     __shared__ __attribute__((aligned(1024))) char smem[Geom<MT, NT>::kSmemBytes];
     const int T = tiles_m * tiles_n;
     const int my_tiles = (T - static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x) - 1) /
@@ -64,8 +64,8 @@ k_gemm_tn(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, bf16_t* ou
         out += static_cast<int64_t>(blockIdx.y) * M * e.ld_out * 2;   // float elements
     }
     if (wave >= kConsumers) {
-        produce<MT, CONV, NT>(smem, Operands{A, B, M, N, K, cv, ldk, e.bias}, KT, my_tiles, tiles_m,
-                              tiles_n, group_m, wave - kConsumers, lane);
+        produce<MT, NT>(smem, Operands{A, B, M, N, K, ldk, e.bias}, KT, my_tiles, tiles_m, tiles_n,
+                        group_m, wave - kConsumers, lane);
     } else {
         consume<MT, ACT, MODE, NT>(smem, e, out, M, N, KT, my_tiles, tiles_m, tiles_n, group_m, wave, lane);
     }
@@ -359,9 +359,9 @@ bool aligned(const void* p, int bytes) {
     return (reinterpret_cast<uintptr_t>(p) % bytes) == 0;
 }
 
-template <int ACT, int MODE, bool CONV = false, int MT = kMaxMT, int NT = kNT>
+template <int ACT, int MODE, int MT = kMaxMT, int NT = kNT>
 void launch_tn(const bf16_t* a, const bf16_t* b, bf16_t* out, int64_t m, int64_t n, int64_t k,
-               const Epi& e, hipStream_t s, const ConvGeom& cv = ConvGeom{}) {
+               const Epi& e, hipStream_t s) {
     constexpr int BM = Geom<MT, NT>::BM;
     const int tiles_m = static_cast<int>((m + BM - 1) / BM);
     const int tiles_n = static_cast<int>((n + kBN<NT> - 1) / kBN<NT>);
@@ -371,8 +371,7 @@ void launch_tn(const bf16_t* a, const bf16_t* b, bf16_t* out, int64_t m, int64_t
     // 16 / MT M-tiles (1024 rows; 960 at the 192-row tile) at a time whatever the tile height.
     int grid = min(tiles, device_cus() & ~7);
     if (grid < 8) grid = min(tiles, device_cus());
-    k_gemm_tn<ACT, MODE, CONV, MT, NT><<<grid, kWgThreads, 0, s>>>(a, b, out, m, n, k, e, tiles_m, tiles_n,
-                                                               16 / MT, cv);
+    k_gemm_tn<ACT, MODE, MT, NT><<<grid, kWgThreads, 0, s>>>(a, b, out, m, n, k, e, tiles_m, tiles_n, 16 / MT);
 }
 
 // The tile shape of a GEMM that runs whole (no split-K): the height (64 MT rows) and width (16 NT
@@ -464,8 +463,8 @@ void launch_tn_splitk(const bf16_t* a, const bf16_t* b, float* partial, int64_t 
     e.ld_out = n;
     e.ld_k = k;
     e.vt_dim = 72;
-    k_gemm_tn<0, EPI_F32, false, MT, NT><<<dim3(grid, splits), kWgThreads, 0, s>>>(
-        a, b, reinterpret_cast<bf16_t*>(partial), m, n, k / splits, e, tiles_m, tiles_n, 16 / MT, ConvGeom{});
+    k_gemm_tn<0, EPI_F32, MT, NT><<<dim3(grid, splits), kWgThreads, 0, s>>>(
+        a, b, reinterpret_cast<bf16_t*>(partial), m, n, k / splits, e, tiles_m, tiles_n, 16 / MT);
 }
 
 // The partials of an S-slice split on the tile shape splitk_tile_shape picks for it.
@@ -625,10 +624,10 @@ template <int ACT, int MT, int NT = kNT>
 void launch_tn_mode(int mode, const bf16_t* a, const bf16_t* b, bf16_t* out, int64_t m, int64_t n,
                     int64_t k, const Epi& e, hipStream_t s) {
     switch (mode) {
-        case EPI_STORE: launch_tn<ACT, EPI_STORE, false, MT, NT>(a, b, out, m, n, k, e, s); break;
-        case EPI_ROW_ADD: launch_tn<ACT, EPI_ROW_ADD, false, MT, NT>(a, b, out, m, n, k, e, s); break;
-        case EPI_RESIDUAL: launch_tn<ACT, EPI_RESIDUAL, false, MT, NT>(a, b, out, m, n, k, e, s); break;
-        default: launch_tn<ACT, EPI_GATED, false, MT, NT>(a, b, out, m, n, k, e, s); break;
+        case EPI_STORE: launch_tn<ACT, EPI_STORE, MT, NT>(a, b, out, m, n, k, e, s); break;
+        case EPI_ROW_ADD: launch_tn<ACT, EPI_ROW_ADD, MT, NT>(a, b, out, m, n, k, e, s); break;
+        case EPI_RESIDUAL: launch_tn<ACT, EPI_RESIDUAL, MT, NT>(a, b, out, m, n, k, e, s); break;
+        default: launch_tn<ACT, EPI_GATED, MT, NT>(a, b, out, m, n, k, e, s); break;
     }
 }
 
@@ -766,38 +765,6 @@ void launch_gemm_bf16(const bf16_t* a, const bf16_t* b, const bf16_t* bias, bf16
         default: launch_tn_mt<0>(mt, mode, a, b, out, m, n, k, e, s); break;
     }
     launch_check("gemm (mfma)");
-}
-
-void launch_conv3x3_bf16(const ConvGeom& cv, const bf16_t* wr, const bf16_t* bias, bf16_t* out,
-                         int64_t c_out, const GemmEpilogue& ep, hipStream_t s) {
-    const int64_t m = static_cast<int64_t>(cv.H) * cv.W, k = 9 * static_cast<int64_t>(cv.c_in);
-    if (m == 0 || c_out == 0) return;
-    require(cv.in && cv.zero && wr && out, "conv3x3: null operand");
-    require(cv.c_in % 64 == 0 && cv.c_in > 0, "conv3x3 (mfma): c_in must be a positive multiple of 64");
-    require(c_out % 8 == 0, "conv3x3 (mfma): c_out must be a multiple of 8");
-    require(cv.up ? (cv.in_h * 2 == cv.H && cv.in_w * 2 == cv.W) : (cv.in_h == cv.H && cv.in_w == cv.W),
-            "conv3x3: input and output sizes disagree");
-    require(!ep.vt && !ep.row_add && !ep.gate, "conv3x3: epilogue must be a plain store or a residual add");
-    require(aligned(cv.in, 16) && aligned(cv.zero, 16) && aligned(wr, 16) && aligned(out, 16) &&
-                (!bias || aligned(bias, 16)) && (!ep.residual || aligned(ep.residual, 16)),
-            "conv3x3: operands must be 16-byte aligned");
-    require(static_cast<int64_t>(cv.in_h) * cv.in_w * cv.c_in < (int64_t{1} << 31),
-            "conv3x3: input too large for 32-bit pixel offsets");
-    Epi e{bias, ep.act, ep.round_mid, nullptr, 1, ep.residual, nullptr, 1,
-          ep.ld_out > 0 ? ep.ld_out : c_out, 0, nullptr, 0, 0, 0, 0, 0, 72};
-    require(ep.act == 0, "conv3x3: no activation epilogue (the decoder's SiLU follows a GroupNorm)");
-    ProfileScope ps(K_GEMM, s, 2.0 * static_cast<double>(m) * c_out * k);
-    // The decoder's channel counts are powers of two: 128-wide tiles cover them exactly, where
-    // 144-wide ones would pad every tile row by 16 columns (11% of the MFMAs).
-    const bool narrow = c_out % 128 == 0 && c_out % 144 != 0;
-    if (ep.residual) {
-        if (narrow) launch_tn<0, EPI_RESIDUAL, true, kMaxMT, 8>(cv.in, wr, out, m, c_out, k, e, s, cv);
-        else launch_tn<0, EPI_RESIDUAL, true>(cv.in, wr, out, m, c_out, k, e, s, cv);
-    } else {
-        if (narrow) launch_tn<0, EPI_STORE, true, kMaxMT, 8>(cv.in, wr, out, m, c_out, k, e, s, cv);
-        else launch_tn<0, EPI_STORE, true>(cv.in, wr, out, m, c_out, k, e, s, cv);
-    }
-    launch_check("conv3x3 (mfma)");
 }
 
 int gemm_splitk_choice(int64_t m, int64_t n, int64_t k) {

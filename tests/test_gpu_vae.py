@@ -74,6 +74,25 @@ def test_conv2d_matches_oracle(hip, shape):
     assert np.array_equal(host(again), got), "not byte-identical across two calls"
 
 
+@pytest.mark.parametrize("ci,H,W,co", [(64, 209, 203, 40), (64, 144, 139, 136), (128, 33, 47, 64),
+                                       (192, 3, 1, 264), (64, 1, 70, 8), (128, 17, 16, 24)],
+                         ids=lambda v: str(v))
+def test_conv3x3_patch_shapes_match_oracle(hip, ci, H, W, co):
+    """The implicit-GEMM convolution's patch heights (16, 8 and 4 rows of 16 pixels, by the size of
+    the image) and its 32-channel tile: images that end inside a patch row and a patch column, odd
+    and single-row sizes, one to three channel chunks, ragged channel tiles."""
+    x = randn_bf16(RNG, (1, ci, H, W))
+    w = randn_bf16(RNG, (co, ci, 3, 3), float(1 / np.sqrt(ci * 9)))
+    b = randn_bf16(RNG, (co,), 0.1)
+    want = np.zeros((1, co, H, W), np.uint16)
+    st("stock_conv2d", addr(x), addr(w), addr(b), addr(want), 1, ci, H, W, co, 3, 1, BF16, 0)
+    out = empty((1, co, H, W))
+    dx, dw, db = dev(x), dev(w), dev(b)
+    call("bh_conv2d", dx.data_ptr(), dw.data_ptr(), db.data_ptr(), out.data_ptr(), 1, ci, H, W, co, 3, 1,
+         BF16, None)
+    assert_within(from_bf16(host(out)), from_bf16(want), "gemm", f"conv {ci} {H}x{W} {co}")
+
+
 @pytest.mark.parametrize("case", [(1, 128, 256, 32, True), (2, 512, 64, 32, True), (1, 64, 100, 32, False),
                                   (1, 256, 1024, 32, True)])
 def test_group_norm_matches_oracle(hip, case):
