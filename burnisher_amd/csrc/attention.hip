@@ -462,11 +462,13 @@ struct AttnPlan {
 
 AttnPlan plan_attention(const bf16_t* q, const bf16_t* k, const bf16_t* v, const bf16_t* out,
                         const AttnShape& sh, const void* key_mask, const bf16_t* bias) {
-    // head_dim 512, one head, self-attention, unmasked (the VAE mid-block): its own kernel.
+    // head_dim 512, one head, self-attention, unmasked (the VAE mid-block): its own kernel. Its key
+    // splits are limited to the allocation-free entry point's scratch whatever the entry point, so
+    // both take the same splits and give the same bits.
     if (sh.head_dim == 512 && sh.heads == 1 && sh.q_len == sh.kv_len && !key_mask && !bias &&
         sh.ld_q == 512 && sh.ld_kv == 512 && sh.ld_o == 512 && aligned16(q) && aligned16(k) &&
         aligned16(v) && aligned16(out))
-        return {AttnPlan::FLASH512, 512 * vt512_ld(sh.kv_len)};
+        return {AttnPlan::FLASH512, flash512_scratch_elems(sh.kv_len, flash512_splits(sh.kv_len, kNoAllocScratchBytes))};
     // head_dim 72 (the DiT): V transposed once, then the flash kernel built for that width.
     const bool fast72 = !bias && sh.head_dim == 72 && sh.kv_len <= 16384 && sh.ld_q % 8 == 0 &&
                         sh.ld_kv % 8 == 0 && sh.ld_o % 4 == 0 && aligned16(q) && aligned16(k) &&
@@ -523,9 +525,10 @@ void launch_attention_bf16(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf
     };
     if (plan.kind == AttnPlan::FLASH512) {
         bf16_t* vt = vt_for(plan.vt_elems);
+        const int sp = flash512_splits(sh.q_len, kNoAllocScratchBytes);
         for (int64_t b = 0; b < sh.batch; ++b) {
             const int64_t off = b * sh.q_len * 512;
-            launch_attention512(q + off, k + off, v + off, vt, out + off, sh.q_len, sh.scale, s);
+            launch_attention512(q + off, k + off, v + off, vt, sp, out + off, sh.q_len, sh.scale, s);
         }
         return;
     }

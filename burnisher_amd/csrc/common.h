@@ -306,10 +306,13 @@ std::vector<std::pair<std::string, std::vector<int64_t>>> t5_tensor_shapes(const
 // The VAE decoder's tensors with their checkpoint shapes (vae_engine.cpp).
 std::vector<std::pair<std::string, std::vector<int64_t>>> vae_tensor_shapes(const bh_vae_config& c);
 // Keys per V^T row for the head_dim-512 attention (S rounded up to 32).
-int64_t vt512_ld(int64_t S);
-// Single-head attention at head_dim 512: q, k, v, out [S, 512]; vt is scratch of 512 x vt512_ld(S).
-void launch_attention512(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16_t* vt, bf16_t* out,
-                         int64_t S, float scale, hipStream_t s);
+// Single-head attention at head_dim 512 (flash512.hip): q, k, v, out [S, 512], the keys split over
+// `splits` workgroups per query block; scratch holds flash512_scratch_elems (V^T, then the splits'
+// fp32 partials). flash512_splits chooses the splits that fit beside V^T in `scratch_bytes`.
+int flash512_splits(int64_t S, int64_t scratch_bytes);
+int64_t flash512_scratch_elems(int64_t S, int splits);
+void launch_attention512(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16_t* scratch, int splits,
+                         bf16_t* out, int64_t S, float scale, hipStream_t s);
 
 // bf16 out[m, n] = A[m, k] . B[n, k]^T (+bias) with `ep`. Picks the MFMA tile kernel, the
 // small-M kernel or the reference-order kernel by shape.

@@ -1,6 +1,6 @@
 // Kernels of the VAE decoder (the vae-decode stage, reference src/models/vae_decoder.cpp) on
 // gfx950. The decoder engine (vae_engine.cpp) keeps activations channels-last, [pixels, channels]
-// bf16, so that a 3x3 convolution is an implicit GEMM (gemm.hip, launch_conv3x3_bf16) and the
+// bf16, so that a 3x3 convolution is an implicit GEMM (conv.hip, launch_conv3x3_bf16) and the
 // mid-block attention reads its tokens in place. This file holds what is not a GEMM:
 //   - k_transpose       [R, C] -> [C, R] per batch: NCHW <-> NHWC at the stage's two ends, and
 //                       the reference's TransposeArgs op (ops.h:184-191);
@@ -12,8 +12,8 @@
 //   - k_conv_direct     a convolution in the reference's summation order, for the layers too thin
 //                       for the MFMA tile (conv_in: 4 input channels; conv_out: 3 outputs);
 //   - k_upsample_nchw   the reference's UpsampleArgs op (the engine fuses the upsample into the
-//                       next convolution's gather instead);
-//   - k_vt512, k_flash512  the mid-block's single-head, head_dim-512 attention.
+//                       next convolution's gather instead).
+// The convolutions are in conv.hip, the mid-block's attention in flash512.hip.
 #include "common.h"
 
 #include <algorithm>
@@ -263,187 +263,6 @@ __global__ void __launch_bounds__(256) k_upsample_nchw(const bf16_t* __restrict_
     }
 }
 
-// ---- the mid-block attention: one head, head_dim 512 ------------------------------------------
-//
-// softmax(Q K^T / sqrt(512)) V over S tokens, Q, K, O [S, 512] and V given transposed,
-// vt[d][slot(key)] (keys permuted within 32-key chunks so that the eight keys a lane group holds
-// after a pair of 16x16 score tiles are one 16-byte fragment, see k_vt512; zero past S up to a
-// multiple of 32). A workgroup of four waves owns 64 queries, a wave one
-// 16-query tile; keys stream in blocks of 32 through two LDS stages of 64 KiB (the block's K rows
-// and V^T rows), filled by direct global->LDS loads issued by all four waves after the block
-// barrier. Both products run on v_mfma_f32_16x16x32_bf16 with transposed tiles, as in the
-// head_dim-72 kernel: S^T = K Q^T (K from LDS, Q in registers: 16 fragments), O^T += V^T P^T
-// (V^T from LDS, P in registers as it comes out of the softmax). O^T is 32 16-row tiles: 128
-// accumulator registers per lane.
-//
-// K rows in LDS are 1 KiB (512 dims); 16-byte chunk c of row r sits at c ^ (r & 15), so the 16
-// rows a fragment read touches hit 16 different chunks of one 256-byte span (all 64 banks).
-//
-// Softmax in fp32 with the running maximum in log2 units; it moves only when a block beats it by
-// more than 8 (any fixed reference gives the same normalised result; the bound keeps P below
-// 2^8). P is rounded to bf16 for the MFMA and the denominator sums those rounded values. Keys
-// past S score -inf.
-constexpr int kA5Q = 64;                 // queries per workgroup
-constexpr int kA5Kv = 32;                // keys per block
-constexpr int kA5D = 512;
-constexpr int kA5KBytes = kA5Kv * kA5D * 2;   // 32 KiB
-constexpr int kA5VBytes = kA5D * kA5Kv * 2;   // 32 KiB
-constexpr int kA5Stage = kA5KBytes + kA5VBytes;
-
-struct A5Args {
-    const bf16_t* q;
-    const bf16_t* k;
-    const bf16_t* vt;
-    bf16_t* out;
-    int S;
-    int64_t vt_ld;
-    float c;   // scale * log2(e)
-};
-
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-// One global_load_lds_dwordx4: lane L's 16 bytes at `src` land at LDS address lds + 16 L.
-__device__ __forceinline__ void a5_dma16(const void* src, const char* lds) {
-    const uint32_t l = static_cast<uint32_t>(
-        reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const char*)(lds)));
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                 :
-                 : "s"(l), "v"(src)
-                 : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-__device__ __forceinline__ bf16x8_t a5_frag(const char* p) { return *reinterpret_cast<const bf16x8_t*>(p); }
-
-__device__ __forceinline__ float a5_pair(float v, bool swap32, bool is_max) {
-    const uint32_t x = __float_as_uint(v);
-    const auto r = swap32 ? __builtin_amdgcn_permlane32_swap(x, x, false, false)
-                          : __builtin_amdgcn_permlane16_swap(x, x, false, false);
-    const float a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
-    return is_max ? fmaxf(a, b) : a + b;
-}
-
-// Block j's 64 KiB: pieces 0..31 are K rows (1 KiB each, swizzled), 32..63 V^T rows 16(p-32)..+15
-// (64 bytes each); wave w issues pieces 4i + w.
-__device__ __forceinline__ void a5_dma_block(char* st, const A5Args& a, int j, int wave, int lane) {
-    const int key0 = j * kA5Kv;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int piece = i * 4 + wave;
-        if (piece < 32) {
-            const int key = min(key0 + piece, a.S - 1);
-            const int c = lane ^ (piece & 15);
-            a5_dma16(a.k + static_cast<int64_t>(key) * kA5D + c * 8, st + piece * 1024);
-        } else {
-            const int d = (piece - 32) * 16 + (lane >> 2);
-            a5_dma16(a.vt + static_cast<int64_t>(d) * a.vt_ld + key0 + (lane & 3) * 8,
-                     st + kA5KBytes + (piece - 32) * 1024);
-        }
-    }
-}
-
-__global__ void __launch_bounds__(256, 1) k_flash512(A5Args a) {
-    __shared__ __attribute__((aligned(1024))) char smem[2 * kA5Stage];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lr = lane & 15, hi = lane >> 4;
-    const int q = blockIdx.x * kA5Q + wave * 16 + lr;
-    const int qc = min(q, a.S - 1);
-    bf16x8_t qf[16];
-#pragma unroll
-    for (int ks = 0; ks < 16; ++ks) qf[ks] = a5_frag(reinterpret_cast<const char*>(a.q + static_cast<int64_t>(qc) * kA5D + 32 * ks + 8 * hi));
-    f32x4_t o[32];
-#pragma unroll
-    for (int dt = 0; dt < 32; ++dt) o[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.0f;
-    const int nblk = (a.S + kA5Kv - 1) / kA5Kv;
-    a5_dma_block(smem, a, 0, wave, lane);
-    for (int j = 0; j < nblk; ++j) {
-        // block j has landed (every wave's loads) and nobody still reads the other stage
-        __builtin_amdgcn_sched_barrier(0);
-        asm volatile("" ::: "memory");
-        s_waitcnt<0, 0>();
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
-        if (j + 1 < nblk) a5_dma_block(smem + ((j + 1) & 1) * kA5Stage, a, j + 1, wave, lane);
-        const char* st = smem + (j & 1) * kA5Stage;
-        f32x4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < 16; ++ks) {
-            const int pc = ((4 * ks + hi) ^ lr) * 16;
-            const bf16x8_t k0 = a5_frag(st + lr * 1024 + pc);
-            const bf16x8_t k1 = a5_frag(st + (16 + lr) * 1024 + pc);
-            s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qf[ks], s0, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qf[ks], s1, 0, 0, 0);
-        }
-        // scores in log2 units; keys past S never count
-        const int kb = j * kA5Kv + 4 * hi;
-        float x[8];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            x[t] = kb + t < a.S ? s0[t] * a.c : -INFINITY;
-            x[4 + t] = kb + 16 + t < a.S ? s1[t] * a.c : -INFINITY;
-        }
-        float mx = x[0];
-#pragma unroll
-        for (int t = 1; t < 8; ++t) mx = fmaxf(mx, x[t]);
-        mx = a5_pair(mx, true, true);
-        mx = a5_pair(mx, false, true);
-        if (__any(mx > m + 8.0f)) {
-            const float mn = fmaxf(m, mx);
-            const float alpha = exp2f(m - mn);   // 0 on the first block (m = -inf)
-            m = mn;
-            l *= alpha;
-#pragma unroll
-            for (int dt = 0; dt < 32; ++dt)
-#pragma unroll
-                for (int t = 0; t < 4; ++t) o[dt][t] *= alpha;
-        }
-        bf16x8_t pf;
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const __bf16 pb = static_cast<__bf16>(exp2f(x[t] - m));
-            pf[t] = pb;
-            l += static_cast<float>(pb);
-        }
-#pragma unroll
-        for (int dt = 0; dt < 32; ++dt) {
-            const bf16x8_t vf = a5_frag(st + kA5KBytes + (16 * dt + lr) * 64 + hi * 16);
-            o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, o[dt], 0, 0, 0);
-        }
-    }
-    l = a5_pair(l, true, false);
-    l = a5_pair(l, false, false);
-    if (q >= a.S) return;
-    bf16_t* orow = a.out + static_cast<int64_t>(q) * kA5D + 4 * hi;
-    const float rl = __frcp_rn(l);   // one reciprocal per query, a multiply per output
-#pragma unroll
-    for (int dt = 0; dt < 32; ++dt) {
-        const uint32_t lo = f2bf2(o[dt][0] * rl, o[dt][1] * rl);
-        const uint32_t hi2 = f2bf2(o[dt][2] * rl, o[dt][3] * rl);
-        *reinterpret_cast<uint2*>(orow + 16 * dt) = make_uint2(lo, hi2);
-    }
-}
-
-// V [S, 512] -> vt[d][slot(key)], zero for S <= key < vt_ld. A 32-key x 32-dim tile per block.
-__global__ void __launch_bounds__(256) k_vt512(const bf16_t* __restrict__ v, bf16_t* __restrict__ vt,
-                                               int S, int64_t vt_ld) {
-    __shared__ bf16_t tile[32][33];
-    const int key0 = blockIdx.x * 32, d0 = blockIdx.y * 32;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-#pragma unroll
-    for (int i = ty; i < 32; i += 8) {
-        const int key = key0 + i;
-        tile[i][tx] = key < S ? v[static_cast<int64_t>(key) * kA5D + d0 + tx] : bf16_t{0};
-    }
-    __syncthreads();
-    // storage slot tx of the chunk holds key (tx & 3) | ((tx >> 3) & 3) << 2 | ((tx >> 2) & 1) << 4
-    const int kk = (tx & 3) | (((tx >> 3) & 3) << 2) | (((tx >> 2) & 1) << 4);
-#pragma unroll
-    for (int i = ty; i < 32; i += 8) vt[static_cast<int64_t>(d0 + i) * vt_ld + key0 + tx] = tile[kk][i];
-}
-
 int grid_for(int64_t n, int per_block) {
     return static_cast<int>(std::min<int64_t>((n + per_block - 1) / per_block, 65535LL * 16));
 }
@@ -686,24 +505,6 @@ void launch_upsample_nchw(const bf16_t* in, bf16_t* out, int64_t planes, int64_t
     ProfileScope ps(K_ELEMENTWISE, s, 2.0 * static_cast<double>(n + planes * H * W));
     k_upsample_nchw<<<grid_for(n, 256), 256, 0, s>>>(in, out, planes, H, W, f);
     launch_check("upsample");
-}
-
-int64_t vt512_ld(int64_t S) { return (S + 31) / 32 * 32; }
-
-void launch_attention512(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16_t* vt, bf16_t* out,
-                         int64_t S, float scale, hipStream_t s) {
-    require(S > 0 && S < (int64_t{1} << 30), "attention (head_dim 512): sequence length");
-    const int64_t ld = vt512_ld(S);
-    {
-        ProfileScope ps(K_ELEMENTWISE, s, 4.0 * static_cast<double>(S) * kA5D);
-        k_vt512<<<dim3(static_cast<unsigned>(ld / 32), kA5D / 32), 256, 0, s>>>(v, vt, static_cast<int>(S), ld);
-        launch_check("attention (head_dim 512): V transpose");
-    }
-    A5Args a{q, k, vt, out, static_cast<int>(S), ld,
-             (scale > 0.0f ? scale : 1.0f / std::sqrt(static_cast<float>(kA5D))) * 1.4426950408889634f};
-    ProfileScope ps(K_ATTN_SELF, s, 4.0 * static_cast<double>(S) * S * kA5D);
-    k_flash512<<<static_cast<unsigned>((S + kA5Q - 1) / kA5Q), 256, 0, s>>>(a);
-    launch_check("attention (head_dim 512)");
 }
 
 }  // namespace bh

@@ -38,7 +38,8 @@ struct bh_vae {
     std::vector<void*> allocs;
     bf16_t* buf[4] = {nullptr, nullptr, nullptr, nullptr};
     int64_t buf_elems = 0;
-    bf16_t *q = nullptr, *k = nullptr, *v = nullptr, *vt = nullptr, *o = nullptr;
+    bf16_t *q = nullptr, *k = nullptr, *v = nullptr, *o = nullptr;
+    int attn_splits = 1;   // key splits of the mid-block attention at width 512
     bf16_t* zero = nullptr;
     bf16_t* conv_out_bias = nullptr;   // decoder.conv_out.bias padded to 8 outputs
     bh::GroupNormScratch gn;
@@ -217,7 +218,9 @@ struct Run {
         give(normed);
         const float scale = 1.0f / std::sqrt(static_cast<float>(ch));
         if (ch == 512) {
-            launch_attention512(e.q, e.k, e.v, e.vt, e.o, S, scale, s);
+            bf16_t* scratch = take();   // V^T and the key splits' partials, in a free activation buffer
+            launch_attention512(e.q, e.k, e.v, scratch, e.attn_splits, e.o, S, scale, s);
+            give(scratch);
         } else {
             AttnShape sh{1, 1, S, S, ch, ch, ch, ch, scale};
             if (ch <= 128) launch_attention_bf16(e.q, e.k, e.v, e.o, sh, nullptr, false, s);
@@ -336,6 +339,10 @@ int bh_vae_create(const bh_vae_config* cfg, const bh_vae_weights* w, int64_t lat
             }
         }
         most = std::max(most, h * h * 3);
+        if (p.rev[0] == 512) {   // the attention's scratch is an activation buffer
+            most = std::max(most, bh::flash512_scratch_elems(latent_hw * latent_hw, 1));
+            e->attn_splits = bh::flash512_splits(latent_hw * latent_hw, most * 2);
+        }
         e->buf_elems = most;
         for (auto& b : e->buf) b = static_cast<bf16_t*>(e->alloc(most * 2));
         const int64_t S = latent_hw * latent_hw, ch = p.rev[0];
@@ -343,7 +350,6 @@ int bh_vae_create(const bh_vae_config* cfg, const bh_vae_weights* w, int64_t lat
         e->k = static_cast<bf16_t*>(e->alloc(S * ch * 2));
         e->v = static_cast<bf16_t*>(e->alloc(S * ch * 2));
         e->o = static_cast<bf16_t*>(e->alloc(S * ch * 2));
-        e->vt = static_cast<bf16_t*>(e->alloc(ch * bh::vt512_ld(S) * 2));
         e->zero = static_cast<bf16_t*>(e->alloc(256));
         e->gn.max_chunks = 2048;
         e->gn.part = static_cast<double*>(e->alloc(e->gn.max_chunks * 64 * 8));

@@ -143,6 +143,22 @@ def test_attention_head_dim_512_matches_oracle(hip, S):
     assert_within(from_bf16(host(out)), from_bf16(want), "attention", f"head_dim 512 S={S}")
 
 
+@pytest.mark.parametrize("S,spread", [(1, 1.0), (33, 8.0), (128, 8.0), (129, 1.0), (1055, 8.0), (2048, 1.0)])
+def test_attention_head_dim_512_splits_and_rescales(hip, S, spread):
+    """One key to 64 blocks of 32: a single block, ragged last blocks and query blocks, key splits
+    (from a few hundred tokens on), and scores spread wide enough (standard deviation 8) that the
+    running maximum moves in most blocks and splits carry very different maxima."""
+    q, k, v = (randn_bf16(RNG, (1, S, 1, 512), sc) for sc in (spread, 1.0, 1.0))
+    want = np.zeros_like(q)
+    st("stock_attention", addr(q), addr(k), addr(v), addr(want), 1, 1, S, S, 512, 0.0, None, None, F32,
+       BF16, 0, 0)
+    out = empty((1, S, 1, 512))
+    dq, dk, dv = dev(q), dev(k), dev(v)
+    call("bh_attention", dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), out.data_ptr(), 1, 1,
+         S, S, 512, 0.0, None, None, F32, BF16, None)
+    assert_within(from_bf16(host(out)), from_bf16(want), "attention", f"head_dim 512 S={S} spread {spread}")
+
+
 def decode(wl):
     import burnisher_amd as bh
     tensors, latent = wl.to_device()
