@@ -258,26 +258,31 @@ struct ConvGeom {
     int c_in = 0;
     int up = 0;
 };
+// With `stats` it also writes, for every run of four output channels, conv3x3_stats_rows pairs (sum,
+// sum of squares) in fp64 over disjoint sets of the stored pixels: stats[(run * rows + r) * 2 + {0, 1}].
+// 0 rows: the shape has no such sums.
+int64_t conv3x3_stats_rows(const ConvGeom& cv, int64_t c_out);
 void launch_conv3x3_bf16(const ConvGeom& cv, const bf16_t* wr, const bf16_t* bias, bf16_t* out,
-                         int64_t c_out, const GemmEpilogue& ep, hipStream_t s);
+                         int64_t c_out, const GemmEpilogue& ep, hipStream_t s, double* stats = nullptr);
 
 // ---- the VAE decoder's kernels (vae.hip) ----
 // [batch][R][C] -> [batch][C][R], bf16.
 void launch_transpose_bf16(const bf16_t* in, bf16_t* out, int64_t batch, int64_t R, int64_t C,
                            hipStream_t s);
-// Device scratch of a channels-last GroupNorm: per-chunk fp64 partials and the group statistics.
+// Device scratch of a GroupNorm: fp64 partial sums and the group statistics.
 struct GroupNormScratch {
-    double* part = nullptr;   // max_chunks * 64
+    double* part = nullptr;   // 2 * 64 * max_chunks, or what conv3x3_stats_rows asks for
     double* mean = nullptr;   // 64
     float* inv = nullptr;     // 64
     int64_t max_chunks = 0;
 };
 bool gn_nhwc_supported(int64_t C, int64_t G);
 // GroupNorm over x [S, C] (channels-last, batch 1), G groups of C/G channels, then optionally
-// SiLU; each rounded to bf16 as the reference stores them. out may alias x.
+// SiLU; each rounded to bf16 as the reference stores them. out may alias x. stats_rows > 0: sc.part
+// already holds x's sums as launch_conv3x3_bf16 writes them (C/G a multiple of four).
 void launch_group_norm_nhwc(const bf16_t* x, bf16_t* out, int64_t S, int64_t C, int64_t G,
                             float eps, const bf16_t* w, const bf16_t* b, bool silu,
-                            GroupNormScratch& sc, hipStream_t s);
+                            GroupNormScratch& sc, hipStream_t s, int64_t stats_rows = 0);
 // Stride-1 "same" convolution, channels-last, w in the checkpoint layout [co][ci][k][k], in the
 // reference's summation order (bit-identical with it).
 void launch_conv_direct_nhwc(const bf16_t* x, const bf16_t* w, const bf16_t* bias, bf16_t* out,
@@ -305,7 +310,6 @@ void launch_group_norm_nchw(const bf16_t* x, const bf16_t* w, const bf16_t* b, b
 std::vector<std::pair<std::string, std::vector<int64_t>>> t5_tensor_shapes(const bh_t5_config& c);
 // The VAE decoder's tensors with their checkpoint shapes (vae_engine.cpp).
 std::vector<std::pair<std::string, std::vector<int64_t>>> vae_tensor_shapes(const bh_vae_config& c);
-// Keys per V^T row for the head_dim-512 attention (S rounded up to 32).
 // Single-head attention at head_dim 512 (flash512.hip): q, k, v, out [S, 512], the keys split over
 // `splits` workgroups per query block; scratch holds flash512_scratch_elems (V^T, then the splits'
 // fp32 partials). flash512_splits chooses the splits that fit beside V^T in `scratch_bytes`.

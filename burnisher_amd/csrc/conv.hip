@@ -90,6 +90,8 @@ struct ConvArgs {
     int H, W, in_w, c_in, up;
     int c_out;
     int tiles_x, tiles_n, tiles;   // patches per row, channel tiles, all tiles
+    double* stats;         // or null: see wave_stats
+    int64_t stats_rows;
 };
 
 // Tile v -> patch origin and first channel. Workgroup b runs on XCD b % 8, so tiles are renumbered
@@ -274,14 +276,35 @@ __device__ __forceinline__ void conv_step(f32x4_t (&acc)[MT][NT], bf16x8_t (&a0)
     }
 }
 
+// Sums of the stored outputs for the GroupNorm that follows: for each run of four channels, the sum
+// and the sum of squares in fp64 over a wave's pixels of it, at
+// stats[(channel / 4) * stats_rows + row] with row = patch * waves + wave. Both are sums of exactly
+// converted bf16 values (a square has 16 significant bits), so neither loses a bit that matters at
+// any image size. The sixteen pixels of a patch row are sixteen neighbouring lanes, summed with
+// rotations within them. Costs ~1.2 us per 256 x 128 tile; a pass over the output costs 14 us at
+// 128 channels of 512 x 512 (54 at 1024 x 1024) and two launches.
+__device__ __forceinline__ double row16_sum(double v) {
+#define BH_ROR(N)                                                                                  \
+    {                                                                                              \
+        const uint64_t b = __builtin_bit_cast(uint64_t, v);                                        \
+        const uint32_t lo = __builtin_amdgcn_mov_dpp(static_cast<int>(b), 0x120 + N, 0xf, 0xf, false);       \
+        const uint32_t hi = __builtin_amdgcn_mov_dpp(static_cast<int>(b >> 32), 0x120 + N, 0xf, 0xf, false); \
+        v += __builtin_bit_cast(double, static_cast<uint64_t>(hi) << 32 | lo);                     \
+    }
+    BH_ROR(8) BH_ROR(4) BH_ROR(2) BH_ROR(1)
+#undef BH_ROR
+    return v;
+}
+
 // A wave's MW x 16 pixels by 16 NW channels, from image row y0 and channel n0: bias, then the
 // residual add (the sum rounded first where the reference stores it), one rounding. A lane holds 8
 // consecutive channels of one pixel of each row per 32 channels. The residual's loads are issued
 // before the stores: a load behind a store waits for that store's acknowledgement. Rows are addressed by
 // a scalar base and one 32-bit lane offset.
-template <int MW, int MODE, int NW>
+template <int MW, int MODE, int NW, bool STATS>
 __device__ __forceinline__ void conv_epilogue(const f32x4_t (&acc)[MW][NW], const ConvArgs& a, const Epi& e,
-                                              int y0, int x0, int n0, int lane, const bf16_t* bl) {
+                                              int y0, int x0, int n0, int lane, const bf16_t* bl,
+                                              int64_t stats_row) {
     constexpr int kP = NW / 2;
     const int lr = lane & 15, hi = lane >> 4;
     const bool xok = x0 + lr < a.W;
@@ -304,6 +327,7 @@ __device__ __forceinline__ void conv_epilogue(const f32x4_t (&acc)[MW][NW], cons
         if (n0 + 32 * p + 8 * hi >= a.c_out) break;
         float bias[8];
         bias_or_neg_zero(e, e.bias ? ld_raw<8>(bl + 32 * p + 8 * hi) : uint4{}, bias);
+        double sum[2] = {0.0, 0.0}, sq[2] = {0.0, 0.0};
 #pragma unroll
         for (int i = 0; i < MW; ++i) {
             if (y0 + i >= a.H || !xok) continue;
@@ -315,12 +339,33 @@ __device__ __forceinline__ void conv_epilogue(const f32x4_t (&acc)[MW][NW], cons
 #pragma unroll
                 for (int q = 0; q < 8; ++q) v[q] = __fadd_rn(t[q], e.round_mid ? round_bf16(v[q]) : v[q]);
             }
-            *reinterpret_cast<uint4*>(a.out + base + i * row + 32 * p + lo) = pack8(v);
+            const uint4 packed = pack8(v);
+            *reinterpret_cast<uint4*>(a.out + base + i * row + 32 * p + lo) = packed;
+            if (STATS) {
+                unpack8(packed, v);
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    const double x = static_cast<double>(v[q]);
+                    sum[q >> 2] += x;
+                    sq[q >> 2] = __builtin_fma(x, x, sq[q >> 2]);
+                }
+            }
+        }
+        if (STATS) {   // a lane's sixteen neighbours share its channels, so none has left the loop
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const double s1 = row16_sum(sum[h]), s2 = row16_sum(sq[h]);
+                double* to = a.stats + ((static_cast<int64_t>(n0 + 32 * p + 8 * hi) / 4 + h) * a.stats_rows + stats_row) * 2;
+                if (lr == 0) {
+                    to[0] = s1;
+                    to[1] = s2;
+                }
+            }
         }
     }
 }
 
-template <int MT, int MODE, int NT>
+template <int MT, int MODE, int NT, bool STATS>
 __device__ __forceinline__ void conv_consume(char* smem, const ConvArgs& a, const Epi& e, int my_tiles,
                                              int wave, int lane) {
     using G = Halo<MT, NT>;
@@ -367,12 +412,15 @@ __device__ __forceinline__ void conv_consume(char* smem, const ConvArgs& a, cons
         int y0, x0, n0;
         conv_tile<MT, NT>(a, blockIdx.x + it * gridDim.x, y0, x0, n0);
         const char* slot = smem + G::kBiasOff + (it % G::kBiasSlots) * kBiasSlotBytes;
-        conv_epilogue<MW, MODE, NW>(acc, a, e, y0 + MW * wm, x0, n0 + 16 * NW * wn, lane,
-                                    reinterpret_cast<const bf16_t*>(slot) + 16 * NW * wn);
+        constexpr int kWM = 4 / G::WN;
+        const int64_t patch_index = static_cast<int64_t>(y0 / G::PY) * a.tiles_x + x0 / 16;
+        conv_epilogue<MW, MODE, NW, STATS>(acc, a, e, y0 + MW * wm, x0, n0 + 16 * NW * wn, lane,
+                                           reinterpret_cast<const bf16_t*>(slot) + 16 * NW * wn,
+                                           patch_index * kWM + wm);
     }
 }
 
-template <int MT, int MODE, int NT>
+template <int MT, int MODE, int NT, bool STATS>
 __global__ void __launch_bounds__(kWgThreads, 1) k_conv3x3(ConvArgs a, Epi e) {
     __shared__ __attribute__((aligned(1024))) char smem[Halo<MT, NT>::kSmemBytes];
     const int my_tiles = (a.tiles - static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x) - 1) /
@@ -380,7 +428,7 @@ __global__ void __launch_bounds__(kWgThreads, 1) k_conv3x3(ConvArgs a, Epi e) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (wave >= kConsumers) conv_produce<MT, NT>(smem, a, e.bias, my_tiles, wave - kConsumers, lane);
-    else conv_consume<MT, MODE, NT>(smem, a, e, my_tiles, wave, lane);
+    else conv_consume<MT, MODE, NT, STATS>(smem, a, e, my_tiles, wave, lane);
 }
 
 int device_cus() {
@@ -401,14 +449,22 @@ int device_cus() {
 int patches(const ConvGeom& cv, int mt) { return ((cv.H + 4 * mt - 1) / (4 * mt)) * ((cv.W + 15) / 16); }
 
 template <int MT, int MODE, int NT>
-void launch_conv(const ConvGeom& cv, const bf16_t* w, bf16_t* out, int64_t c_out, const Epi& e, hipStream_t s) {
-    ConvArgs a{cv.in, cv.zero, w, out, cv.H, cv.W, cv.in_w, cv.c_in, cv.up, static_cast<int>(c_out), 0, 0, 0};
+void launch_conv(const ConvGeom& cv, const bf16_t* w, bf16_t* out, int64_t c_out, const Epi& e, double* stats,
+                 hipStream_t s) {
+    ConvArgs a{cv.in, cv.zero, w, out, cv.H, cv.W, cv.in_w, cv.c_in, cv.up, static_cast<int>(c_out), 0, 0, 0,
+               stats, static_cast<int64_t>(patches(cv, MT)) * (4 / Halo<MT, NT>::WN)};
     a.tiles_x = (cv.W + 15) / 16;
     a.tiles_n = static_cast<int>((c_out + 16 * NT - 1) / (16 * NT));
     a.tiles = patches(cv, MT) * a.tiles_n;
     int grid = min(a.tiles, device_cus() & ~7);
     if (grid < 8) grid = min(a.tiles, device_cus());
-    k_conv3x3<MT, MODE, NT><<<grid, kWgThreads, 0, s>>>(a, e);
+    if constexpr (NT == 8) {
+        if (stats) {
+            k_conv3x3<MT, MODE, NT, true><<<grid, kWgThreads, 0, s>>>(a, e);
+            return;
+        }
+    }
+    k_conv3x3<MT, MODE, NT, false><<<grid, kWgThreads, 0, s>>>(a, e);
 }
 
 // The patch height: the least estimated time, rounds of tiles over the CUs times a step's cycles.
@@ -432,15 +488,15 @@ int conv_rows(const ConvGeom& cv, int64_t c_out) {
 
 template <int MODE>
 void launch_conv_mode(const ConvGeom& cv, const bf16_t* w, bf16_t* out, int64_t c_out, const Epi& e,
-                      hipStream_t s) {
+                      double* stats, hipStream_t s) {
     if (c_out <= 32) {   // the decoder's conv_out: one 32-wide tile column
-        launch_conv<4, MODE, 2>(cv, w, out, c_out, e, s);
+        launch_conv<4, MODE, 2>(cv, w, out, c_out, e, nullptr, s);
         return;
     }
     switch (conv_rows(cv, c_out)) {
-        case 1: launch_conv<1, MODE, 8>(cv, w, out, c_out, e, s); break;
-        case 2: launch_conv<2, MODE, 8>(cv, w, out, c_out, e, s); break;
-        default: launch_conv<4, MODE, 8>(cv, w, out, c_out, e, s); break;
+        case 1: launch_conv<1, MODE, 8>(cv, w, out, c_out, e, stats, s); break;
+        case 2: launch_conv<2, MODE, 8>(cv, w, out, c_out, e, stats, s); break;
+        default: launch_conv<4, MODE, 8>(cv, w, out, c_out, e, stats, s); break;
     }
 }
 
@@ -448,8 +504,17 @@ bool aligned(const void* p, int bytes) { return (reinterpret_cast<uintptr_t>(p) 
 
 }  // namespace
 
+int64_t conv3x3_stats_rows(const ConvGeom& cv, int64_t c_out) {
+    if (c_out <= 32) return 0;
+    switch (conv_rows(cv, c_out)) {
+        case 1: return static_cast<int64_t>(patches(cv, 1)) * (4 / Halo<1, 8>::WN);
+        case 2: return static_cast<int64_t>(patches(cv, 2)) * (4 / Halo<2, 8>::WN);
+        default: return static_cast<int64_t>(patches(cv, 4)) * (4 / Halo<4, 8>::WN);
+    }
+}
+
 void launch_conv3x3_bf16(const ConvGeom& cv, const bf16_t* wr, const bf16_t* bias, bf16_t* out,
-                         int64_t c_out, const GemmEpilogue& ep, hipStream_t s) {
+                         int64_t c_out, const GemmEpilogue& ep, hipStream_t s, double* stats) {
     const int64_t m = static_cast<int64_t>(cv.H) * cv.W, k = 9 * static_cast<int64_t>(cv.c_in);
     if (m == 0 || c_out == 0) return;
     require(cv.in && cv.zero && wr && out, "conv3x3: null operand");
@@ -467,8 +532,9 @@ void launch_conv3x3_bf16(const ConvGeom& cv, const bf16_t* wr, const bf16_t* bia
           ep.ld_out > 0 ? ep.ld_out : c_out, 0, nullptr, 0, 0, 0, 0, 0, 72};
     require(ep.act == 0, "conv3x3: no activation epilogue (the decoder's SiLU follows a GroupNorm)");
     ProfileScope ps(K_GEMM, s, 2.0 * static_cast<double>(m) * c_out * k);
-    if (ep.residual) launch_conv_mode<EPI_RESIDUAL>(cv, wr, out, c_out, e, s);
-    else launch_conv_mode<EPI_STORE>(cv, wr, out, c_out, e, s);
+    require(!stats || conv3x3_stats_rows(cv, c_out) > 0, "conv3x3: this shape sums no statistics");
+    if (ep.residual) launch_conv_mode<EPI_RESIDUAL>(cv, wr, out, c_out, e, stats, s);
+    else launch_conv_mode<EPI_STORE>(cv, wr, out, c_out, e, stats, s);
     launch_check("conv3x3 (mfma)");
 }
 

@@ -4,9 +4,9 @@
 // mid-block attention reads its tokens in place. This file holds what is not a GEMM:
 //   - k_transpose       [R, C] -> [C, R] per batch: NCHW <-> NHWC at the stage's two ends, and
 //                       the reference's TransposeArgs op (ops.h:184-191);
-//   - GroupNorm         two deterministic fp64 passes (sum, then squared deviations) over
-//                       per-chunk partials, then one pass that normalises, applies the affine
-//                       and, optionally, SiLU (the reference's norm then activation, each rounded
+//   - GroupNorm         fp64 sums and sums of squares in a fixed order (from the convolution that
+//                       wrote the tensor, or one pass over it), then one pass that normalises,
+//                       applies the affine and, optionally, SiLU (the reference's norm then activation, each rounded
 //                       to bf16 as the reference stores them, ops_cpu.cpp:186-224, 265-274; the
 //                       SiLU with the hardware exp2 and reciprocal, within one bf16 ulp);
 //   - k_conv_direct     a convolution in the reference's summation order, for the layers too thin
@@ -48,77 +48,88 @@ __global__ void __launch_bounds__(256) k_transpose(const bf16_t* __restrict__ in
 
 // ---- GroupNorm over [pixels, C] --------------------------------------------------------------
 //
+// One pass sums x and x^2 in fp64; the group's mean and variance follow from the two sums. A bf16
+// value's square is exact in fp64 and both sums lose nothing that matters (they are exact up to 2^37
+// times the smallest square), so the only cancellation is in the variance, n * sum(x^2) - sum(x)^2,
+// which is formed in twice the precision: it equals the two-pass form's for any mean. Bound by
+// reading x once (the two-pass form read it twice: 1.6 ms of a 1024px decode).
+//
 // A workgroup owns a chunk of pixels; thread t holds channel octet t % (C/8) of pixels
-// t / (C/8), t / (C/8) + 256/(C/8), ... and sums its eight channels in fp64; the workgroup then
-// sums each group's channels and rows in a fixed order into part[chunk][group]. Pass 0 sums x,
-// pass 1 sums (x - mean[group])^2. Sums of bf16 values in fp64 are exact up to 2^45 times the
-// smallest term's ulp, so the group mean does not depend on the order; the squared deviations
-// round at the last fp64 bit, far below the float they are converted to.
+// t / (C/8), t / (C/8) + 256/(C/8), ...; the workgroup then sums each group's channels and rows in a
+// fixed order into part[group][chunk].
 constexpr int kGnThreads = 256;
 
-__global__ void __launch_bounds__(kGnThreads) k_gn_partial(const bf16_t* __restrict__ x, int64_t S,
-                                                         int C, int G, int64_t px_per_chunk,
-                                                         const double* __restrict__ mean,
-                                                         double* __restrict__ part) {
-    __shared__ double red[kGnThreads][9];
+__global__ void __launch_bounds__(kGnThreads) k_gn_stats(const bf16_t* __restrict__ x, int64_t S, int C, int G,
+                                                       int64_t px_per_chunk, double* __restrict__ part) {
+    __shared__ double red[kGnThreads][17];
     const int oct = C / 8, per_row = kGnThreads / oct;   // C/8 divides 256 (checked by the host)
     const int t = threadIdx.x, o = t % oct, prow = t / oct;
     const int cpg = C / G;
     const int64_t p0 = static_cast<int64_t>(blockIdx.x) * px_per_chunk;
     const int64_t p1 = min(S, p0 + px_per_chunk);
-    double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    double mu[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) mu[q] = mean ? mean[(o * 8 + q) / cpg] : 0.0;
+    double sum[8] = {0, 0, 0, 0, 0, 0, 0, 0}, sq[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (int64_t p = p0 + prow; p < p1; p += per_row) {
         const uint4 raw = *reinterpret_cast<const uint4*>(x + p * C + o * 8);
         const uint32_t w4[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            const float v = __uint_as_float(q & 1 ? (w4[q >> 1] & 0xffff0000u) : (w4[q >> 1] << 16));
-            if (mean) {
-                const double d = static_cast<double>(v) - mu[q];
-                acc[q] += d * d;
-            } else {
-                acc[q] += static_cast<double>(v);
-            }
+            const double v = __uint_as_float(q & 1 ? (w4[q >> 1] & 0xffff0000u) : (w4[q >> 1] << 16));
+            sum[q] += v;
+            sq[q] = __builtin_fma(v, v, sq[q]);
         }
     }
 #pragma unroll
-    for (int q = 0; q < 8; ++q) red[t][q] = acc[q];
+    for (int q = 0; q < 8; ++q) {
+        red[t][q] = sum[q];
+        red[t][8 + q] = sq[q];
+    }
     __syncthreads();
-    if (t < G) {
+    if (t < 2 * G) {
+        const int g = t >> 1, h = (t & 1) * 8;
         double s = 0.0;
         for (int r = 0; r < per_row; ++r)
-            for (int c = t * cpg; c < (t + 1) * cpg; ++c) s += red[r * oct + c / 8][c % 8];
-        part[static_cast<int64_t>(blockIdx.x) * G + t] = s;
+            for (int c = g * cpg; c < (g + 1) * cpg; ++c) s += red[r * oct + c / 8][h + c % 8];
+        part[(static_cast<int64_t>(g) * gridDim.x + blockIdx.x) * 2 + (t & 1)] = s;
     }
 }
 
-// Pass 0: mean[g] = sum / n. Pass 1: var = sum / n, inv[g] = 1 / sqrt(float(var) + eps), the
-// reference's rounding (ops_cpu.cpp:208-210). One workgroup per group: thread t sums chunks t,
-// t + 256, ... in order, then a fixed pairwise tree over the 256 threads, so the result is the same
-// on every run.
-__global__ void __launch_bounds__(256) k_gn_finalize(const double* __restrict__ part, int chunks, int G,
-                                                     double n, int pass, float eps,
-                                                     double* __restrict__ mean, float* __restrict__ inv) {
-    __shared__ double red[256];
+// Group g's statistics from its `count` pairs at part[g * count]: mean = s1 / n, var = (n s2 - s1^2) /
+// n^2, inv = 1 / sqrt(float(var) + eps), the reference's rounding (ops_cpu.cpp:208-210). One workgroup
+// per group, summed in a fixed order.
+constexpr int kGnFinThreads = 512;
+
+__global__ void __launch_bounds__(kGnFinThreads) k_gn_finalize(const double* __restrict__ part, int64_t count,
+                                                              double n, float eps, double* __restrict__ mean,
+                                                              float* __restrict__ inv) {
+#pragma clang fp contract(off)
+    __shared__ double red[2][kGnFinThreads];
     const int g = blockIdx.x, t = threadIdx.x;
-    double s = 0.0;
-    for (int c = t; c < chunks; c += 256) s += part[static_cast<int64_t>(c) * G + g];
-    red[t] = s;
+    const double2* src = reinterpret_cast<const double2*>(part) + g * count;
+    double a = 0.0, b = 0.0;
+#pragma unroll 4
+    for (int64_t c = t; c < count; c += kGnFinThreads) {
+        const double2 v = src[c];
+        a += v.x;
+        b += v.y;
+    }
+    red[0][t] = a;
+    red[1][t] = b;
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (t < w) red[t] += red[t + w];
+    for (int w = kGnFinThreads / 2; w > 0; w >>= 1) {
+        if (t < w) {
+            red[0][t] += red[0][t + w];
+            red[1][t] += red[1][t + w];
+        }
         __syncthreads();
     }
     if (t != 0) return;
-    if (pass == 0) {
-        mean[g] = red[0] / n;
-    } else {
-        const double var = red[0] / n;
-        inv[g] = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(static_cast<float>(var), eps)));
-    }
+    const double s1 = red[0][0], s2 = red[1][0];
+    // n s2 - s1^2 with each product as a rounded value and its exact remainder
+    const double p = n * s2, q = s1 * s1;
+    const double num = (p - q) + (__builtin_fma(n, s2, -p) - __builtin_fma(s1, s1, -q));
+    const double var = num <= 0.0 ? 0.0 : num / (n * n);   // a NaN stays one
+    mean[g] = s1 / n;
+    inv[g] = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(static_cast<float>(var), eps)));
 }
 
 // SiLU with the hardware exp2 and reciprocal: a few fp32 ulps from x / (1 + exp(-x)), which moves
@@ -305,10 +316,10 @@ void* op_workspace(int slot, size_t bytes) {
 GroupNormScratch op_gn_scratch() {
     GroupNormScratch sc;
     sc.max_chunks = 2048;
-    char* base = static_cast<char*>(op_workspace(SLOT_GN, 2048 * 64 * 8 + 64 * 8 + 64 * 4));
+    char* base = static_cast<char*>(op_workspace(SLOT_GN, 2048 * 64 * 16 + 64 * 8 + 64 * 4));
     sc.part = reinterpret_cast<double*>(base);
-    sc.mean = reinterpret_cast<double*>(base + 2048 * 64 * 8);
-    sc.inv = reinterpret_cast<float*>(base + 2048 * 64 * 8 + 64 * 8);
+    sc.mean = reinterpret_cast<double*>(base + 2048 * 64 * 16);
+    sc.inv = reinterpret_cast<float*>(base + 2048 * 64 * 16 + 64 * 8);
     return sc;
 }
 
@@ -446,17 +457,19 @@ bool gn_nhwc_supported(int64_t C, int64_t G) {
 
 void launch_group_norm_nhwc(const bf16_t* x, bf16_t* out, int64_t S, int64_t C, int64_t G,
                             float eps, const bf16_t* w, const bf16_t* b, bool silu,
-                            GroupNormScratch& sc, hipStream_t s) {
+                            GroupNormScratch& sc, hipStream_t s, int64_t stats_rows) {
     require(gn_nhwc_supported(C, G), "groupnorm (nhwc): unsupported channel / group count");
-    const int chunks = static_cast<int>(std::min<int64_t>(sc.max_chunks, std::max<int64_t>(1, (S + 15) / 16)));
-    const int64_t per = (S + chunks - 1) / chunks;
+    require(stats_rows == 0 || (C / G) % 4 == 0, "groupnorm (nhwc): sums come by runs of four channels");
     const int ci = static_cast<int>(C), gi = static_cast<int>(G);
     const double n = static_cast<double>(S) * (C / G);
     ProfileScope ps(K_NORM, s, 4.0 * static_cast<double>(S * C));
-    k_gn_partial<<<chunks, kGnThreads, 0, s>>>(x, S, ci, gi, per, nullptr, sc.part);
-    k_gn_finalize<<<gi, 256, 0, s>>>(sc.part, chunks, gi, n, 0, eps, sc.mean, sc.inv);
-    k_gn_partial<<<chunks, kGnThreads, 0, s>>>(x, S, ci, gi, per, sc.mean, sc.part);
-    k_gn_finalize<<<gi, 256, 0, s>>>(sc.part, chunks, gi, n, 1, eps, sc.mean, sc.inv);
+    int64_t count = stats_rows * (C / G / 4);
+    if (count == 0) {
+        const int chunks = static_cast<int>(std::min<int64_t>(sc.max_chunks, std::max<int64_t>(1, (S + 15) / 16)));
+        k_gn_stats<<<chunks, kGnThreads, 0, s>>>(x, S, ci, gi, (S + chunks - 1) / chunks, sc.part);
+        count = chunks;
+    }
+    k_gn_finalize<<<gi, kGnFinThreads, 0, s>>>(sc.part, count, n, eps, sc.mean, sc.inv);
     const int blocks = grid_for(S * (C / 8), 256);
 #define BH_GN_APPLY(W_, B_, S_) \
     k_gn_apply<W_, B_, S_><<<blocks, 256, 0, s>>>(x, out, S, ci, gi, sc.mean, sc.inv, w, b)

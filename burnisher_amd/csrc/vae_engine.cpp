@@ -43,6 +43,7 @@ struct bh_vae {
     bf16_t* zero = nullptr;
     bf16_t* conv_out_bias = nullptr;   // decoder.conv_out.bias padded to 8 outputs
     bh::GroupNormScratch gn;
+    int64_t gn_part_bytes = 0;
     int64_t bytes = 0;
 
     ~bh_vae() {
@@ -148,9 +149,24 @@ struct Run {
             if (e.buf[i] == p) free_mask |= 1 << i;
     }
 
+    // The tensor whose sums the last convolution left in e.gn.part (null: none), and their rows.
+    const bf16_t* summed = nullptr;
+    int64_t sum_rows = 0;
+
     void gn(const bf16_t* x, bf16_t* out, const std::string& n, int64_t ch, int64_t h, bool silu) {
         launch_group_norm_nhwc(x, out, h * h, ch, e.cfg.norm_num_groups, static_cast<float>(e.cfg.eps),
-                               e.at(n + ".weight"), e.at(n + ".bias"), silu, e.gn, s);
+                               e.at(n + ".weight"), e.at(n + ".bias"), silu, e.gn, s, x == summed ? sum_rows : 0);
+        if (x != summed || out == x) summed = nullptr;   // e.gn.part or the tensor has changed
+    }
+
+    // A convolution whose output a GroupNorm reads next, with its sums where the widths allow.
+    void conv_summed(const ConvGeom& g, const bf16_t* w, const bf16_t* bias, bf16_t* out, int64_t co,
+                     const GemmEpilogue& ep) {
+        const int64_t rows = (co / e.cfg.norm_num_groups) % 4 == 0 ? conv3x3_stats_rows(g, co) : 0;
+        const bool fits = rows > 0 && rows * (co / 4) * 16 <= e.gn_part_bytes;
+        launch_conv3x3_bf16(g, w, bias, out, co, ep, s, fits ? e.gn.part : nullptr);
+        summed = fits ? out : nullptr;
+        sum_rows = fits ? rows : 0;
     }
 
     // 3x3 "same" conv of x (h_in x h_in, ci) to out (h x h, co); up: h = 2 h_in, nearest.
@@ -168,7 +184,7 @@ struct Run {
             GemmEpilogue ep;
             ep.residual = residual;
             ep.round_mid = residual != nullptr;
-            launch_conv3x3_bf16(g, e.rw.at(n + ".weight"), e.at(n + ".bias"), out, co, ep, s);
+            conv_summed(g, e.rw.at(n + ".weight"), e.at(n + ".bias"), out, co, ep);
             return;
         }
         require(!up && !residual, "vae: a thin convolution cannot be an upsampler or carry a residual");
@@ -182,6 +198,7 @@ struct Run {
         GemmEpilogue ep;
         ep.residual = residual;
         ep.round_mid = residual != nullptr;
+        if (out == summed) summed = nullptr;
         launch_gemm_bf16(x, e.at(n + ".weight"), e.at(n + ".bias"), out, rows, co, ci, ep, s);
     }
 
@@ -251,8 +268,8 @@ struct Run {
             g.zero = e.zero;
             g.H = g.W = g.in_h = g.in_w = static_cast<int>(h);
             g.c_in = 64;
-            launch_conv3x3_bf16(g, e.rw.at("decoder.conv_in.weight"), e.at("decoder.conv_in.bias"), b,
-                                p.rev[0], GemmEpilogue{}, s);
+            conv_summed(g, e.rw.at("decoder.conv_in.weight"), e.at("decoder.conv_in.bias"), b, p.rev[0],
+                        GemmEpilogue{});
         }
         std::swap(a, b);
         give(b);
@@ -352,7 +369,20 @@ int bh_vae_create(const bh_vae_config* cfg, const bh_vae_weights* w, int64_t lat
         e->o = static_cast<bf16_t*>(e->alloc(S * ch * 2));
         e->zero = static_cast<bf16_t*>(e->alloc(256));
         e->gn.max_chunks = 2048;
-        e->gn.part = static_cast<double*>(e->alloc(e->gn.max_chunks * 64 * 8));
+        {   // sums: the standalone pass's, or those of the convolution with the most
+            int64_t bytes = e->gn.max_chunks * 64 * 16, side = latent_hw;
+            for (size_t i = 0; i < p.rev.size(); ++i) {
+                bh::ConvGeom g;
+                g.H = g.W = static_cast<int>(side);
+                bytes = std::max(bytes, bh::conv3x3_stats_rows(g, p.rev[i]) * (p.rev[i] / 4) * 16);
+                if (i + 1 == p.rev.size()) break;
+                side *= 2;
+                g.H = g.W = static_cast<int>(side);   // the upsampler's output, and the next block's
+                bytes = std::max(bytes, bh::conv3x3_stats_rows(g, p.rev[i]) * (p.rev[i] / 4) * 16);
+            }
+            e->gn.part = static_cast<double*>(e->alloc(bytes));
+            e->gn_part_bytes = bytes;
+        }
         e->gn.mean = static_cast<double*>(e->alloc(64 * 8));
         e->gn.inv = static_cast<float*>(e->alloc(64 * 4));
         // repack every 3x3 weight the MFMA conv reads

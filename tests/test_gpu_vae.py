@@ -111,6 +111,36 @@ def test_group_norm_matches_oracle(hip, case):
     assert_within(from_bf16(host(out)), from_bf16(want), "norm", f"groupnorm {case}")
 
 
+@pytest.mark.parametrize("case", ["constant", "offset", "one_outlier", "inf", "nan"])
+def test_group_norm_statistics_edges(hip, case):
+    """The one-pass statistics (sums of x and x^2) where they could cancel or spread: a constant
+    group (variance 0), a mean 200 times the deviation, one huge value, an infinity, a NaN (their
+    groups become NaN, the others keep their values)."""
+    C, S, G = 128, 300, 32
+    x = from_bf16(randn_bf16(RNG, (C, S), 1.0)).astype(np.float32)
+    if case == "constant":
+        x[4:8] = 3.140625
+    elif case == "offset":
+        x = x * 0.5 + 100.0
+    elif case == "one_outlier":
+        x[9, 17] = 3.0e4
+    elif case == "inf":
+        x[12, 3] = np.inf
+    else:
+        x[20, 200] = np.nan
+    from helpers import to_bf16
+    bits = to_bf16(x).reshape(1, C * S)
+    want = np.zeros_like(bits)
+    st("stock_group_norm", addr(bits), None, None, addr(want), 1, C * S, 1e-6, G, C, BF16, 0)
+    out = empty((1, C * S))
+    dx = dev(bits)
+    call("bh_norm", dx.data_ptr(), None, None, out.data_ptr(), 1, C * S, 1e-6, 0, G, C, BF16, None)
+    got, ref = from_bf16(host(out)), from_bf16(want)
+    assert np.array_equal(np.isnan(got), np.isnan(ref)), case
+    ok = ~np.isnan(ref)
+    assert_within(got[ok], ref[ok], "norm", f"groupnorm {case}")
+
+
 def test_upsample_and_transpose_match_oracle(hip):
     x = randn_bf16(RNG, (2, 5, 6, 7))
     want = np.zeros((2, 5, 12, 14), np.uint16)
@@ -200,8 +230,10 @@ def check_decode(got, want, where):
 
 @pytest.mark.parametrize("cfg,latent_hw", [(SDXL_VAE, 8),
                                            (dict(SDXL_VAE, block_out_channels=(64, 128, 128, 128),
-                                                 layers_per_block=1), 6)],
-                         ids=["sdxl_widths_8", "narrow_6"])
+                                                 layers_per_block=1), 6),
+                                           (dict(SDXL_VAE, block_out_channels=(128, 128), layers_per_block=0), 104),
+                                           (dict(SDXL_VAE, block_out_channels=(128, 256), layers_per_block=0), 71)],
+                         ids=["sdxl_widths_8", "narrow_6", "patch16_104", "patch8_71"])
 def test_vae_decoder_matches_oracle(hip, cfg, latent_hw):
     wl = make_vae_workload(cfg, latent_hw=latent_hw, seed=5)
     check_decode(decode(wl), oracle_decode(wl), f"{cfg['block_out_channels']} latent {latent_hw}")
