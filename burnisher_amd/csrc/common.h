@@ -246,6 +246,55 @@ struct GemmEpilogue {
     int64_t splitk_ws_floats = 0;
 };
 
+// A channel of a GroupNorm: its group's mean and 1 / sqrt(var + eps), and its own affine.
+struct alignas(16) NormChannel {
+    float mean, inv, w, b;
+};
+
+// SiLU with the hardware exp2 and reciprocal: a few fp32 ulps from x / (1 + exp(-x)), which moves
+// the bf16 value it is rounded to by at most one ulp (the same bound as a device expf).
+__device__ __forceinline__ float silu_hw(float x) {
+    return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x));
+}
+
+// Eight values of eight channels normalised and rounded to bf16: (x - mean) * inv, * w, + b, each
+// operation rounded (the reference's order).
+__device__ __forceinline__ uint4 norm8(const uint4& raw, const NormChannel (&c)[8]) {
+    const uint32_t in[4] = {raw.x, raw.y, raw.z, raw.w};
+    uint32_t out[4];
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+        float v[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const NormChannel& n = c[2 * h + k];
+            const float x = __uint_as_float(k ? (in[h] & 0xffff0000u) : (in[h] << 16));
+            v[k] = __fadd_rn(__fmul_rn(__fmul_rn(__fsub_rn(x, n.mean), n.inv), n.w), n.b);
+        }
+        out[h] = f2bf2(v[0], v[1]);
+    }
+    return make_uint4(out[0], out[1], out[2], out[3]);
+}
+// The decoder's form, GroupNorm then SiLU, each rounded to bf16: (x - mean) * (inv * w) + b with one
+// rounding of the product and sum (two fewer than norm8, and two instructions) and the hardware
+// SiLU. `c` from norm_silu_channel.
+__device__ __forceinline__ NormChannel norm_silu_channel(NormChannel c) {
+    c.inv *= c.w;
+    return c;
+}
+__device__ __forceinline__ uint4 norm_silu8(const uint4& raw, const NormChannel (&c)[8]) {
+    const uint32_t in[4] = {raw.x, raw.y, raw.z, raw.w};
+    uint32_t out[4];
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+        const NormChannel &p = c[2 * h], &q = c[2 * h + 1];
+        const uint32_t r = f2bf2(__builtin_fmaf(__uint_as_float(in[h] << 16) - p.mean, p.inv, p.b),
+                                 __builtin_fmaf(__uint_as_float(in[h] & 0xffff0000u) - q.mean, q.inv, q.b));
+        out[h] = f2bf2(silu_hw(__uint_as_float(r << 16)), silu_hw(__uint_as_float(r & 0xffff0000u)));
+    }
+    return make_uint4(out[0], out[1], out[2], out[3]);
+}
+
 // A 3x3, stride-1, pad-1 convolution read as a GEMM (batch 1, NHWC): out[H*W, c_out] =
 // im2col(in)[H*W, 9*c_in] . W[c_out, 9*c_in]^T with W repacked [c_out][ky][kx][c_in]. With `up`
 // the input is in_h x in_w = H/2 x W/2 and upsampled 2x (nearest) on the fly. `zero` points at
@@ -258,31 +307,36 @@ struct ConvGeom {
     int c_in = 0;
     int up = 0;
 };
-// With `stats` it also writes, for every run of four output channels, conv3x3_stats_rows pairs (sum,
+// With `norm` the input is normalised on the way in: every value becomes norm_silu8's of its channel,
+// as launch_group_norm_apply would have stored it. With `stats` it also writes, for every run of four output channels, conv3x3_stats_rows pairs (sum,
 // sum of squares) in fp64 over disjoint sets of the stored pixels: stats[(run * rows + r) * 2 + {0, 1}].
 // 0 rows: the shape has no such sums.
 int64_t conv3x3_stats_rows(const ConvGeom& cv, int64_t c_out);
 void launch_conv3x3_bf16(const ConvGeom& cv, const bf16_t* wr, const bf16_t* bias, bf16_t* out,
-                         int64_t c_out, const GemmEpilogue& ep, hipStream_t s, double* stats = nullptr);
+                         int64_t c_out, const GemmEpilogue& ep, hipStream_t s, double* stats = nullptr,
+                         const NormChannel* norm = nullptr);
 
 // ---- the VAE decoder's kernels (vae.hip) ----
 // [batch][R][C] -> [batch][C][R], bf16.
 void launch_transpose_bf16(const bf16_t* in, bf16_t* out, int64_t batch, int64_t R, int64_t C,
                            hipStream_t s);
-// Device scratch of a GroupNorm: fp64 partial sums and the group statistics.
+// Device scratch of a GroupNorm: fp64 partial sums and the channels' statistics and affine.
 struct GroupNormScratch {
-    double* part = nullptr;   // 2 * 64 * max_chunks, or what conv3x3_stats_rows asks for
-    double* mean = nullptr;   // 64
-    float* inv = nullptr;     // 64
+    double* part = nullptr;           // 2 * 64 * max_chunks, or what conv3x3_stats_rows asks for
+    NormChannel* channels = nullptr;  // 2048 (the widest supported norm)
     int64_t max_chunks = 0;
 };
 bool gn_nhwc_supported(int64_t C, int64_t G);
-// GroupNorm over x [S, C] (channels-last, batch 1), G groups of C/G channels, then optionally
-// SiLU; each rounded to bf16 as the reference stores them. out may alias x. stats_rows > 0: sc.part
-// already holds x's sums as launch_conv3x3_bf16 writes them (C/G a multiple of four).
-void launch_group_norm_nhwc(const bf16_t* x, bf16_t* out, int64_t S, int64_t C, int64_t G,
-                            float eps, const bf16_t* w, const bf16_t* b, bool silu,
-                            GroupNormScratch& sc, hipStream_t s, int64_t stats_rows = 0);
+// The statistics of x [S, C] (channels-last, batch 1) over G groups of C/G channels with the affine
+// (null: 1 and 0) into sc.channels. stats_rows > 0: sc.part already holds x's sums as
+// launch_conv3x3_bf16 writes them (C/G a multiple of four).
+void launch_group_norm_channels(const bf16_t* x, int64_t S, int64_t C, int64_t G, float eps,
+                                const bf16_t* w, const bf16_t* b, GroupNormScratch& sc, hipStream_t s,
+                                int64_t stats_rows = 0);
+// The GroupNorm of x with them, then optionally SiLU, each rounded to bf16 as the reference stores
+// it. out may alias x.
+void launch_group_norm_apply(const bf16_t* x, bf16_t* out, int64_t S, int64_t C, bool silu,
+                             const GroupNormScratch& sc, hipStream_t s);
 // Stride-1 "same" convolution, channels-last, w in the checkpoint layout [co][ci][k][k], in the
 // reference's summation order (bit-identical with it).
 void launch_conv_direct_nhwc(const bf16_t* x, const bf16_t* w, const bf16_t* bias, bf16_t* out,

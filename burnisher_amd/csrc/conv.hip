@@ -23,6 +23,15 @@
 // patch row, whatever the tap, so they cover all 64 banks once and the swizzle of a lane depends on
 // (lane, kx) only.
 //
+// With NORM the convolution reads the raw tensor and applies its GroupNorm and SiLU itself: each
+// producer wave normalises the patch rows it loaded, in LDS, as soon as they have landed, so the
+// normalised tensor is never written to or read from memory. A pixel is normalised once per patch
+// and chunk (1.27 times on average, once per 128 output channels) on waves that otherwise only issue
+// loads, under the consumers' MFMAs; the ~10 vector instructions per value take issue slots from
+// them (512 -> 512 at 128 x 128: 57 -> 75 us with the raw tensor read in place of the normalised
+// one), less than the pass they replace as a whole: decode at 512px 3.32 -> 2.84 ms, at 1024px
+// 11.95 -> 10.44 ms (interleaved A/B).
+//
 // Measured against the per-tap gather it replaces (256 x 128 tiles, three 48 KiB stages): 512 ->
 // 512 channels at 128 x 128 pixels 74.5 -> 56.7 us (1036 -> 1364 TFLOP/s); 128 -> 128 at
 // 512 x 512 (18 steps a tile) 83.5 -> 64 us; 512 -> 512 at 64 x 64 (64 tiles there, 256 here)
@@ -42,9 +51,9 @@ using namespace gk;
 constexpr int kPW = 18;                 // patch row: 16 output pixels and the border
 constexpr int kPRow = kPW * kRowBytes;  // its bytes in LDS
 
-constexpr int cmin(int a, int b) { return a < b ? a : b; }
+__host__ __device__ constexpr int cmin(int a, int b) { return a < b ? a : b; }
 
-template <int MT, int NT>
+template <int MT, int NT, bool NORM = false>
 struct Halo {
     static constexpr int PY = 4 * MT;                          // output rows of a patch
     // The consumers as WM x WN: each reads WM-th of the patch rows' and WN-th of the weights'
@@ -58,19 +67,25 @@ struct Halo {
     static constexpr int kBBlocks = 2 * NT;
     static constexpr int kBBytes = kBBlocks * 1024;
     static constexpr int kBiasSlots = 4;
-    // weight stages, after two patch buffers and the bias slots
-    static constexpr int S = cmin(8, (160 * 1024 - 2 * kABytes - kBiasSlots * kBiasSlotBytes) / kBBytes);
+    static constexpr int kNormBytes = NORM ? 1024 : 0;         // a chunk's 64 channels of NormChannel
+    // weight stages, after two patch buffers, the bias slots and the channels' norm
+    static constexpr int S = cmin(8, (160 * 1024 - 2 * kABytes - kBiasSlots * kBiasSlotBytes - 2 * kNormBytes) / kBBytes);
     static constexpr int D = S - 1;                            // steps the weights are issued ahead
     static constexpr int kBOff = 2 * kABytes;
     static constexpr int kBiasOff = kBOff + S * kBBytes;
-    static constexpr int kSmemBytes = kBiasOff + kBiasSlots * kBiasSlotBytes;
+    static constexpr int kNormOff = kBiasOff + kBiasSlots * kBiasSlotBytes;
+    static constexpr int kDumpOff = kNormOff + kNormBytes;     // where items past the patch's end go
+    static constexpr int kSmemBytes = kDumpOff + kNormBytes;
     static constexpr int kBItems = (kBBlocks + 3) / 4;         // DMA instructions per wave and step
     static constexpr int kAItems = (kABlocks + 3) / 4;         // per wave and chunk
     // The next chunk's patch goes out in the first kASteps taps of a chunk, kAPer items a tap:
     // before (in issue order) the weights of that chunk's first step, which go out at tap 9 - D.
-    static constexpr int kAPer = (kAItems + (10 - D) - 1) / (10 - D);
+    // Items of tap t have landed at the barrier of tap t + D - 1; normalised there, they must be
+    // complete at the barrier of tap 8, when the consumers read ahead into the next chunk.
+    static constexpr int kTaps = 9 - D;
+    static constexpr int kAPer = (kAItems + kTaps - 1) / kTaps;
     static constexpr int kASteps = (kAItems + kAPer - 1) / kAPer;
-    static_assert(S >= 3 && kASteps <= 10 - D && kSmemBytes <= 160 * 1024, "LDS plan");
+    static_assert(S >= 3 && kASteps + D - 2 <= 7 && kSmemBytes <= 160 * 1024, "LDS plan");
     // DMA instructions a wave issues in a step of this tap (taps count modulo 9).
     static constexpr int issued(int tap) { return kBItems + (tap < kASteps ? kAPer : 0); }
     // At a step's barrier the weights of the next step (issued D - 1 steps ago) have landed: the
@@ -90,8 +105,9 @@ struct ConvArgs {
     int H, W, in_w, c_in, up;
     int c_out;
     int tiles_x, tiles_n, tiles;   // patches per row, channel tiles, all tiles
-    double* stats;         // or null: see wave_stats
+    double* stats;         // or null: see row16_sum
     int64_t stats_rows;
+    const NormChannel* norm;   // [c_in], NORM only
 };
 
 // Tile v -> patch origin and first channel. Workgroup b runs on XCD b % 8, so tiles are renumbered
@@ -107,20 +123,28 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& a, int v, int& y0, int
     x0 = (patch - ty * a.tiles_x) * 16;
 }
 
+__device__ __forceinline__ uint32_t lds_addr(const char* p) {
+    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const char*)(p)));
+}
+
 // The producer waves. `cur` and `next` are the weight sources of the chunk being multiplied and of
 // the one after it (across tiles); past the last chunk the sources repeat it, so that every step
 // issues the same number of instructions, into buffers nobody reads again.
-template <int MT, int NT>
+template <int MT, int NT, bool NORM>
 __device__ __forceinline__ void conv_produce(char* smem, const ConvArgs& a, const bf16_t* bias,
                                              int my_tiles, int wave, int lane) {
-    using G = Halo<MT, NT>;
+    using G = Halo<MT, NT, NORM>;
     const int sub = lane >> 3, slot = lane & 7;
     const int chunks = a.c_in >> 6;
     const int64_t k = 9 * static_cast<int64_t>(a.c_in);
     int aoff[G::kAItems];                 // element offset of each patch item's source, -1 outside
     const bf16_t *cur[G::kBItems], *next[G::kBItems];
 
+    // Items past the patch's end, there to keep the count, repeat its last block; where that block
+    // may be normalised already, they go to a spare KiB instead.
+    auto exists = [&](int i) { return i < G::kAItems && i * 4 + wave < G::kABlocks; };
     auto block_of = [&](int i) { return min(i * 4 + wave, G::kABlocks - 1); };
+    const int octet = lane & 7;   // of the channels this lane normalises
     auto tile_sources = [&](int it) {
         int y0, x0, n0;
         conv_tile<MT, NT>(a, blockIdx.x + it * gridDim.x, y0, x0, n0);
@@ -152,9 +176,41 @@ __device__ __forceinline__ void conv_produce(char* smem, const ConvArgs& a, cons
     auto issue_patch = [&](int first, int cb, char* buf) {
 #pragma unroll
         for (int q = 0; q < G::kAPer; ++q) {
-            const int i = min(first + q, G::kAItems - 1);
+            const int i = cmin(first + q, G::kAItems - 1);
             const bf16_t* src = aoff[i] < 0 ? a.zero + slot * 8 : a.in + aoff[i] + cb * 64;
-            dma16(src, buf + block_of(i) * 1024);
+            dma16(src, NORM && !exists(first + q) ? smem + G::kDumpOff : buf + block_of(i) * 1024);
+        }
+    };
+    // The channels' norm of chunk cb, 16 bytes a channel, into its LDS slot (wave 0).
+    auto issue_norm = [&](int cb) {
+        if (NORM && wave == 0) dma16(a.norm + cb * 64 + lane, smem + G::kNormOff);
+    };
+    // This lane's octet of them, from LDS.
+    NormChannel nc[NORM ? 8 : 1];
+    auto read_norm = [&]() {
+        if constexpr (NORM) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+                nc[q] = norm_silu_channel(reinterpret_cast<const NormChannel*>(smem + G::kNormOff)[octet * 8 + q]);
+        }
+    };
+    // The items of issue_patch(first, ...) normalised in place: lane L takes channel octet L % 8 of
+    // the pixel L / 8 of each block, wherever the swizzle put it; pixels outside the image stay
+    // zero, as the convolution pads the normalised tensor.
+    auto normalise_patch = [&](int first, char* buf) {
+        if constexpr (NORM) {
+            uint4 raw[G::kAPer];
+            char* at[G::kAPer];
+#pragma unroll
+            for (int q = 0; q < G::kAPer; ++q) {
+                const int row = block_of(first + q) * 8 + sub;
+                at[q] = buf + row * kRowBytes + (octet ^ (((row % kPW) >> 1) & 7)) * 16;
+                if (exists(first + q)) raw[q] = *reinterpret_cast<const uint4*>(at[q]);
+            }
+#pragma unroll
+            for (int q = 0; q < G::kAPer; ++q)
+                if (exists(first + q) && aoff[cmin(first + q, G::kAItems - 1)] >= 0)
+                    *reinterpret_cast<uint4*>(at[q]) = norm_silu8(raw[q], nc);
         }
     };
     int bst = 0;   // the stage the next weights go to
@@ -168,10 +224,17 @@ __device__ __forceinline__ void conv_produce(char* smem, const ConvArgs& a, cons
     tile_sources(0);
 #pragma unroll
     for (int i = 0; i < G::kBItems; ++i) cur[i] = next[i];
+    issue_norm(0);
 #pragma unroll
     for (int q = 0; q < G::kASteps; ++q) issue_patch(q * G::kAPer, 0, smem);
 #pragma unroll
     for (int t = 0; t < G::D; ++t) issue_weights(cur, t);
+    if (NORM) {
+        wait_and_join<0>();   // every wave sees the channels' norm
+        read_norm();
+#pragma unroll
+        for (int q = 0; q < G::kASteps; ++q) normalise_patch(q * G::kAPer, smem);
+    }
     const int total = my_tiles * chunks;
     int it = 0, cb = 0;   // of the chunk after the one being multiplied
     for (int c = 0; c < total; ++c) {
@@ -204,9 +267,13 @@ __device__ __forceinline__ void conv_produce(char* smem, const ConvArgs& a, cons
                     for (int i = 0; i < G::kBItems; ++i) next[i] = cur[i] + 64;
                 }
             }
+            if (tap == 0) issue_norm(cb);
             if (tap < G::kASteps) issue_patch(tap * G::kAPer, cb, nbuf);
             if (tap + G::D < 9) issue_weights(cur, tap + G::D);
             else issue_weights(next, tap + G::D - 9);
+            if (tap == G::D - 1) read_norm();
+            if (tap >= G::D - 1 && tap - (G::D - 1) < G::kASteps)
+                normalise_patch((tap - (G::D - 1)) * G::kAPer, nbuf);
         }
 #pragma unroll
         for (int i = 0; i < G::kBItems; ++i) cur[i] = next[i];
@@ -227,10 +294,6 @@ __device__ __forceinline__ void conv_join() {
 __device__ __forceinline__ bf16x8_t lds_frag(uint32_t addr) {
     return *reinterpret_cast<__attribute__((address_space(3))) const bf16x8_t*>(addr);
 }
-__device__ __forceinline__ uint32_t lds_addr(const char* p) {
-    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const char*)(p)));
-}
-
 // One k-step: a0 and b hold the first K=32 half's fragments (read during the step before); the
 // second half's (64 bytes further, in swizzled slots: address ^ 64) are read under the first
 // half's MFMAs and the next step's first half under the second half's.
@@ -341,7 +404,7 @@ __device__ __forceinline__ void conv_epilogue(const f32x4_t (&acc)[MW][NW], cons
             }
             const uint4 packed = pack8(v);
             *reinterpret_cast<uint4*>(a.out + base + i * row + 32 * p + lo) = packed;
-            if (STATS) {
+            if (STATS && a.stats) {
                 unpack8(packed, v);
 #pragma unroll
                 for (int q = 0; q < 8; ++q) {
@@ -351,7 +414,7 @@ __device__ __forceinline__ void conv_epilogue(const f32x4_t (&acc)[MW][NW], cons
                 }
             }
         }
-        if (STATS) {   // a lane's sixteen neighbours share its channels, so none has left the loop
+        if (STATS && a.stats) {   // a lane's sixteen neighbours share its channels, so none has left the loop
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const double s1 = row16_sum(sum[h]), s2 = row16_sum(sq[h]);
@@ -365,10 +428,11 @@ __device__ __forceinline__ void conv_epilogue(const f32x4_t (&acc)[MW][NW], cons
     }
 }
 
-template <int MT, int MODE, int NT, bool STATS>
+template <int MT, int MODE, int NT, bool STATS, bool NORM>
 __device__ __forceinline__ void conv_consume(char* smem, const ConvArgs& a, const Epi& e, int my_tiles,
                                              int wave, int lane) {
-    using G = Halo<MT, NT>;
+    using G = Halo<MT, NT, NORM>;
+    if (NORM) wait_and_join<63>();   // the producers' barrier over the first chunk's norm
     const int lr = lane & 15, hi = lane >> 4, sw = (lr >> 1) & 7;
     // this lane's offset in a 16-row weight block and in a patch row for tap column kx
     const uint32_t lb = lr * kRowBytes + ((hi ^ sw) * 16);
@@ -420,15 +484,15 @@ __device__ __forceinline__ void conv_consume(char* smem, const ConvArgs& a, cons
     }
 }
 
-template <int MT, int MODE, int NT, bool STATS>
+template <int MT, int MODE, int NT, bool STATS, bool NORM>
 __global__ void __launch_bounds__(kWgThreads, 1) k_conv3x3(ConvArgs a, Epi e) {
-    __shared__ __attribute__((aligned(1024))) char smem[Halo<MT, NT>::kSmemBytes];
+    __shared__ __attribute__((aligned(1024))) char smem[Halo<MT, NT, NORM>::kSmemBytes];
     const int my_tiles = (a.tiles - static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x) - 1) /
                          static_cast<int>(gridDim.x);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    if (wave >= kConsumers) conv_produce<MT, NT>(smem, a, e.bias, my_tiles, wave - kConsumers, lane);
-    else conv_consume<MT, MODE, NT, STATS>(smem, a, e, my_tiles, wave, lane);
+    if (wave >= kConsumers) conv_produce<MT, NT, NORM>(smem, a, e.bias, my_tiles, wave - kConsumers, lane);
+    else conv_consume<MT, MODE, NT, STATS, NORM>(smem, a, e, my_tiles, wave, lane);
 }
 
 int device_cus() {
@@ -448,23 +512,34 @@ int device_cus() {
 
 int patches(const ConvGeom& cv, int mt) { return ((cv.H + 4 * mt - 1) / (4 * mt)) * ((cv.W + 15) / 16); }
 
-template <int MT, int MODE, int NT>
-void launch_conv(const ConvGeom& cv, const bf16_t* w, bf16_t* out, int64_t c_out, const Epi& e, double* stats,
-                 hipStream_t s) {
+struct ConvExtra {
+    double* stats;
+    const NormChannel* norm;
+};
+
+template <int MT, int NT>
+void launch_conv(const ConvGeom& cv, const bf16_t* w, bf16_t* out, int64_t c_out, const Epi& e,
+                 const ConvExtra& x, hipStream_t s) {
     ConvArgs a{cv.in, cv.zero, w, out, cv.H, cv.W, cv.in_w, cv.c_in, cv.up, static_cast<int>(c_out), 0, 0, 0,
-               stats, static_cast<int64_t>(patches(cv, MT)) * (4 / Halo<MT, NT>::WN)};
+               x.stats, static_cast<int64_t>(patches(cv, MT)) * (4 / Halo<MT, NT>::WN), x.norm};
     a.tiles_x = (cv.W + 15) / 16;
     a.tiles_n = static_cast<int>((c_out + 16 * NT - 1) / (16 * NT));
     a.tiles = patches(cv, MT) * a.tiles_n;
     int grid = min(a.tiles, device_cus() & ~7);
     if (grid < 8) grid = min(a.tiles, device_cus());
+    // The combinations the decoder and the single op use; null sums are skipped.
     if constexpr (NT == 8) {
-        if (stats) {
-            k_conv3x3<MT, MODE, NT, true><<<grid, kWgThreads, 0, s>>>(a, e);
+        if (x.norm) {
+            if (e.residual) k_conv3x3<MT, EPI_RESIDUAL, NT, true, true><<<grid, kWgThreads, 0, s>>>(a, e);
+            else k_conv3x3<MT, EPI_STORE, NT, true, true><<<grid, kWgThreads, 0, s>>>(a, e);
             return;
         }
+        if (e.residual) k_conv3x3<MT, EPI_RESIDUAL, NT, true, false><<<grid, kWgThreads, 0, s>>>(a, e);
+        else if (x.stats) k_conv3x3<MT, EPI_STORE, NT, true, false><<<grid, kWgThreads, 0, s>>>(a, e);
+        else k_conv3x3<MT, EPI_STORE, NT, false, false><<<grid, kWgThreads, 0, s>>>(a, e);
+    } else {
+        k_conv3x3<MT, EPI_STORE, NT, false, false><<<grid, kWgThreads, 0, s>>>(a, e);
     }
-    k_conv3x3<MT, MODE, NT, false><<<grid, kWgThreads, 0, s>>>(a, e);
 }
 
 // The patch height: the least estimated time, rounds of tiles over the CUs times a step's cycles.
@@ -486,20 +561,6 @@ int conv_rows(const ConvGeom& cv, int64_t c_out) {
     return best;
 }
 
-template <int MODE>
-void launch_conv_mode(const ConvGeom& cv, const bf16_t* w, bf16_t* out, int64_t c_out, const Epi& e,
-                      double* stats, hipStream_t s) {
-    if (c_out <= 32) {   // the decoder's conv_out: one 32-wide tile column
-        launch_conv<4, MODE, 2>(cv, w, out, c_out, e, nullptr, s);
-        return;
-    }
-    switch (conv_rows(cv, c_out)) {
-        case 1: launch_conv<1, MODE, 8>(cv, w, out, c_out, e, stats, s); break;
-        case 2: launch_conv<2, MODE, 8>(cv, w, out, c_out, e, stats, s); break;
-        default: launch_conv<4, MODE, 8>(cv, w, out, c_out, e, stats, s); break;
-    }
-}
-
 bool aligned(const void* p, int bytes) { return (reinterpret_cast<uintptr_t>(p) % bytes) == 0; }
 
 }  // namespace
@@ -514,7 +575,8 @@ int64_t conv3x3_stats_rows(const ConvGeom& cv, int64_t c_out) {
 }
 
 void launch_conv3x3_bf16(const ConvGeom& cv, const bf16_t* wr, const bf16_t* bias, bf16_t* out,
-                         int64_t c_out, const GemmEpilogue& ep, hipStream_t s, double* stats) {
+                         int64_t c_out, const GemmEpilogue& ep, hipStream_t s, double* stats,
+                         const NormChannel* norm) {
     const int64_t m = static_cast<int64_t>(cv.H) * cv.W, k = 9 * static_cast<int64_t>(cv.c_in);
     if (m == 0 || c_out == 0) return;
     require(cv.in && cv.zero && wr && out, "conv3x3: null operand");
@@ -533,8 +595,18 @@ void launch_conv3x3_bf16(const ConvGeom& cv, const bf16_t* wr, const bf16_t* bia
     require(ep.act == 0, "conv3x3: no activation epilogue (the decoder's SiLU follows a GroupNorm)");
     ProfileScope ps(K_GEMM, s, 2.0 * static_cast<double>(m) * c_out * k);
     require(!stats || conv3x3_stats_rows(cv, c_out) > 0, "conv3x3: this shape sums no statistics");
-    if (ep.residual) launch_conv_mode<EPI_RESIDUAL>(cv, wr, out, c_out, e, stats, s);
-    else launch_conv_mode<EPI_STORE>(cv, wr, out, c_out, e, stats, s);
+    require((!ep.residual && !norm) || c_out > 32, "conv3x3: the narrow tile is a plain store");
+    require(!norm || (!cv.up && aligned(norm, 16)), "conv3x3: a normalised input is not upsampled");
+    const ConvExtra x{stats, norm};
+    if (c_out <= 32) {   // the decoder's conv_out: one 32-wide tile column
+        launch_conv<4, 2>(cv, wr, out, c_out, e, x, s);
+    } else {
+        switch (conv_rows(cv, c_out)) {
+            case 1: launch_conv<1, 8>(cv, wr, out, c_out, e, x, s); break;
+            case 2: launch_conv<2, 8>(cv, wr, out, c_out, e, x, s); break;
+            default: launch_conv<4, 8>(cv, wr, out, c_out, e, x, s); break;
+        }
+    }
     launch_check("conv3x3 (mfma)");
 }
 

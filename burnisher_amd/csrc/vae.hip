@@ -5,10 +5,9 @@
 //   - k_transpose       [R, C] -> [C, R] per batch: NCHW <-> NHWC at the stage's two ends, and
 //                       the reference's TransposeArgs op (ops.h:184-191);
 //   - GroupNorm         fp64 sums and sums of squares in a fixed order (from the convolution that
-//                       wrote the tensor, or one pass over it), then one pass that normalises,
-//                       applies the affine and, optionally, SiLU (the reference's norm then activation, each rounded
-//                       to bf16 as the reference stores them, ops_cpu.cpp:186-224, 265-274; the
-//                       SiLU with the hardware exp2 and reciprocal, within one bf16 ulp);
+//                       wrote the tensor, or one pass over it), applied with its SiLU (each
+//                       rounded to bf16 as the reference stores them, ops_cpu.cpp:186-224,
+//                       265-274) by a pass, or by the convolution that reads the tensor;
 //   - k_conv_direct     a convolution in the reference's summation order, for the layers too thin
 //                       for the MFMA tile (conv_in: 4 input channels; conv_out: 3 outputs);
 //   - k_upsample_nchw   the reference's UpsampleArgs op (the engine fuses the upsample into the
@@ -94,26 +93,28 @@ __global__ void __launch_bounds__(kGnThreads) k_gn_stats(const bf16_t* __restric
 }
 
 // Group g's statistics from its `count` pairs at part[g * count]: mean = s1 / n, var = (n s2 - s1^2) /
-// n^2, inv = 1 / sqrt(float(var) + eps), the reference's rounding (ops_cpu.cpp:208-210). One workgroup
-// per group, summed in a fixed order.
+// n^2, inv = 1 / sqrt(float(var) + eps), the reference's rounding (ops_cpu.cpp:208-210), with the affine
+// to the group's channels. One workgroup per group, summed in a fixed order.
 constexpr int kGnFinThreads = 512;
 
 __global__ void __launch_bounds__(kGnFinThreads) k_gn_finalize(const double* __restrict__ part, int64_t count,
-                                                              double n, float eps, double* __restrict__ mean,
-                                                              float* __restrict__ inv) {
+                                                              double n, float eps, int cpg,
+                                                              const bf16_t* __restrict__ w,
+                                                              const bf16_t* __restrict__ b,
+                                                              NormChannel* __restrict__ channels) {
 #pragma clang fp contract(off)
     __shared__ double red[2][kGnFinThreads];
     const int g = blockIdx.x, t = threadIdx.x;
     const double2* src = reinterpret_cast<const double2*>(part) + g * count;
-    double a = 0.0, b = 0.0;
+    double x1 = 0.0, x2 = 0.0;
 #pragma unroll 4
     for (int64_t c = t; c < count; c += kGnFinThreads) {
         const double2 v = src[c];
-        a += v.x;
-        b += v.y;
+        x1 += v.x;
+        x2 += v.y;
     }
-    red[0][t] = a;
-    red[1][t] = b;
+    red[0][t] = x1;
+    red[1][t] = x2;
     __syncthreads();
     for (int w = kGnFinThreads / 2; w > 0; w >>= 1) {
         if (t < w) {
@@ -122,69 +123,40 @@ __global__ void __launch_bounds__(kGnFinThreads) k_gn_finalize(const double* __r
         }
         __syncthreads();
     }
-    if (t != 0) return;
     const double s1 = red[0][0], s2 = red[1][0];
     // n s2 - s1^2 with each product as a rounded value and its exact remainder
     const double p = n * s2, q = s1 * s1;
     const double num = (p - q) + (__builtin_fma(n, s2, -p) - __builtin_fma(s1, s1, -q));
     const double var = num <= 0.0 ? 0.0 : num / (n * n);   // a NaN stays one
-    mean[g] = s1 / n;
-    inv[g] = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(static_cast<float>(var), eps)));
+    NormChannel nc;
+    nc.mean = static_cast<float>(s1 / n);
+    nc.inv = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(static_cast<float>(var), eps)));
+    for (int c = g * cpg + t; c < (g + 1) * cpg; c += kGnFinThreads) {
+        nc.w = w ? bf2f(w[c]) : 1.0f;
+        nc.b = b ? bf2f(b[c]) : -0.0f;   // x + (-0.0) is x exactly
+        channels[c] = nc;
+    }
 }
 
-// SiLU with the hardware exp2 and reciprocal: a few fp32 ulps from x / (1 + exp(-x)), which moves
-// the bf16 value it is rounded to by at most one ulp (the same bound as a device expf).
-__device__ __forceinline__ float silu_hw(float x) {
-    return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x));
-}
-
-// (x - float(mean)) * inv, * weight[c], + bias[c] (separate roundings, the reference's order),
-// rounded to bf16; with SILU, SiLU of that bf16 value, rounded again. In place is allowed (each
-// element is read before it is written by the same thread). The grid stride is a multiple of 256
-// and C/8 divides 256, so a thread always sees the same eight channels: their statistics and
-// affine are read once, before the loop.
-template <bool W, bool B, bool SILU>
-__global__ void __launch_bounds__(256) k_gn_apply(const bf16_t* x, bf16_t* out, int64_t S, int C, int G,
-                                                  const double* __restrict__ mean,
-                                                  const float* __restrict__ inv,
-                                                  const bf16_t* __restrict__ w,
-                                                  const bf16_t* __restrict__ b) {
-    const int oct = C / 8, cpg = C / G;
+// norm8 or norm_silu8 over [S, C]. In place is allowed (each element is read before it is written by the same thread). The grid stride is a
+// multiple of 256 and C/8 divides 256, so a thread always sees the same eight channels.
+template <bool SILU>
+__global__ void __launch_bounds__(256) k_gn_apply(const bf16_t* x, bf16_t* out, int64_t S, int C,
+                                                  const NormChannel* __restrict__ channels) {
+    const int oct = C / 8;
     const int64_t n = S * oct;
     const int64_t first = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
     const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-    const int c0 = static_cast<int>(first % oct) * 8;
-    float mf[8], iv[8], wv[8], bv[8];
+    NormChannel nc[8];
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-        const int c = c0 + q, g = c / cpg;
-        mf[q] = static_cast<float>(mean[g]);
-        iv[q] = inv[g];
-        wv[q] = W ? bf2f(w[c]) : 1.0f;
-        bv[q] = B ? bf2f(b[c]) : 0.0f;
+        nc[q] = channels[static_cast<int>(first % oct) * 8 + q];
+        if (SILU) nc[q] = norm_silu_channel(nc[q]);
     }
     const uint4* src = reinterpret_cast<const uint4*>(x);
     uint4* dst = reinterpret_cast<uint4*>(out);
     for (int64_t i = first; i < n; i += stride) {
-        const uint4 raw = src[i];
-        const uint32_t w4[4] = {raw.x, raw.y, raw.z, raw.w};
-        uint32_t r4[4];
-#pragma unroll
-        for (int q2 = 0; q2 < 4; ++q2) {
-            float v2[2];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int q = 2 * q2 + h;
-                const float xv = __uint_as_float(h ? (w4[q2] & 0xffff0000u) : (w4[q2] << 16));
-                float v = __fmul_rn(__fsub_rn(xv, mf[q]), iv[q]);
-                if (W) v = __fmul_rn(v, wv[q]);
-                if (B) v = __fadd_rn(v, bv[q]);
-                if (SILU) v = silu_hw(round_bf16(v));
-                v2[h] = v;
-            }
-            r4[q2] = f2bf2(v2[0], v2[1]);
-        }
-        dst[i] = make_uint4(r4[0], r4[1], r4[2], r4[3]);
+        dst[i] = SILU ? norm_silu8(src[i], nc) : norm8(src[i], nc);
     }
 }
 
@@ -316,10 +288,9 @@ void* op_workspace(int slot, size_t bytes) {
 GroupNormScratch op_gn_scratch() {
     GroupNormScratch sc;
     sc.max_chunks = 2048;
-    char* base = static_cast<char*>(op_workspace(SLOT_GN, 2048 * 64 * 16 + 64 * 8 + 64 * 4));
+    char* base = static_cast<char*>(op_workspace(SLOT_GN, 2048 * 64 * 16 + 2048 * sizeof(NormChannel)));
     sc.part = reinterpret_cast<double*>(base);
-    sc.mean = reinterpret_cast<double*>(base + 2048 * 64 * 16);
-    sc.inv = reinterpret_cast<float*>(base + 2048 * 64 * 16 + 64 * 8);
+    sc.channels = reinterpret_cast<NormChannel*>(base + 2048 * 64 * 16);
     return sc;
 }
 
@@ -386,7 +357,8 @@ void launch_group_norm_nchw(const bf16_t* x, const bf16_t* w, const bf16_t* b, b
     GroupNormScratch sc = op_gn_scratch();
     for (int64_t r = 0; r < rows; ++r) {
         launch_transpose_bf16(x + r * cols, xin, 1, C, S, s);
-        launch_group_norm_nhwc(xin, yout, S, C, groups, eps, w, b, false, sc, s);
+        launch_group_norm_channels(xin, S, C, groups, eps, w, b, sc, s);
+        launch_group_norm_apply(xin, yout, S, C, false, sc, s);
         launch_transpose_bf16(yout, out + r * cols, 1, S, C, s);
     }
 }
@@ -455,38 +427,30 @@ bool gn_nhwc_supported(int64_t C, int64_t G) {
            C % G == 0;
 }
 
-void launch_group_norm_nhwc(const bf16_t* x, bf16_t* out, int64_t S, int64_t C, int64_t G,
-                            float eps, const bf16_t* w, const bf16_t* b, bool silu,
-                            GroupNormScratch& sc, hipStream_t s, int64_t stats_rows) {
+void launch_group_norm_channels(const bf16_t* x, int64_t S, int64_t C, int64_t G, float eps,
+                                const bf16_t* w, const bf16_t* b, GroupNormScratch& sc, hipStream_t s,
+                                int64_t stats_rows) {
     require(gn_nhwc_supported(C, G), "groupnorm (nhwc): unsupported channel / group count");
     require(stats_rows == 0 || (C / G) % 4 == 0, "groupnorm (nhwc): sums come by runs of four channels");
     const int ci = static_cast<int>(C), gi = static_cast<int>(G);
-    const double n = static_cast<double>(S) * (C / G);
-    ProfileScope ps(K_NORM, s, 4.0 * static_cast<double>(S * C));
+    ProfileScope ps(K_NORM, s, stats_rows ? 0.0 : 2.0 * static_cast<double>(S * C));
     int64_t count = stats_rows * (C / G / 4);
     if (count == 0) {
         const int chunks = static_cast<int>(std::min<int64_t>(sc.max_chunks, std::max<int64_t>(1, (S + 15) / 16)));
         k_gn_stats<<<chunks, kGnThreads, 0, s>>>(x, S, ci, gi, (S + chunks - 1) / chunks, sc.part);
         count = chunks;
     }
-    k_gn_finalize<<<gi, kGnFinThreads, 0, s>>>(sc.part, count, n, eps, sc.mean, sc.inv);
+    k_gn_finalize<<<gi, kGnFinThreads, 0, s>>>(sc.part, count, static_cast<double>(S) * (C / G), eps, ci / gi, w, b,
+                                               sc.channels);
+    launch_check("groupnorm statistics (nhwc)");
+}
+
+void launch_group_norm_apply(const bf16_t* x, bf16_t* out, int64_t S, int64_t C, bool silu,
+                             const GroupNormScratch& sc, hipStream_t s) {
+    ProfileScope ps(K_NORM, s, 4.0 * static_cast<double>(S * C));
     const int blocks = grid_for(S * (C / 8), 256);
-#define BH_GN_APPLY(W_, B_, S_) \
-    k_gn_apply<W_, B_, S_><<<blocks, 256, 0, s>>>(x, out, S, ci, gi, sc.mean, sc.inv, w, b)
-    if (w && b) {
-        if (silu) BH_GN_APPLY(true, true, true);
-        else BH_GN_APPLY(true, true, false);
-    } else if (w) {
-        if (silu) BH_GN_APPLY(true, false, true);
-        else BH_GN_APPLY(true, false, false);
-    } else if (b) {
-        if (silu) BH_GN_APPLY(false, true, true);
-        else BH_GN_APPLY(false, true, false);
-    } else {
-        if (silu) BH_GN_APPLY(false, false, true);
-        else BH_GN_APPLY(false, false, false);
-    }
-#undef BH_GN_APPLY
+    if (silu) k_gn_apply<true><<<blocks, 256, 0, s>>>(x, out, S, static_cast<int>(C), sc.channels);
+    else k_gn_apply<false><<<blocks, 256, 0, s>>>(x, out, S, static_cast<int>(C), sc.channels);
     launch_check("groupnorm (nhwc)");
 }
 

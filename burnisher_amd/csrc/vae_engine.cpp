@@ -41,7 +41,6 @@ struct bh_vae {
     bf16_t *q = nullptr, *k = nullptr, *v = nullptr, *o = nullptr;
     int attn_splits = 1;   // key splits of the mid-block attention at width 512
     bf16_t* zero = nullptr;
-    bf16_t* conv_out_bias = nullptr;   // decoder.conv_out.bias padded to 8 outputs
     bh::GroupNormScratch gn;
     int64_t gn_part_bytes = 0;
     int64_t bytes = 0;
@@ -153,42 +152,44 @@ struct Run {
     const bf16_t* summed = nullptr;
     int64_t sum_rows = 0;
 
-    void gn(const bf16_t* x, bf16_t* out, const std::string& n, int64_t ch, int64_t h, bool silu) {
-        launch_group_norm_nhwc(x, out, h * h, ch, e.cfg.norm_num_groups, static_cast<float>(e.cfg.eps),
-                               e.at(n + ".weight"), e.at(n + ".bias"), silu, e.gn, s, x == summed ? sum_rows : 0);
-        if (x != summed || out == x) summed = nullptr;   // e.gn.part or the tensor has changed
+    // The GroupNorm `n` of x into e.gn.channels.
+    void gn_channels(const bf16_t* x, const std::string& n, int64_t ch, int64_t h) {
+        launch_group_norm_channels(x, h * h, ch, e.cfg.norm_num_groups, static_cast<float>(e.cfg.eps),
+                                   e.at(n + ".weight"), e.at(n + ".bias"), e.gn, s, x == summed ? sum_rows : 0);
+        if (x != summed) summed = nullptr;   // e.gn.part now holds the sums of a pass
     }
 
-    // A convolution whose output a GroupNorm reads next, with its sums where the widths allow.
-    void conv_summed(const ConvGeom& g, const bf16_t* w, const bf16_t* bias, bf16_t* out, int64_t co,
-                     const GemmEpilogue& ep) {
+    // 3x3 "same" conv of x (h_in x h_in, ci) to out (h x h, co); up: h = 2 h_in, nearest. `norm`: the
+    // input is silu(GroupNorm `norm` of x). The sums of the output for the GroupNorm that reads it
+    // next come with it where the widths allow.
+    //
+    // The convolution normalises its input itself, except the narrow output convolution: it has too
+    // few MFMAs to hide that under (512 x 512: 25 -> 56 us, the pass it would save 27 us).
+    void conv3(bf16_t* x, bf16_t* out, const std::string& n, int64_t ci, int64_t co, int64_t h, bool up,
+               const bf16_t* residual, const std::string& norm) {
+        const bool fused = !norm.empty() && co > 32;
+        if (!norm.empty()) {
+            gn_channels(x, norm, ci, h);
+            if (!fused) launch_group_norm_apply(x, x, h * h, ci, true, e.gn, s);
+        }
+        ConvGeom g;
+        g.in = x;
+        g.zero = e.zero;
+        g.H = g.W = static_cast<int>(h);
+        g.in_h = g.in_w = static_cast<int>(up ? h / 2 : h);
+        g.c_in = static_cast<int>(ci);
+        g.up = up ? 1 : 0;
+        GemmEpilogue ep;
+        ep.residual = residual;
+        ep.round_mid = residual != nullptr;
         const int64_t rows = (co / e.cfg.norm_num_groups) % 4 == 0 ? conv3x3_stats_rows(g, co) : 0;
         const bool fits = rows > 0 && rows * (co / 4) * 16 <= e.gn_part_bytes;
-        launch_conv3x3_bf16(g, w, bias, out, co, ep, s, fits ? e.gn.part : nullptr);
+        const auto padded = e.rw.find(n + ".bias");
+        const bf16_t* bias = padded != e.rw.end() ? padded->second : e.at(n + ".bias");
+        launch_conv3x3_bf16(g, e.rw.at(n + ".weight"), bias, out, co, ep, s,
+                            fits ? e.gn.part : nullptr, fused ? e.gn.channels : nullptr);
         summed = fits ? out : nullptr;
         sum_rows = fits ? rows : 0;
-    }
-
-    // 3x3 "same" conv of x (h_in x h_in, ci) to out (h x h, co); up: h = 2 h_in, nearest.
-    void conv3(const bf16_t* x, bf16_t* out, const std::string& n, int64_t ci, int64_t co, int64_t h,
-               bool up, const bf16_t* residual) {
-        const int64_t hin = up ? h / 2 : h;
-        if (mfma_conv(ci, co)) {
-            ConvGeom g;
-            g.in = x;
-            g.zero = e.zero;
-            g.H = g.W = static_cast<int>(h);
-            g.in_h = g.in_w = static_cast<int>(hin);
-            g.c_in = static_cast<int>(ci);
-            g.up = up ? 1 : 0;
-            GemmEpilogue ep;
-            ep.residual = residual;
-            ep.round_mid = residual != nullptr;
-            conv_summed(g, e.rw.at(n + ".weight"), e.at(n + ".bias"), out, co, ep);
-            return;
-        }
-        require(!up && !residual, "vae: a thin convolution cannot be an upsampler or carry a residual");
-        launch_conv_direct_nhwc(x, e.at(n + ".weight"), e.at(n + ".bias"), out, h, h, ci, co, 3, 1, s);
     }
 
     // out = x . W^T + bias over [h*h, ci] (a 1x1 conv or a linear layer), optionally + residual
@@ -204,31 +205,29 @@ struct Run {
 
     // ResnetBlock2D (vae_decoder.cpp:64-80): returns the output buffer; x is released.
     bf16_t* resnet(bf16_t* x, const std::string& n, int64_t ci, int64_t co, int64_t h) {
-        bf16_t* t = take();
-        gn(x, t, n + ".norm1", ci, h, true);                   // t = silu(norm1(x))
         bf16_t* c1 = take();
-        conv3(t, c1, n + ".conv1", ci, co, h, false, nullptr);  // c1 = conv1(t)
-        gn(c1, c1, n + ".norm2", co, h, true);                  // c1 = silu(norm2(c1))
+        conv3(x, c1, n + ".conv1", ci, co, h, false, nullptr, n + ".norm1");   // c1 = conv1(silu(norm1(x)))
+        bf16_t* out = take();
+        const bf16_t* residual = x;
+        bf16_t* t = nullptr;
         if (ci != co) {
+            t = take();
             linear(x, t, n + ".conv_shortcut", h * h, ci, co, nullptr);   // t = shortcut(x)
-            give(x);
-            bf16_t* out = take();
-            conv3(c1, out, n + ".conv2", co, co, h, false, t);  // out = t + conv2(c1)
-            give(t);
-            give(c1);
-            return out;
+            residual = t;
         }
-        conv3(c1, t, n + ".conv2", co, co, h, false, x);        // t = x + conv2(c1)
+        conv3(c1, out, n + ".conv2", co, co, h, false, residual, n + ".norm2");   // out = residual + conv2(silu(norm2(c1)))
         give(x);
         give(c1);
-        return t;
+        if (t) give(t);
+        return out;
     }
 
     // Spatial self-attention of the mid-block (vae_decoder.cpp:85-118), tokens read in place.
     bf16_t* attention(bf16_t* x, const std::string& n, int64_t ch, int64_t h) {
         const int64_t S = h * h;
         bf16_t* normed = take();
-        gn(x, normed, n + ".group_norm", ch, h, false);
+        gn_channels(x, n + ".group_norm", ch, h);
+        launch_group_norm_apply(x, normed, S, ch, false, e.gn, s);
         linear(normed, e.q, n + ".to_q", S, ch, ch, nullptr);
         linear(normed, e.k, n + ".to_k", S, ch, ch, nullptr);
         linear(normed, e.v, n + ".to_v", S, ch, ch, nullptr);
@@ -262,15 +261,7 @@ struct Run {
         // conv_in: the latent's channels zero-padded to one 64-channel k-tile, on the MFMA kernel
         // (the padded weights are zero there, so the sums are those of the thin convolution)
         launch_pad_rows(b, a, h * h, zc, 64, s);
-        {
-            ConvGeom g;
-            g.in = a;
-            g.zero = e.zero;
-            g.H = g.W = g.in_h = g.in_w = static_cast<int>(h);
-            g.c_in = 64;
-            conv_summed(g, e.rw.at("decoder.conv_in.weight"), e.at("decoder.conv_in.bias"), b, p.rev[0],
-                        GemmEpilogue{});
-        }
+        conv3(a, b, "decoder.conv_in", 64, p.rev[0], h, false, nullptr, "");
         std::swap(a, b);
         give(b);
         bf16_t* x = a;
@@ -288,24 +279,16 @@ struct Run {
                 // nearest 2x upsample folded into the upsampler conv's gather (vae_decoder.cpp:170-175)
                 bf16_t* y = take();
                 conv3(x, y, "decoder.up_blocks." + std::to_string(i) + ".upsamplers.0.conv", co, co, 2 * h,
-                      true, nullptr);
+                      true, nullptr, "");
                 give(x);
                 x = y;
                 h *= 2;
             }
         }
-        gn(x, x, "decoder.conv_norm_out", prev, h, true);
         // conv_out: 3 outputs padded to 8 (zero weights and bias), on the MFMA kernel; the
         // transpose to NCHW keeps the first 3 channels
         bf16_t* y = take();
-        {
-            ConvGeom g;
-            g.in = x;
-            g.zero = e.zero;
-            g.H = g.W = g.in_h = g.in_w = static_cast<int>(h);
-            g.c_in = static_cast<int>(prev);
-            launch_conv3x3_bf16(g, e.rw.at("decoder.conv_out.weight"), e.conv_out_bias, y, 8, GemmEpilogue{}, s);
-        }
+        conv3(x, y, "decoder.conv_out", prev, 8, h, false, nullptr, "decoder.conv_norm_out");
         launch_transpose_keep_bf16(y, image, h * h, 8, 3, s);
         give(x);
         give(y);
@@ -383,8 +366,7 @@ int bh_vae_create(const bh_vae_config* cfg, const bh_vae_weights* w, int64_t lat
             e->gn.part = static_cast<double*>(e->alloc(bytes));
             e->gn_part_bytes = bytes;
         }
-        e->gn.mean = static_cast<double*>(e->alloc(64 * 8));
-        e->gn.inv = static_cast<float*>(e->alloc(64 * 4));
+        e->gn.channels = static_cast<bh::NormChannel*>(e->alloc(2048 * sizeof(bh::NormChannel)));
         // repack every 3x3 weight the MFMA conv reads
         auto repack = [&](const std::string& n, int64_t ci, int64_t co) {
             if (!bh::mfma_conv(ci, co) || e->rw.count(n + ".weight")) return;
@@ -417,8 +399,9 @@ int bh_vae_create(const bh_vae_config* cfg, const bh_vae_weights* w, int64_t lat
             bf16_t* ro = static_cast<bf16_t*>(e->alloc(8 * prev * 9 * 2));
             bh::launch_repack3x3_pad(e->at("decoder.conv_out.weight"), ro, 3, prev, 8, prev, nullptr);
             e->rw["decoder.conv_out.weight"] = ro;
-            e->conv_out_bias = static_cast<bf16_t*>(e->alloc(16));   // zero-filled by alloc
-            bh::hip_check(hipMemcpy(e->conv_out_bias, e->at("decoder.conv_out.bias"), 3 * 2,
+            bf16_t* bo = static_cast<bf16_t*>(e->alloc(16));   // zero-filled by alloc
+            e->rw["decoder.conv_out.bias"] = bo;
+            bh::hip_check(hipMemcpy(bo, e->at("decoder.conv_out.bias"), 3 * 2,
                                     hipMemcpyDeviceToDevice), "hipMemcpy (conv_out bias)");
         }
         bh::hip_check(hipDeviceSynchronize(), "vae_create");
