@@ -112,11 +112,12 @@ def test_group_norm_matches_oracle(hip, case):
 
 
 @pytest.mark.parametrize("case", ["constant", "offset", "one_outlier", "inf", "nan"])
-def test_group_norm_statistics_edges(hip, case):
+@pytest.mark.parametrize("S", [300, 304], ids=["scalar", "vector"])
+def test_group_norm_statistics_edges(hip, case, S):
     """The one-pass statistics (sums of x and x^2) where they could cancel or spread: a constant
     group (variance 0), a mean 200 times the deviation, one huge value, an infinity, a NaN (their
     groups become NaN, the others keep their values)."""
-    C, S, G = 128, 300, 32
+    C, G = 128, 32
     x = from_bf16(randn_bf16(RNG, (C, S), 1.0)).astype(np.float32)
     if case == "constant":
         x[4:8] = 3.140625
@@ -158,6 +159,19 @@ def test_upsample_and_transpose_match_oracle(hip):
         dsrc = dev(src)
         call("bh_transpose", dsrc.data_ptr(), out.data_ptr(), 3, 37, 70, to_cf, BF16, None)
         assert np.array_equal(host(out), want)
+
+
+@pytest.mark.parametrize("C,S", [(64, 72), (40, 104), (200, 64), (32, 4096), (512, 33), (8, 1000)])
+def test_transpose_wide_tiles_match_oracle(hip, C, S):
+    """16-byte runs on both sides (multiples of 8, whole and ragged 64 x 64 tiles) and the scalar tiles."""
+    B = 1 if C == 8 else 2
+    t = randn_bf16(RNG, (B, C, S))
+    for to_cf in (0, 1):
+        src = t if to_cf == 0 else np.ascontiguousarray(t.transpose(0, 2, 1))
+        out = empty((B, S, C) if to_cf == 0 else (B, C, S))
+        dsrc = dev(src)
+        call("bh_transpose", dsrc.data_ptr(), out.data_ptr(), B, C, S, to_cf, BF16, None)
+        assert np.array_equal(host(out), t.transpose(0, 2, 1) if to_cf == 0 else t)
 
 
 @pytest.mark.parametrize("S", [64, 100, 333])
