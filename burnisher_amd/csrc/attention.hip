@@ -1,8 +1,8 @@
 // Flash attention for the dit-step on gfx950: softmax(scale * Q K^T, key mask) V over
 // head-last [batch, seq, heads, head_dim] operands, bf16 in and out, fp32 scores and softmax.
 //
-// Workgroup = 4 waves = 256 query rows of one (batch, head); each wave owns 64 query rows as 4
-// tiles of 16. K/V stream through LDS in blocks of 64 keys, double-buffered, with the next
+// Workgroup = 4 waves = 256 query rows of one (batch, head), each wave 4 tiles of 16, or 64 rows, a
+// tile a wave, where 256-row workgroups would leave the chip idle (flash_query_tiles). K/V stream through LDS in blocks of 64 keys, double-buffered, with the next
 // block's global loads in flight in registers while the current block is multiplied.
 //
 // Both products run on v_mfma_f32_16x16x32_bf16 and the kernel computes TRANSPOSED tiles:
@@ -31,9 +31,7 @@ namespace bh {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kQRows = 256;   // query rows per workgroup
 constexpr int kKvBlk = 64;    // keys per LDS block
-constexpr int kQT = 4;        // 16-row query tiles per wave
 constexpr int kKT = 4;        // 16-key tiles per block
 constexpr int kMaxFlagBlocks = 256;
 constexpr float kLog2e = 1.4426950408889634f;
@@ -59,9 +57,12 @@ __device__ __forceinline__ float mask_at(const void* m, int f32, int64_t i) {
     return f32 ? static_cast<const float*>(m)[i] : bf2f(static_cast<const bf16_t*>(m)[i]);
 }
 
-// KS: K=32 steps of the score product (head_dim padded to 32*KS); DT: 16-row tiles of V^T.
-template <int KS, int DT, bool VEC>
-__global__ void __launch_bounds__(kThreads, 1) k_flash(AttnArgs a) {
+// KS: K=32 steps of the score product (head_dim padded to 32*KS); DT: 16-row tiles of V^T; kQT: 16-row
+// query tiles per wave (64 kQT query rows per workgroup).
+// A one-tile workgroup is a chain of memory latencies, so two or more share a CU.
+template <int KS, int DT, bool VEC, int kQT>
+__global__ void __launch_bounds__(kThreads, kQT == 4 ? 1 : 2) k_flash(AttnArgs a) {
+    constexpr int kQRows = 64 * kQT;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     const int stage_elems = kKvBlk * a.k_row + DT * 16 * a.v_row;
     bf16_t* smem = reinterpret_cast<bf16_t*>(smem_raw);
@@ -117,11 +118,15 @@ __global__ void __launch_bounds__(kThreads, 1) k_flash(AttnArgs a) {
             bf16x8_t f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) f[e] = static_cast<__bf16>(0.0f);
-            if (qrow < a.Sq && d0 < D8) {
+            if (VEC) {   // D % 8 == 0; queries past the end read the last one, dims past D are zeroed
+                f = *reinterpret_cast<const bf16x8_t*>(a.q + (b * a.Sq + min(qrow, a.Sq - 1)) * a.ld_q + h * D +
+                                                       min(d0, D8 - 8));
+                if (d0 >= D8)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) f[e] = static_cast<__bf16>(0.0f);
+            } else if (qrow < a.Sq && d0 < D8) {
                 const bf16_t* src = a.q + (b * a.Sq + qrow) * a.ld_q + h * D + d0;
-                if (VEC) {
-                    f = *reinterpret_cast<const bf16x8_t*>(src);
-                } else {
+                {
                     bf16_t tmp[8];
 #pragma unroll
                     for (int e = 0; e < 8; ++e) tmp[e] = (d0 + e < D) ? src[e] : 0;
@@ -141,6 +146,17 @@ __global__ void __launch_bounds__(kThreads, 1) k_flash(AttnArgs a) {
 #pragma unroll
         for (int i = 0; i < kMaxChunks; ++i) {
             const int cidx = tid + i * kThreads;
+            if (VEC) {
+                // No branch around a load (each would be waited for by itself): past the last chunk
+                // or key the last one is read again, and only what a key contributes is kept.
+                const int cc = min(cidx, nchunks - 1), row = cc / chunks_per_row, ch = cc % chunks_per_row;
+                const int64_t kv = static_cast<int64_t>(blk) * kKvBlk + row;
+                const int64_t off = (b * a.Skv + min(kv, a.Skv - 1)) * a.ld_kv + h * D + ch * 8;
+                rk[i] = *reinterpret_cast<const uint4*>(a.k + off);
+                rv[i] = *reinterpret_cast<const uint4*>(a.v + off);
+                if (kv >= a.Skv) rk[i] = rv[i] = make_uint4(0, 0, 0, 0);
+                continue;
+            }
             rk[i] = make_uint4(0, 0, 0, 0);
             rv[i] = make_uint4(0, 0, 0, 0);
             if (cidx < nchunks) {
@@ -148,20 +164,15 @@ __global__ void __launch_bounds__(kThreads, 1) k_flash(AttnArgs a) {
                 const int64_t kv = static_cast<int64_t>(blk) * kKvBlk + row;
                 if (kv < a.Skv) {
                     const int64_t off = (b * a.Skv + kv) * a.ld_kv + h * D + ch * 8;
-                    if (VEC) {
-                        rk[i] = *reinterpret_cast<const uint4*>(a.k + off);
-                        rv[i] = *reinterpret_cast<const uint4*>(a.v + off);
-                    } else {
-                        bf16_t tk[8], tv[8];
+                    bf16_t tk[8], tv[8];
 #pragma unroll
-                        for (int e = 0; e < 8; ++e) {
-                            const bool in = ch * 8 + e < D;
-                            tk[e] = in ? a.k[off + e] : 0;
-                            tv[e] = in ? a.v[off + e] : 0;
-                        }
-                        rk[i] = *reinterpret_cast<const uint4*>(tk);
-                        rv[i] = *reinterpret_cast<const uint4*>(tv);
+                    for (int e = 0; e < 8; ++e) {
+                        const bool in = ch * 8 + e < D;
+                        tk[e] = in ? a.k[off + e] : 0;
+                        tv[e] = in ? a.v[off + e] : 0;
                     }
+                    rk[i] = *reinterpret_cast<const uint4*>(tk);
+                    rv[i] = *reinterpret_cast<const uint4*>(tv);
                 }
             }
         }
@@ -188,6 +199,34 @@ __global__ void __launch_bounds__(kThreads, 1) k_flash(AttnArgs a) {
             mbuf[stage * kKvBlk + tid] = kv < a.Skv ? mask_at(a.mask, a.mask_f32, b * a.Skv + kv) : 1.0f;
         }
     };
+    // The bias of a block as this lane's scores need it (four keys per tile): loaded with the block's
+    // K and V, one 8-byte load per tile where rows are 8-byte aligned. Keys past the end read the
+    // last valid ones; their scores become -inf.
+    uint2 braw[kKT][kQT];
+    auto load_bias = [&](int blk) {
+        if (!a.bias) return;
+        const bf16_t* brow[kQT];
+#pragma unroll
+        for (int u = 0; u < kQT; ++u) brow[u] = a.bias + (h * a.Sq + min(q0 + u * 16 + c16, a.Sq - 1)) * a.Skv;
+        const int64_t kv0 = static_cast<int64_t>(blk) * kKvBlk + g * 4, last = a.Skv - 1;
+        if (a.bias_vec) {
+#pragma unroll
+            for (int u = 0; u < kQT; ++u)
+#pragma unroll
+                for (int t = 0; t < kKT; ++t)
+                    braw[t][u] = *reinterpret_cast<const uint2*>(brow[u] + min(kv0 + t * 16, a.Skv - 4));
+            return;
+        }
+#pragma unroll
+        for (int u = 0; u < kQT; ++u)
+#pragma unroll
+            for (int t = 0; t < kKT; ++t) {
+                const int64_t kv = kv0 + t * 16;
+                const uint32_t v0 = brow[u][min(kv, last)], v1 = brow[u][min(kv + 1, last)];
+                const uint32_t v2 = brow[u][min(kv + 2, last)], v3 = brow[u][min(kv + 3, last)];
+                braw[t][u] = make_uint2(v0 | v1 << 16, v2 | v3 << 16);
+            }
+    };
     auto block_live = [&](int blk) { return !use_flags || !any_valid || blk_ok[blk] != 0; };
 
     // ---- online softmax state ----
@@ -209,6 +248,7 @@ __global__ void __launch_bounds__(kThreads, 1) k_flash(AttnArgs a) {
     while (blk < nblk && !block_live(blk)) ++blk;
     if (blk < nblk) {
         load_kv(blk);
+        load_bias(blk);
         store_kv(blk, 0);
     }
     __syncthreads();
@@ -244,28 +284,18 @@ __global__ void __launch_bounds__(kThreads, 1) k_flash(AttnArgs a) {
             }
         }
 
-        // the bias of this lane's four keys per (t, u): one 8-byte load when rows are 8-byte aligned
         float bvals[kKT][kQT][4];
         if (a.bias) {
 #pragma unroll
-            for (int u = 0; u < kQT; ++u) {
-                const int64_t qi = min(q0 + u * 16 + c16, a.Sq - 1);
-                const bf16_t* brow = a.bias + (h * a.Sq + qi) * a.Skv;
+            for (int u = 0; u < kQT; ++u)
 #pragma unroll
                 for (int t = 0; t < kKT; ++t) {
-                    const int64_t kv = kvb + t * 16 + g * 4;
-                    if (a.bias_vec && kv + 3 < a.Skv) {
-                        const uint2 raw = *reinterpret_cast<const uint2*>(brow + kv);
-                        bvals[t][u][0] = __uint_as_float(raw.x << 16);
-                        bvals[t][u][1] = __uint_as_float(raw.x & 0xffff0000u);
-                        bvals[t][u][2] = __uint_as_float(raw.y << 16);
-                        bvals[t][u][3] = __uint_as_float(raw.y & 0xffff0000u);
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) bvals[t][u][r] = kv + r < a.Skv ? bf2f(brow[kv + r]) : 0.0f;
-                    }
+                    bvals[t][u][0] = __uint_as_float(braw[t][u].x << 16);
+                    bvals[t][u][1] = __uint_as_float(braw[t][u].x & 0xffff0000u);
+                    bvals[t][u][2] = __uint_as_float(braw[t][u].y << 16);
+                    bvals[t][u][3] = __uint_as_float(braw[t][u].y & 0xffff0000u);
                 }
-            }
+            if (next < nblk) load_bias(next);
         }
         // scale, mask, running max, exponentials (base 2 with log2(e) folded into the scale)
         float mvals[kKT][4];
@@ -454,6 +484,16 @@ bf16_t* vt_workspace(size_t elems) {
     return static_cast<bf16_t*>(ptr[dev]);
 }
 
+// Query tiles per wave of the generic flash kernel: 4 (each K/V fragment read feeds four MFMAs) where
+// that makes four workgroups or more per CU; else 1, four times the workgroups and a quarter of the
+// work in each (a workgroup's key blocks run one after another, so its time sets the launch's), and
+// less padding in the last query block. T5 at 64 heads: 120 queries 17 -> 8.6 us, 2 x 300 queries 37 -> 31 us
+// in the encoder (16 us warm).
+int flash_query_tiles(const AttnShape& sh) {
+    const int64_t big = sh.batch * sh.heads * ((sh.q_len + 255) / 256);
+    return big >= 1024 ? 4 : 1;
+}
+
 // Which kernel launch_attention_bf16 runs for these operands, and the V^T elements it needs.
 struct AttnPlan {
     enum Kind { FLASH512, FLASH72, FLASH } kind;
@@ -559,8 +599,11 @@ void launch_attention_bf16(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf
     // 16-byte fragment reads of 8 consecutive rows are conflict-free when the row is an odd
     // multiple of 16 bytes; pad a row that is a multiple of 32 bytes by 16 bytes.
     a.k_row = (d8 % 16 == 0) ? d8 + 8 : d8;
-    a.v_row = kKvBlk + 8;
-    a.qb = static_cast<int>((sh.q_len + kQRows - 1) / kQRows);
+    // V^T rows of 136 bytes: the transposed 2-byte writes of a wave (8 chunks of 8 rows) then meet
+    // two to a bank instead of four, and 16 rows' 8-byte reads touch all banks once.
+    a.v_row = kKvBlk + 4;
+    const int qt = flash_query_tiles(sh);
+    a.qb = static_cast<int>((sh.q_len + 64 * qt - 1) / (64 * qt));
     const int ks = static_cast<int>((sh.head_dim + 31) / 32);
     const int dt = static_cast<int>((sh.head_dim + 15) / 16);
     const size_t lds = sizeof(bf16_t) * 2 * (kKvBlk * a.k_row + dt * 16 * a.v_row) +
@@ -570,21 +613,20 @@ void launch_attention_bf16(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf
                          sh.head_dim;
     ProfileScope ps(sh.q_len == sh.kv_len ? K_ATTN_SELF : K_ATTN_CROSS, s, flops);
     // Above 64 KiB of dynamic LDS (head_dim > 96) the launch must opt in to the larger size.
+#define BH_FLASH_K(KS_, DT_, VEC_, QT_)                                                    \
+    do {                                                                                   \
+        if (lds > 65536)                                                                   \
+            hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_flash<KS_, DT_, VEC_, QT_>), \
+                                          hipFuncAttributeMaxDynamicSharedMemorySize,      \
+                                          static_cast<int>(lds)), "hipFuncSetAttribute");  \
+        k_flash<KS_, DT_, VEC_, QT_><<<grid, kThreads, lds, s>>>(a);                       \
+    } while (0)
 #define BH_FLASH(KS_, DT_)                                                                 \
     do {                                                                                   \
-        if (vec) {                                                                         \
-            if (lds > 65536)                                                               \
-                hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_flash<KS_, DT_, true>), \
-                                              hipFuncAttributeMaxDynamicSharedMemorySize,  \
-                                              static_cast<int>(lds)), "hipFuncSetAttribute"); \
-            k_flash<KS_, DT_, true><<<grid, kThreads, lds, s>>>(a);                        \
-        } else {                                                                           \
-            if (lds > 65536)                                                               \
-                hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_flash<KS_, DT_, false>), \
-                                              hipFuncAttributeMaxDynamicSharedMemorySize,  \
-                                              static_cast<int>(lds)), "hipFuncSetAttribute"); \
-            k_flash<KS_, DT_, false><<<grid, kThreads, lds, s>>>(a);                       \
-        }                                                                                  \
+        if (vec && qt == 4) BH_FLASH_K(KS_, DT_, true, 4);                                 \
+        else if (vec) BH_FLASH_K(KS_, DT_, true, 1);                                       \
+        else if (qt == 4) BH_FLASH_K(KS_, DT_, false, 4);                                  \
+        else BH_FLASH_K(KS_, DT_, false, 1);                                               \
     } while (0)
     if (ks == 1 && dt == 1) BH_FLASH(1, 1);
     else if (ks == 1) BH_FLASH(1, 2);
@@ -595,6 +637,7 @@ void launch_attention_bf16(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf
     else if (dt == 7) BH_FLASH(4, 7);
     else BH_FLASH(4, 8);
 #undef BH_FLASH
+#undef BH_FLASH_K
     launch_check("attention (flash)");
 }
 

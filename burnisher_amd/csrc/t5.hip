@@ -3,6 +3,7 @@
 // gated GELU run on the shared kernels.
 #include "common.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace bh {
@@ -63,19 +64,39 @@ __global__ void __launch_bounds__(256) k_gather(const T* __restrict__ table,
 }
 
 // bias[h, q, k] = rel[bucket[k - q + S - 1], h]: rel is [buckets, heads] (the checkpoint layout),
-// bucket holds the 2S-1 relative positions' buckets. 8 keys per thread, one 16-byte store.
+// bucket holds the 2S-1 relative positions' buckets. A head per blockIdx.y: its biases of all
+// relative positions are gathered into LDS once, then every row of the head is a window of them,
+// eight keys a thread, one 16-byte store where rows are 16-byte aligned. A value gathered per key
+// from global memory (two dependent loads each, two-byte stores) took 31 us at 64 heads x 300.
+constexpr int kRelMax = 16384;   // 2S - 1 of the largest sequence the encoder takes (8192)
+
 __global__ void __launch_bounds__(256) k_rel_bias(const bf16_t* __restrict__ rel,
                                                   const int* __restrict__ bucket,
-                                                  bf16_t* __restrict__ bias, int64_t heads,
-                                                  int64_t S) {
-    const int64_t per_row = (S + 7) / 8, n = heads * S * per_row;
-    for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < n;
-         i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-        const int64_t row = i / per_row, k0 = (i - row * per_row) * 8;
-        const int64_t h = row / S, q = row - h * S;
-        bf16_t* dst = bias + row * S + k0;
-        for (int e = 0; e < 8 && k0 + e < S; ++e)
-            dst[e] = rel[static_cast<int64_t>(bucket[k0 + e - q + S - 1]) * heads + h];
+                                                  bf16_t* __restrict__ bias, int heads, int S, int vec) {
+    extern __shared__ bf16_t pos[];   // [2S - 1]
+    const int h = blockIdx.y;
+    for (int i = threadIdx.x; i < 2 * S - 1; i += 256) pos[i] = rel[static_cast<int64_t>(bucket[i]) * heads + h];
+    __syncthreads();
+    const int per_row = (S + 7) / 8;
+    bf16_t* head = bias + static_cast<int64_t>(h) * S * S;
+    for (int64_t i = blockIdx.x * 256 + threadIdx.x; i < static_cast<int64_t>(S) * per_row; i += gridDim.x * 256) {
+        const int q = static_cast<int>(i / per_row), k0 = static_cast<int>(i - static_cast<int64_t>(q) * per_row) * 8;
+        bf16_t* dst = head + static_cast<int64_t>(q) * S + k0;
+        const bf16_t* src = pos + k0 - q + S - 1;
+        if (vec == 8) {
+            uint32_t w[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = src[2 * e] | static_cast<uint32_t>(src[2 * e + 1]) << 16;
+            *reinterpret_cast<uint4*>(dst) = make_uint4(w[0], w[1], w[2], w[3]);
+        } else if (vec == 4) {
+#pragma unroll
+            for (int e = 0; e < 8; e += 4)
+                if (k0 + e < S)
+                    *reinterpret_cast<uint2*>(dst + e) = make_uint2(src[e] | static_cast<uint32_t>(src[e + 1]) << 16,
+                                                                    src[e + 2] | static_cast<uint32_t>(src[e + 3]) << 16);
+        } else {
+            for (int e = 0; e < 8 && k0 + e < S; ++e) dst[e] = src[e];
+        }
     }
 }
 
@@ -110,8 +131,15 @@ void launch_gather(const void* table, const float* ids, void* out, int64_t rows,
 void launch_rel_bias(const bf16_t* rel, const int* bucket, bf16_t* bias, int64_t heads, int64_t S,
                      hipStream_t s) {
     if (heads * S == 0) return;
+    require(2 * S - 1 < kRelMax && heads <= 65535, "relative bias: sequence or heads out of range");
     ProfileScope ps(K_ELEMENTWISE, s, 2.0 * heads * S * S);
-    k_rel_bias<<<grid_of(heads * S * ((S + 7) / 8)), 256, 0, s>>>(rel, bucket, bias, heads, S);
+    const int64_t items = S * ((S + 7) / 8);
+    const int vec = !aligned16(bias) ? 1 : S % 8 == 0 ? 8 : S % 4 == 0 ? 4 : 1;
+    // a few passes of each workgroup over its head, which pay for gathering the head's positions
+    const dim3 grid(static_cast<unsigned>(std::max<int64_t>(1, std::min<int64_t>(64, (items + 1023) / 1024))),
+                    static_cast<unsigned>(heads));
+    k_rel_bias<<<grid, 256, static_cast<size_t>(2 * S - 1) * sizeof(bf16_t), s>>>(
+        rel, bucket, bias, static_cast<int>(heads), static_cast<int>(S), vec);
     launch_check("relative bias");
 }
 

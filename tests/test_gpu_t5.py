@@ -53,7 +53,8 @@ def test_gather_bit_identical(hip, cols):
     assert np.array_equal(o32.cpu().numpy(), t32[[1, 2, 3, 49]])
 
 
-@pytest.mark.parametrize("shape", [(2, 4, 37, 64), (2, 8, 300, 64), (1, 3, 70, 16)],
+@pytest.mark.parametrize("shape", [(2, 4, 37, 64), (2, 8, 300, 64), (1, 3, 70, 16), (2, 512, 70, 64),
+                                   (1, 1024, 33, 30)],
                          ids=lambda s: "x".join(map(str, s)))
 def test_attention_with_relative_bias_and_mask(hip, shape):
     import torch
@@ -118,10 +119,11 @@ def check(got, want, where):
 
 @pytest.mark.parametrize("cfg,batch,seq,lengths", [
     (SMALL, 2, 9, [3, 9]),
+    (dict(SMALL, num_layers=1), 2, 44, [3, 44]),   # relative-bias rows stored 8 bytes at a time
     (dict(SMALL, gated=0, num_layers=1), 2, 9, [9, 5]),
     (dict(SMALL, d_model=256, d_ff=640, d_kv=64, num_heads=4, vocab_size=1000, num_layers=3), 2, 77, [1, 40]),
     (dict(T5_XXL, num_layers=1), 2, 48, [1, 30]),
-], ids=["small", "plain_gelu", "mid", "xxl_widths_1layer"])
+], ids=["small", "small_44", "plain_gelu", "mid", "xxl_widths_1layer"])
 def test_encoder_matches_oracle(hip, cfg, batch, seq, lengths):
     wl = make_t5_workload(cfg, batch=batch, seq=seq, lengths=lengths, seed=9)
     check(device_encode(wl), stock_encode(wl), f"{cfg['d_model']}x{cfg['num_layers']} B{batch} S{seq}")
