@@ -244,6 +244,8 @@ struct GemmEpilogue {
     int splitk = 0;
     float* splitk_ws = nullptr;
     int64_t splitk_ws_floats = 0;
+    // A second output, silu(out) rounded, [m, n]: at most 8 rows, K a multiple of 8.
+    bf16_t* silu_out = nullptr;
 };
 
 // A channel of a GroupNorm: its group's mean and 1 / sqrt(var + eps), and its own affine.
@@ -520,6 +522,25 @@ void launch_patch(const void* in, void* out, int64_t batch, int64_t channels, in
 // Cos-first sinusoidal timestep embedding, fp64, rounded to bf16, broadcast to `batch` rows
 // (weights.cpp:107-121 and the host broadcast at pixart_dit.cpp:156-160).
 void launch_timestep_embedding(double t, int dim, int64_t batch, void* out, bool f32, hipStream_t s);
+// The engine's first launch: patchify (2 x 2 patches of 4 channels), patch embedding, position table
+// and timestep embedding (256 wide, `batch` rows), the bits of launch_patch + launch_gemm_bf16 +
+// launch_timestep_embedding.
+bool dit_embed_supported(const void* latent, const void* w, const void* pos, int64_t in_channels, int64_t patch,
+                         int64_t rows, int64_t cols);
+void launch_dit_embed(const void* latent, const bf16_t* w, const bf16_t* bias, const bf16_t* pos, bf16_t* x,
+                      int64_t batch, int64_t grid, int64_t cols, double t, bf16_t* temb, hipStream_t s);
+// The engine's last launch: LayerNorm, modulation by emb + table rows 0 (shift) and 1 (scale), the
+// projection to n = channels * patch^2 columns and unpatchify, the bits of the separate launches.
+bool dit_head_supported(int64_t rows, int64_t cols, int64_t n, const void* w, const void* bias);
+void launch_dit_head(const bf16_t* x, const bf16_t* emb, const bf16_t* table, const bf16_t* w, const bf16_t* bias,
+                     bf16_t* out, int64_t batch, int64_t grid, int64_t cols, int64_t channels, int64_t patch,
+                     float eps, hipStream_t s);
+// The adaLN projection of at most 8 rows and every layer's chunks of it (launch_gemm_bf16 to
+// [batch, 6 channels], then launch_chunk_all) in one launch. Every table 16-byte aligned.
+bool adaln_chunks_supported(int64_t batch, int64_t channels, const void* w);
+void launch_adaln_chunks(const bf16_t* a, const bf16_t* w, const bf16_t* bias, const bf16_t* const* tables_dev,
+                         bf16_t* out, float* out_f32, int64_t layers, int64_t batch, int64_t channels,
+                         hipStream_t s);
 // ScaleArgs: out[i] = in[i] * scale, one rounding (out may alias in).
 void launch_scale(const void* in, void* out, int64_t n, float scale, bool f32, hipStream_t s);
 

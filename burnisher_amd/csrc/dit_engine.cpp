@@ -35,6 +35,8 @@
 namespace bh {
 namespace {
 
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
 struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
@@ -112,6 +114,7 @@ struct bh_dit {
 
     DevBuf pos_table, patches, x, normed, modded, q, k, v, qkv, ctx, proj, q2, kc, vc, ff0;
     DevBuf temb, h_t, emb_t, silu_t, modulation, cap_h, cap, kv_all, chunks, tables_dev;
+    bool tables_aligned = true;   // every layer's table may be read 16 bytes at a time
     DevBuf chunks_f32;   // the chunks as floats, scales as 1 + scale (fused norm kernel)
     DevBuf shift, scale, gate, zero, tokens;
     // The fused plan's packed projections: every layer's [3d, d] Q/K/V weight and [3d] bias, and
@@ -320,31 +323,47 @@ void forward_fused(bh_dit& e, const void* latent, double t, const void* caption,
     const float eps = static_cast<float>(c.eps);
     const GemmEpilogue plain;
 
-    {
-        ProfileScope ps(K_ELEMENTWISE, s, 4.0 * e.B * e.N * e.patch_in);
-        launch_patch(latent, e.patches.p, B, c.in_channels, e.grid, P, false, false, s);
-    }
-    {   // patch embedding, then + position table (AddArgs broadcast over the batch)
+    // patch embedding, then + position table (AddArgs broadcast over the batch); timestep embedding
+    if (M > 8 && dit_embed_supported(latent, e.w.pos_embed_w, e.pos_table.p, c.in_channels, P, M, d)) {
+        ProfileScope ps(K_GEMM, s, 2.0 * M * d * e.patch_in);
+        launch_dit_embed(latent, static_cast<const bf16_t*>(e.w.pos_embed_w), static_cast<const bf16_t*>(e.w.pos_embed_b),
+                         e.pos_table.bf(), e.x.bf(), B, e.grid, d, t, e.temb.bf(), s);
+    } else {
+        {
+            ProfileScope ps(K_ELEMENTWISE, s, 4.0 * M * e.patch_in);
+            launch_patch(latent, e.patches.p, B, c.in_channels, e.grid, P, false, false, s);
+        }
         GemmEpilogue ep;
         ep.round_mid = true;
         ep.row_add = e.pos_table.bf();
         ep.row_add_period = N;
         gemm(e, e.patches.bf(), e.w.pos_embed_w, e.w.pos_embed_b, e.x.bf(), M, d, e.patch_in, ep, s);
+        ProfileScope ps(K_ELEMENTWISE, s, 2.0 * B * 256);
+        launch_timestep_embedding(t, 256, B, e.temb.p, false, s);
     }
-    {   // adaLN-single: one modulation vector per step
-        {
-            ProfileScope ps(K_ELEMENTWISE, s, 2.0 * B * 256);
-            launch_timestep_embedding(t, 256, B, e.temb.p, false, s);
-        }
+    // adaLN-single: one modulation vector per step, and every layer's chunks of it
+    {
         GemmEpilogue silu;
         silu.act = 2;
         gemm(e, e.temb.bf(), e.w.t_emb1_w, e.w.t_emb1_b, e.h_t.bf(), B, d, 256, silu, s);
+    }
+    const bf16_t* const* tables = static_cast<const bf16_t* const*>(e.tables_dev.p);
+    if (e.tables_aligned && adaln_chunks_supported(B, d, e.w.adaln_w) && aligned16(e.w.t_emb2_w)) {
+        GemmEpilogue two;
+        two.silu_out = e.silu_t.bf();
+        gemm(e, e.h_t.bf(), e.w.t_emb2_w, e.w.t_emb2_b, e.emb_t.bf(), B, d, d, two, s);
+        launch_adaln_chunks(e.silu_t.bf(), static_cast<const bf16_t*>(e.w.adaln_w),
+                            static_cast<const bf16_t*>(e.w.adaln_b), tables, e.chunks.bf(),
+                            static_cast<float*>(e.chunks_f32.p), L, B, d, s);
+    } else {
         gemm(e, e.h_t.bf(), e.w.t_emb2_w, e.w.t_emb2_b, e.emb_t.bf(), B, d, d, plain, s);
         {
             ProfileScope ps(K_ELEMENTWISE, s, 4.0 * B * d);
             launch_activation(e.emb_t.p, e.silu_t.p, B * d, 2, nullptr, false, s);
         }
         gemm(e, e.silu_t.bf(), e.w.adaln_w, e.w.adaln_b, e.modulation.bf(), B, 6 * d, d, plain, s);
+        ProfileScope ps(K_ELEMENTWISE, s, 2.0 * (B * 6 * d + L * 6 * d + L * 6 * B * d));
+        launch_chunk_all(e.modulation.bf(), tables, e.chunks.bf(), static_cast<float*>(e.chunks_f32.p), L, B, d, s);
     }
     if (!caption_ready) {   // caption projection, then every layer's cross-attention K and V
         GemmEpilogue gelu;
@@ -363,11 +382,6 @@ void forward_fused(bh_dit& e, const void* latent, double t, const void* caption,
             kv.vt_dim = c.head_dim;
         }
         gemm(e, e.cap.bf(), e.kv_w, e.kv_b, e.kv_all.bf(), e.Mcap, L * 2 * d, d, kv, s);
-    }
-    {
-        ProfileScope ps(K_ELEMENTWISE, s, 2.0 * (B * 6 * d + L * 6 * d + L * 6 * B * d));
-        launch_chunk_all(e.modulation.bf(), static_cast<const bf16_t* const*>(e.tables_dev.p),
-                         e.chunks.bf(), static_cast<float*>(e.chunks_f32.p), L, B, d, s);
     }
     const float scale = 1.0f / std::sqrt(static_cast<float>(Dh));
     const bool mask_f32 = mask_dtype == BH_F32;
@@ -535,6 +549,14 @@ void forward_fused(bh_dit& e, const void* latent, double t, const void* caption,
     }
 
     // output head: shift = emb_t + table[0], scale = emb_t + table[1] (pixart_dit.cpp:287-294)
+    const bf16_t* head_table = static_cast<const bf16_t*>(e.w.out_table);
+    if (aligned16(head_table) && dit_head_supported(M, d, e.patch_out, e.w.proj_out_w, e.w.proj_out_b)) {
+        ProfileScope ps(K_GEMM, s, 2.0 * M * d * e.patch_out);
+        launch_dit_head(e.x.bf(), e.emb_t.bf(), head_table, static_cast<const bf16_t*>(e.w.proj_out_w),
+                        static_cast<const bf16_t*>(e.w.proj_out_b), static_cast<bf16_t*>(out), B, e.grid, d,
+                        c.out_channels, P, eps, s);
+        return;
+    }
     {
         ProfileScope ps(K_ELEMENTWISE, s, 6.0 * B * d);
         launch_chunk(e.emb_t.p, e.w.out_table, e.shift.p, B, d, 1, 0, 0, false, s);
@@ -713,6 +735,7 @@ int bh_dit_create(const bh_dit_config* cfg, const bh_dit_weights* w, int64_t bat
                     d2d(bk + bb, bw.attn2_v_b, bb, nullptr);
                 }
                 tables[l] = static_cast<const bf16_t*>(bw.scale_shift_table);
+                e->tables_aligned = e->tables_aligned && aligned16(tables[l]);
             }
             e->kv_w = kv_packed ? static_cast<const bf16_t*>(e->blocks[0].attn2_k_w) : e->w_kv.bf();
             e->kv_b = kv_packed ? static_cast<const bf16_t*>(e->blocks[0].attn2_k_b) : e->b_kv.bf();

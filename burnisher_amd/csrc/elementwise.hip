@@ -718,7 +718,7 @@ __device__ inline void store_f64(float* p, int64_t i, double v) { p[i] = static_
 __device__ inline void store_f64(bf16_t* p, int64_t i, double v) { p[i] = bf16_from_f64(v); }
 
 template <typename T>
-__global__ void k_timestep_embedding(double t, int dim, int64_t batch, T* out) {
+__device__ __forceinline__ void timestep_row(double t, int dim, int64_t batch, T* out) {
     const int half = dim / 2;
     for (int i = threadIdx.x; i < half; i += blockDim.x) {
         const double freq = exp(-log(10000.0) * static_cast<double>(i) / half);
@@ -728,6 +728,197 @@ __global__ void k_timestep_embedding(double t, int dim, int64_t batch, T* out) {
             store_f64(out, b * dim + i, c);
             store_f64(out, b * dim + half + i, s);
         }
+    }
+}
+template <typename T>
+__global__ void k_timestep_embedding(double t, int dim, int64_t batch, T* out) {
+    timestep_row(t, dim, batch, out);
+}
+
+// The DiT's first launch: patchify, the patch embedding (K = 16: 2 x 2 pixels of 4 channels), the
+// position table's row, and in the last workgroup the timestep embedding. A wave owns 128 output
+// columns (two a lane, their weights in registers) and a band of tokens: the token's 16 inputs are
+// the same for all its lanes, so they come straight from the latent as scalar loads, eight pixel
+// pairs each, four tokens in flight. Products and sums in the order (and rounding) of the small-K
+// GEMM, so the bits are those of patchify + GEMM + embedding in three launches.
+constexpr int kEmbedCols = 128, kEmbedUnroll = 4;
+
+__global__ void __launch_bounds__(256) k_dit_embed(
+    const uint32_t* __restrict__ latent, const bf16_t* __restrict__ w, const bf16_t* __restrict__ bias,
+    const bf16_t* __restrict__ pos, bf16_t* __restrict__ x, int rows, int tokens, int cols, int grid, int band,
+    double t, int batch, bf16_t* __restrict__ temb) {
+    if (blockIdx.x == gridDim.x - 1) {
+        timestep_row(t, 256, batch, temb);
+        return;
+    }
+    const int chunks = (cols + kEmbedCols - 1) / kEmbedCols;
+    const int id = static_cast<int>(blockIdx.x) * 4 + wave_index();
+    const int m0 = id / chunks * band, m1 = min(rows, m0 + band);
+    const int n = id % chunks * kEmbedCols + static_cast<int>(threadIdx.x % kWave) * 2;
+    if (m0 >= rows || n >= cols) return;
+    float wf[2][16], bf[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const V8 v = load8(w + static_cast<int64_t>(n + r) * 16 + h * 8);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) wf[r][h * 8 + e] = v.f[e];
+        }
+        bf[r] = bias ? bf2f(bias[n + r]) : -0.0f;   // v + (-0.0) is v exactly
+    }
+    for (int m = m0; m < m1; m += kEmbedUnroll) {
+        uint32_t a[kEmbedUnroll][8], add[kEmbedUnroll];
+#pragma unroll
+        for (int i = 0; i < kEmbedUnroll; ++i) {
+            const int row = min(m + i, m1 - 1), b = row / tokens, tok = row - b * tokens;
+            const int ty = tok / grid, tx = tok - ty * grid;
+            // pixel pairs: a latent row is `grid` of them, a channel 2 grid rows
+            const uint32_t* p = latent + (static_cast<int64_t>(b) * 8 * grid + 2 * ty) * grid + tx;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int ky = 0; ky < 2; ++ky)
+                    a[i][c * 2 + ky] = p[(static_cast<int64_t>(c) * 2 * grid + ky) * grid];
+            add[i] = *reinterpret_cast<const uint32_t*>(pos + static_cast<int64_t>(tok) * cols + n);
+        }
+#pragma unroll
+        for (int i = 0; i < kEmbedUnroll; ++i) {
+            float v[2];
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                float acc = 0.f;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    acc = __fadd_rn(acc, __fmul_rn(__uint_as_float(a[i][k] << 16), wf[r][2 * k]));
+                    acc = __fadd_rn(acc, __fmul_rn(__uint_as_float(a[i][k] & 0xffff0000u), wf[r][2 * k + 1]));
+                }
+                const float pe = r ? __uint_as_float(add[i] & 0xffff0000u) : __uint_as_float(add[i] << 16);
+                v[r] = __fadd_rn(round_bf16(__fadd_rn(acc, bf[r])), pe);
+            }
+            if (m + i < m1)
+                *reinterpret_cast<uint32_t*>(x + static_cast<int64_t>(m + i) * cols + n) = f2bf2(v[0], v[1]);
+        }
+    }
+}
+
+// ---- the DiT's output head --------------------------------------------------------------------
+//
+// LayerNorm, shift and 1 + scale (emb + table rows 0 and 1, rounded as the chunk op stores them),
+// the projection to a patch and unpatchify, for 16 token rows per workgroup: the modulated rows
+// and the projected ones stay in LDS. As two chunk launches, a norm, a GEMM (whose 32 output
+// columns fill a quarter of one column tile) and an unpatchify pass the same work was five
+// launches, none of them long enough to hide its own start. One wave owns 16 output columns and walks K in the GEMM's
+// order, so every output has the bits of those five launches; its weight fragments are requested
+// before the norm, whose latency covers them. Rows: eight waves of two rows each.
+constexpr int kHeadRows = 16, kHeadMaxN = 128, kHeadMaxC = 1920;
+using bf16x8_t = __bf16 __attribute__((ext_vector_type(8)));
+using f32x4_t = float __attribute__((ext_vector_type(4)));
+
+template <int NV, int NP>
+__global__ void __launch_bounds__(512) k_dit_head(
+    const bf16_t* __restrict__ x, const bf16_t* __restrict__ emb, const bf16_t* __restrict__ table,
+    const bf16_t* __restrict__ w, const bf16_t* __restrict__ bias, bf16_t* __restrict__ out, int rows,
+    int tokens, float eps, int n, int grid, int channels, int patch) {
+    using Row = NormRow<NV, NP>;
+    constexpr int kE = Row::kE, kC = kE * kWave;
+    constexpr int kStride = kC * 2 + 16;      // 16 bytes of padding: 16 rows' fragments meet no bank twice
+    constexpr int kSteps = kC / 32;
+    constexpr int kAhead = kSteps < 24 ? kSteps : 24;   // weight fragments in flight
+    __shared__ __attribute__((aligned(16))) char modded[kHeadRows * kStride];
+    __shared__ bf16_t proj[kHeadRows * kHeadMaxN];
+    const int lane = threadIdx.x % kWave, wave = wave_index();
+    const int r0 = blockIdx.x * kHeadRows;
+    const bool mul = wave * 16 < n;
+    const bf16_t* wp = w + static_cast<int64_t>(mul ? wave * 16 + (lane & 15) : 0) * kC + (lane >> 4) * 8;
+    bf16x8_t wf[kAhead];
+    if (mul) {
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) wf[i] = *reinterpret_cast<const bf16x8_t*>(wp + i * 32);
+    }
+    Row in[2], t0, t1;
+    int row[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        row[k] = min(r0 + wave * 2 + k, rows - 1);   // rows past the end repeat the last one, unstored
+        in[k].load(x + static_cast<int64_t>(row[k]) * kC, lane);
+    }
+    t0.load(table, lane);
+    t1.load(table + kC, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    auto at = [](const Row& r, int e) -> float {
+        const uint32_t v = r.raw[e >> 1];
+        return (e & 1) ? __uint_as_float(v & 0xffff0000u) : __uint_as_float(v << 16);
+    };
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        Row em;
+        em.load(emb + static_cast<int64_t>(row[k] / tokens) * kC, lane);
+        double sum = 0.0;
+#pragma unroll
+        for (int e = 0; e < kE; ++e) sum += static_cast<double>(at(in[k], e));
+        const double mean = wave_sum(sum) / static_cast<double>(kC);
+#pragma unroll
+        for (int i = 0; i < kE / 2; ++i) asm volatile("" : "+v"(in[k].raw[i]));
+        double q = 0.0;
+#pragma unroll
+        for (int e = 0; e < kE; ++e) {
+            const double d = static_cast<double>(at(in[k], e)) - mean;
+            q += d * d;
+        }
+        const double var = wave_sum(q) / static_cast<double>(kC);
+        const float inv = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(static_cast<float>(var), eps)));
+        const float fmean = static_cast<float>(mean);
+        uint32_t o[kE / 2];
+#pragma unroll
+        for (int i = 0; i < kE / 2; ++i) {
+            float v[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int e = 2 * i + h;
+                const float sh = round_bf16(__fadd_rn(at(em, e), at(t0, e)));
+                const float sc = round_bf16(__fadd_rn(at(em, e), at(t1, e)));
+                const float nrm = round_bf16(__fmul_rn(__fsub_rn(at(in[k], e), fmean), inv));
+                v[h] = __fadd_rn(__fmul_rn(nrm, __fadd_rn(1.0f, sc)), sh);
+            }
+            o[i] = f2bf2(v[0], v[1]);
+        }
+        char* dst = modded + (wave * 2 + k) * kStride;
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+            *reinterpret_cast<uint4*>(dst + (lane + j * kWave) * 16) =
+                make_uint4(o[4 * j], o[4 * j + 1], o[4 * j + 2], o[4 * j + 3]);
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+            *reinterpret_cast<uint32_t*>(dst + (NV * kWave * 8 + (p * kWave + lane) * 2) * 2) = o[4 * NV + p];
+    }
+    __syncthreads();
+    if (mul) {
+        const char* ap = modded + (lane & 15) * kStride + (lane >> 4) * 16;
+        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < kSteps; ++i) {
+            const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(ap + i * 64);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i % kAhead], a, acc, 0, 0, 0);
+            if (i + kAhead < kSteps) wf[i % kAhead] = *reinterpret_cast<const bf16x8_t*>(wp + (i + kAhead) * 32);
+        }
+        const int n0 = wave * 16 + (lane >> 4) * 4;   // this lane: columns n0 .. n0 + 3 of row lane & 15
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float b = bias ? bf2f(bias[n0 + r]) : -0.0f;   // v + (-0.0) is v exactly
+            proj[(lane & 15) * n + n0 + r] = f2bf(__fadd_rn(acc[r], b));
+        }
+    }
+    __syncthreads();
+    // unpatchify: token layout (ky, kx, c); consecutive threads along an image row
+    const int side = grid * patch;
+    for (int i = threadIdx.x; i < kHeadRows * n; i += 512) {
+        const int kx = i % patch, t = i / patch % kHeadRows, cy = i / (patch * kHeadRows);
+        const int c = cy / patch, ky = cy % patch, r = r0 + t;
+        if (r >= rows) continue;
+        const int b = r / tokens, tok = r % tokens, ty = tok / grid, tx = tok % grid;
+        out[((static_cast<int64_t>(b) * channels + c) * side + ty * patch + ky) * side + tx * patch + kx] =
+            proj[t * n + (ky * patch + kx) * channels + c];
     }
 }
 
@@ -1036,6 +1227,58 @@ void launch_patch(const void* in, void* out, int64_t batch, int64_t channels, in
                                                     grid, patch, inverse);
     }
     launch_check("patch");
+}
+
+bool dit_embed_supported(const void* latent, const void* w, const void* pos, int64_t in_channels, int64_t patch,
+                         int64_t rows, int64_t cols) {
+    return in_channels == 4 && patch == 2 && cols % 2 == 0 && rows < (int64_t{1} << 24) && cols < (int64_t{1} << 16) &&
+           (reinterpret_cast<uintptr_t>(latent) & 3) == 0 && aligned16(w) && aligned16(pos);
+}
+
+void launch_dit_embed(const void* latent, const bf16_t* w, const bf16_t* bias, const bf16_t* pos, bf16_t* x,
+                      int64_t batch, int64_t grid, int64_t cols, double t, bf16_t* temb, hipStream_t s) {
+    const int64_t tokens = grid * grid, rows = batch * tokens;
+    const int64_t chunks = (cols + kEmbedCols - 1) / kEmbedCols;
+    // Tokens per wave: the weights a wave loads (4 KiB) are worth many tokens, the chip wants about
+    // two waves a SIMD. 4 at 1024 tokens, 32 from 8192 on.
+    const int64_t band =
+        std::max<int64_t>(kEmbedUnroll, std::min<int64_t>(32, rows * chunks / 2048 / kEmbedUnroll * kEmbedUnroll));
+    const int64_t waves = (rows + band - 1) / band * chunks;
+    k_dit_embed<<<static_cast<int>((waves + 3) / 4 + 1), 256, 0, s>>>(
+        static_cast<const uint32_t*>(latent), w, bias, pos, x, static_cast<int>(rows), static_cast<int>(tokens),
+        static_cast<int>(cols), static_cast<int>(grid), static_cast<int>(band), t, static_cast<int>(batch), temb);
+    launch_check("dit_embed");
+}
+
+bool dit_head_supported(int64_t rows, int64_t cols, int64_t n, const void* w, const void* bias) {
+    // more than 8 rows: fewer take the small-M GEMM, which sums K in another order
+    return rows > 8 && rows < (int64_t{1} << 31) - kHeadRows && cols % 128 == 0 && cols <= kHeadMaxC && n % 16 == 0 &&
+           n <= kHeadMaxN && aligned16(w) && aligned16(bias);
+}
+
+void launch_dit_head(const bf16_t* x, const bf16_t* emb, const bf16_t* table, const bf16_t* w, const bf16_t* bias,
+                     bf16_t* out, int64_t batch, int64_t grid, int64_t cols, int64_t channels, int64_t patch,
+                     float eps, hipStream_t s) {
+    const int64_t rows = batch * grid * grid, n = channels * patch * patch;
+    require(dit_head_supported(rows, cols, n, w, bias) && aligned16(x) && aligned16(emb) && aligned16(table),
+            "dit_head: shape or alignment");
+    const int blocks = static_cast<int>((rows + kHeadRows - 1) / kHeadRows);
+#define BH_HEAD(NV, NP)                                                                              \
+    case NV * 4 + NP:                                                                                \
+        k_dit_head<NV, NP><<<blocks, 512, 0, s>>>(x, emb, table, w, bias, out, static_cast<int>(rows), \
+                                                  static_cast<int>(grid * grid), eps, static_cast<int>(n), \
+                                                  static_cast<int>(grid), static_cast<int>(channels), \
+                                                  static_cast<int>(patch));                          \
+        break;
+    switch (cols / 128) {
+        BH_HEAD(0, 1) BH_HEAD(0, 2) BH_HEAD(0, 3)
+        BH_HEAD(1, 0) BH_HEAD(1, 1) BH_HEAD(1, 2) BH_HEAD(1, 3)
+        BH_HEAD(2, 0) BH_HEAD(2, 1) BH_HEAD(2, 2) BH_HEAD(2, 3)
+        BH_HEAD(3, 0) BH_HEAD(3, 1) BH_HEAD(3, 2) BH_HEAD(3, 3)
+        default: break;
+    }
+#undef BH_HEAD
+    launch_check("dit_head");
 }
 
 void launch_scale(const void* in, void* out, int64_t n, float scale, bool f32, hipStream_t s) {

@@ -78,54 +78,106 @@ k_gemm_tn(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, bf16_t* ou
 // ---- small M: one wave per output column, both operands read with 16-byte loads ----
 constexpr int kGemvMaxM = 8;
 
-__global__ void __launch_bounds__(256) k_gemv(const bf16_t* __restrict__ A,
-                                              const bf16_t* __restrict__ B, bf16_t* out,
-                                              int64_t M, int64_t N, int64_t K, Epi e, int mode) {
-    const int lane = threadIdx.x & 63;
-    const int64_t n = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-    if (n >= N) return;
-    float part[kGemvMaxM];
+// The dot products of one weight row with M <= MM rows of A, every lane's sums over its octets in
+// order, then over the wave; valid in all lanes. What bounds these launches is the latency of
+// their loads (a wave reads a few KiB), so the octets of four rounds are requested together: with one round trip
+// per round the adaLN projection (6912 x 1152, 16 MB) took three of them.
+template <int MM>
+__device__ __forceinline__ void gemv_row(const bf16_t* __restrict__ A, const bf16_t* __restrict__ Bn, int M,
+                                         int64_t K, int lane, float (&part)[MM]) {
+    constexpr int U = MM <= 2 ? 4 : 1;
 #pragma unroll
-    for (int m = 0; m < kGemvMaxM; ++m) part[m] = 0.f;
+    for (int m = 0; m < MM; ++m) part[m] = 0.f;
     const int64_t chunks = K / 8;
-    for (int64_t c = lane; c < chunks; c += 64) {
-        const uint4 wb = *reinterpret_cast<const uint4*>(B + n * K + c * 8);
-        const uint32_t w[4] = {wb.x, wb.y, wb.z, wb.w};
-        float wf[8];
+    for (int64_t c0 = lane; c0 < chunks; c0 += 64 * U) {
+        uint4 wb[U], ab[U][MM];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            wf[2 * t] = __uint_as_float(w[t] << 16);
-            wf[2 * t + 1] = __uint_as_float(w[t] & 0xffff0000u);
+        for (int u = 0; u < U; ++u) {
+            const int64_t c = min(c0 + u * 64, chunks - 1);   // octets past the end are read again, unused
+            wb[u] = *reinterpret_cast<const uint4*>(Bn + c * 8);
+#pragma unroll
+            for (int m = 0; m < MM; ++m) ab[u][m] = *reinterpret_cast<const uint4*>(A + min(m, M - 1) * K + c * 8);
         }
+        __builtin_amdgcn_sched_barrier(0);   // every request before the first use
 #pragma unroll
-        for (int m = 0; m < kGemvMaxM; ++m) {
-            if (m < M) {
-                const uint4 ab = *reinterpret_cast<const uint4*>(A + m * K + c * 8);
-                const uint32_t a[4] = {ab.x, ab.y, ab.z, ab.w};
+        for (int u = 0; u < U; ++u) {
+            if (c0 + u * 64 >= chunks) break;
+            float wf[8];
+            unpack8(wb[u], wf);
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    part[m] += __uint_as_float(a[t] << 16) * wf[2 * t];
-                    part[m] += __uint_as_float(a[t] & 0xffff0000u) * wf[2 * t + 1];
-                }
+            for (int m = 0; m < MM; ++m) {
+                float af[8];
+                unpack8(ab[u][m], af);
+#pragma unroll
+                for (int t = 0; t < 8; ++t) part[m] += af[t] * wf[t];
             }
         }
     }
 #pragma unroll
-    for (int m = 0; m < kGemvMaxM; ++m) {
-        float v = part[m];
+    for (int m = 0; m < MM; ++m)
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-        part[m] = v;
-    }
+        for (int o = 32; o > 0; o >>= 1) part[m] += __shfl_xor(part[m], o, 64);
+}
+
+template <int MM>
+__global__ void __launch_bounds__(256) k_gemv(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, bf16_t* out,
+                                              int64_t M, int64_t N, int64_t K, Epi e, int mode, bf16_t* silu_out) {
+    const int lane = threadIdx.x & 63;
+    const int64_t n = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+    if (n >= N) return;
+    float part[MM];
+    gemv_row<MM>(A, B + n * K, static_cast<int>(M), K, lane, part);
     if (lane < M) {
         float a = 0.f;
 #pragma unroll
-        for (int m = 0; m < kGemvMaxM; ++m)
+        for (int m = 0; m < MM; ++m)
             if (m == lane) a = part[m];
         const int64_t m = lane;
         float v = e.bias ? __fadd_rn(a, bf2f(e.bias[n])) : a;
         v = finish(e, mode, act_exact(e.act, v), m, n, N);
-        out[m * e.ld_out + n] = f2bf(v);
+        const bf16_t o = f2bf(v);
+        out[m * e.ld_out + n] = o;
+        if (silu_out) silu_out[m * N + n] = f2bf(silu(bf2f(o)));
+    }
+}
+
+// The adaLN projection (n = 6 * channels columns of at most 8 rows) and what the blocks read of it:
+// for every layer, column + the layer's table, as bf16 and, for the norm kernels, as floats (the
+// scale chunks 1 and 4 as 1 + scale). A workgroup owns eight columns, so each layer's piece is one
+// 16-byte store (32 bytes of floats); the projection itself stays in LDS. Compared with a GEMV and a
+// pass over its output this saves a launch (4.6 us at one layer of 1152 channels) and the reread.
+template <int MM>
+__global__ void __launch_bounds__(512) k_adaln_chunks(
+    const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, const bf16_t* __restrict__ bias,
+    const bf16_t* const* __restrict__ tables, bf16_t* __restrict__ out, float* __restrict__ out_f32, int64_t layers,
+    int M, int64_t C) {
+    __shared__ float mod[MM][8];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t n0 = static_cast<int64_t>(blockIdx.x) * 8, n = n0 + wave;   // C % 8 == 0: one chunk a workgroup
+    float part[MM];
+    gemv_row<MM>(A, B + n * C, M, C, lane, part);
+#pragma unroll
+    for (int m = 0; m < MM; ++m)
+        if (lane == m) mod[m][wave] = round_bf16(bias ? __fadd_rn(part[m], bf2f(bias[n])) : part[m]);
+    __syncthreads();
+    const int64_t k = n0 / C, c = n0 - k * C;
+    for (int64_t i = threadIdx.x; i < layers * M; i += 512) {
+        const int64_t l = i / M;
+        const int m = static_cast<int>(i - l * M);
+        float t[8];
+        unpack8(*reinterpret_cast<const uint4*>(tables[l] + n0), t);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) t[q] = __fadd_rn(mod[m][q], t[q]);
+        const int64_t at = ((l * 6 + k) * M + m) * C + c;
+        *reinterpret_cast<uint4*>(out + at) = pack8(t);
+        if (out_f32) {
+            const bool scale = k == 1 || k == 4;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) t[q] = scale ? __fadd_rn(1.0f, round_bf16(t[q])) : round_bf16(t[q]);
+            float4* f = reinterpret_cast<float4*>(out_f32 + at);
+            f[0] = make_float4(t[0], t[1], t[2], t[3]);
+            f[1] = make_float4(t[4], t[5], t[6], t[7]);
+        }
     }
 }
 
@@ -699,10 +751,12 @@ void launch_gemm_bf16(const bf16_t* a, const bf16_t* b, const bf16_t* bias, bf16
     if (k8 && m <= kGemvMaxM) {
         ProfileScope ps(K_GEMV, s, flops);
         const int grid = static_cast<int>((n + 3) / 4);
-        k_gemv<<<grid, 256, 0, s>>>(a, b, out, m, n, k, e, mode);
+        if (m <= 2) k_gemv<2><<<grid, 256, 0, s>>>(a, b, out, m, n, k, e, mode, ep.silu_out);
+        else k_gemv<kGemvMaxM><<<grid, 256, 0, s>>>(a, b, out, m, n, k, e, mode, ep.silu_out);
         launch_check("gemm (small M)");
         return;
     }
+    require(!ep.silu_out, "gemm: the second output needs at most 8 rows and K % 8 == 0");
     // The MFMA kernel's epilogue works on aligned runs of 8 columns.
     const bool vec = (e.ld_out % 8 == 0) && aligned(out, 16) && (!bias || aligned(bias, 16)) &&
                      (!e.residual || aligned(e.residual, 16)) && (!e.gate || aligned(e.gate, 16)) &&
@@ -765,6 +819,22 @@ void launch_gemm_bf16(const bf16_t* a, const bf16_t* b, const bf16_t* bias, bf16
         default: launch_tn_mt<0>(mt, mode, a, b, out, m, n, k, e, s); break;
     }
     launch_check("gemm (mfma)");
+}
+
+bool adaln_chunks_supported(int64_t batch, int64_t channels, const void* w) {
+    return batch <= kGemvMaxM && channels % 8 == 0 && aligned(w, 16);
+}
+
+void launch_adaln_chunks(const bf16_t* a, const bf16_t* w, const bf16_t* bias, const bf16_t* const* tables_dev,
+                         bf16_t* out, float* out_f32, int64_t layers, int64_t batch, int64_t channels,
+                         hipStream_t s) {
+    ProfileScope ps(K_GEMV, s, 2.0 * batch * 6 * channels * channels);
+    const int grid = static_cast<int>(6 * channels / 8), m = static_cast<int>(batch);
+    if (m <= 2)
+        k_adaln_chunks<2><<<grid, 512, 0, s>>>(a, w, bias, tables_dev, out, out_f32, layers, m, channels);
+    else
+        k_adaln_chunks<kGemvMaxM><<<grid, 512, 0, s>>>(a, w, bias, tables_dev, out, out_f32, layers, m, channels);
+    launch_check("adaln_chunks");
 }
 
 int gemm_splitk_choice(int64_t m, int64_t n, int64_t k) {

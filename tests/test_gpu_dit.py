@@ -172,6 +172,29 @@ def test_fused_plan_equals_opwise_plan(hip, hw, layers):
         b.close()
 
 
+@pytest.mark.parametrize("heads,dim,out,batch,hw,layers", [
+    (2, 64, 4, 1, 8, 2),      # 128 channels, 16 output columns, 16 rows
+    (2, 64, 32, 3, 6, 1),     # 128 output columns, 27 rows (a ragged last workgroup), three adaLN rows
+    (5, 128, 8, 2, 10, 2),    # 640 channels: a vector and a pair per lane
+    (3, 72, 8, 2, 12, 1),     # 216 channels: the head's general launches, a part of a column chunk
+    (15, 128, 8, 1, 8, 1),    # 1920 channels, the widest fused head
+    (16, 128, 8, 1, 8, 1),    # past it
+    (4, 32, 8, 9, 4, 1),      # nine rows: past the small-M projections
+    (2, 64, 8, 2, 4, 1),      # eight tokens: no MFMA path at all
+], ids=str)
+def test_first_and_last_launches_equal_the_ops(hip, heads, dim, out, batch, hw, layers):
+    cfg = dict(SMALL, num_heads=heads, head_dim=dim, out_channels=out, num_layers=layers, caption_channels=64)
+    wl = make_workload(cfg, batch=batch, latent_hw=hw, caption_len=8)
+    a, b = Engine(wl, 0), Engine(wl, 1)
+    try:
+        got = a.forward()
+        assert np.all(np.isfinite(from_bf16(got)))
+        assert np.array_equal(got, b.forward())
+    finally:
+        a.close()
+        b.close()
+
+
 @pytest.mark.parametrize("cfg,batch,hw,cap,layers", [
     (PIXART_SIGMA, 2, 64, 300, 2),   # the CFG pair at 512px: one row per stream, head_dim 72
     (SMALL, 3, 8, 5, None),          # groups of two rows and one, the generic attention
