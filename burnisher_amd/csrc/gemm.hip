@@ -461,6 +461,18 @@ TileShape gemm_tile_shape(int64_t m, int64_t n) {
     return best;
 }
 
+// The tile of a transposed V store: 144 columns (whole heads), and 256 rows, four a lane, unless
+// shorter tiles still fit the CUs in one round -- there every tile is its workgroup's last, whose
+// staged epilogue takes 64, 128 or 256 rows, and more tiles share the chip. One 512px block of one
+// image (QKV 1024 x 3456 x 1152: 96 tiles of 256 rows or 192 of 128; the caption's K and V
+// 120 x 2304 x 1152: 16 or 32 of 64): 206 -> 192 us for the whole forward.
+TileShape vt_tile_shape(int64_t m, int64_t n) {
+    const int64_t grid = device_cus() & ~7, tiles_n = (n + BN - 1) / BN;   // launch_tn's grid
+    for (int mt : {1, 2})
+        if ((m + 64 * mt - 1) / (64 * mt) * tiles_n <= grid) return {mt, kNT};
+    return {kMaxMT, kNT};
+}
+
 // Split-K plans in the tile chooser's units (one operand row loaded per k-tile, ~2.75 ns): a
 // launch of S slices on BM x BN tiles costs ceil(tiles * S / CUs) rounds of K / S / 64 k-tiles of
 // BM + BN rows each, plus its fp32 partials, S * M * N * 4 bytes written and read again by the
@@ -811,8 +823,7 @@ void launch_gemm_bf16(const bf16_t* a, const bf16_t* b, const bf16_t* bias, bf16
         return;
     }
     ProfileScope ps(K_GEMM, s, flops, gemm_subclass());
-    // the transposed V store: 256 x 144 tiles
-    const TileShape mt = ep.vt ? TileShape{kMaxMT, kNT} : gemm_tile_shape(m, n);
+    const TileShape mt = ep.vt ? vt_tile_shape(m, n) : gemm_tile_shape(m, n);
     switch (ep.act) {
         case 1: launch_tn_mt<1>(mt, mode, a, b, out, m, n, k, e, s); break;
         case 2: launch_tn_mt<2>(mt, mode, a, b, out, m, n, k, e, s); break;

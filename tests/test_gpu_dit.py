@@ -172,6 +172,22 @@ def test_fused_plan_equals_opwise_plan(hip, hw, layers):
         b.close()
 
 
+@pytest.mark.parametrize("batch,hw,cap", [
+    (1, 64, 120),    # QKV in one round of 128-row tiles, the caption's K and V of 64-row ones
+    (1, 8, 12),      # sixteen tokens: a tile far past the last row
+    (3, 20, 44),     # 64-row tiles that straddle two images, a ragged last one
+    (3, 56, 300),    # 2352 rows: several rounds, 256-row tiles
+], ids=str)
+def test_transposed_v_store_at_every_tile_height(hip, batch, hw, cap):
+    wl = make_workload(PIXART_SIGMA, batch=batch, latent_hw=hw, caption_len=cap, layers=1)
+    a, b = Engine(wl, 0), Engine(wl, 1)
+    try:
+        assert np.array_equal(a.forward(), b.forward())
+    finally:
+        a.close()
+        b.close()
+
+
 @pytest.mark.parametrize("heads,dim,out,batch,hw,layers", [
     (2, 64, 4, 1, 8, 2),      # 128 channels, 16 output columns, 16 rows
     (2, 64, 32, 3, 6, 1),     # 128 output columns, 27 rows (a ragged last workgroup), three adaLN rows
