@@ -276,6 +276,67 @@ __device__ __forceinline__ void smallk_store(const Epi& e, int mode, const float
     *reinterpret_cast<uint4*>(out + static_cast<int64_t>(m) * e.ld_out + n0) = pack8(v);
 }
 
+// The same for the plain and the row-add store at K = 8 or 16 (a patch embedding of 2 x 2 patches,
+// whose row add is the position table). A wave owns 128 columns, two a lane, their weights in registers, and walks a
+// band of rows: a row's K inputs are the same for all its lanes, so they are scalar loads, four rows in flight, and the
+// lanes read and write whole lines. With eight columns a lane the weights' loads were 256 bytes apart and a
+// wave computed only four rows with them: 10368 x 1152 x 16 took 28.5 us, here 19.
+constexpr int kWaveCols = 128, kWaveRows = 4;
+template <int KC>
+__global__ void __launch_bounds__(256) k_gemm_smallk_wave(const uint32_t* __restrict__ A, const bf16_t* __restrict__ B,
+                                                          bf16_t* out, int M, int N, int band, Epi e, int mode) {
+    constexpr int kK = 8 * KC;
+    const int chunks = (N + kWaveCols - 1) / kWaveCols;
+    const int id = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+    const int m0 = id / chunks * band, m1 = min(M, m0 + band);
+    const int n = id % chunks * kWaveCols + static_cast<int>(threadIdx.x & 63) * 2;
+    if (m0 >= M || n >= N) return;
+    float w[2][kK], bias[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+            float f[8];
+            unpack8(*reinterpret_cast<const uint4*>(B + static_cast<int64_t>(n + r) * kK + 8 * c), f);
+#pragma unroll
+            for (int t = 0; t < 8; ++t) w[r][8 * c + t] = f[t];
+        }
+        bias[r] = e.bias ? bf2f(e.bias[n + r]) : -0.0f;   // v + (-0.0) is v exactly
+    }
+    for (int m = m0; m < m1; m += kWaveRows) {
+        uint32_t a[kWaveRows][kK / 2], add[kWaveRows];
+#pragma unroll
+        for (int i = 0; i < kWaveRows; ++i) {
+            const int row = min(m + i, m1 - 1);
+#pragma unroll
+            for (int t = 0; t < kK / 2; ++t) a[i][t] = A[static_cast<int64_t>(row) * (kK / 2) + t];
+            if (mode == EPI_ROW_ADD)
+                add[i] = *reinterpret_cast<const uint32_t*>(
+                    e.row_add + static_cast<int64_t>(row % static_cast<int>(e.row_add_period)) * N + n);
+        }
+#pragma unroll
+        for (int i = 0; i < kWaveRows; ++i) {
+            float v[2];
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                float acc = 0.f;
+#pragma unroll
+                for (int t = 0; t < kK / 2; ++t) {
+                    acc = __fadd_rn(acc, __fmul_rn(__uint_as_float(a[i][t] << 16), w[r][2 * t]));
+                    acc = __fadd_rn(acc, __fmul_rn(__uint_as_float(a[i][t] & 0xffff0000u), w[r][2 * t + 1]));
+                }
+                v[r] = act_exact(e.act, __fadd_rn(acc, bias[r]));
+                if (mode == EPI_ROW_ADD) {
+                    if (e.round_mid) v[r] = round_bf16(v[r]);
+                    v[r] = __fadd_rn(v[r], r ? __uint_as_float(add[i] & 0xffff0000u) : __uint_as_float(add[i] << 16));
+                }
+            }
+            if (m + i < m1)
+                *reinterpret_cast<uint32_t*>(out + static_cast<int64_t>(m + i) * e.ld_out + n) = f2bf2(v[0], v[1]);
+        }
+    }
+}
+
 template <int KC>
 __global__ void __launch_bounds__(256) k_gemm_smallk(const bf16_t* __restrict__ A,
                                                      const bf16_t* __restrict__ B, bf16_t* out,
@@ -298,60 +359,6 @@ __global__ void __launch_bounds__(256) k_gemm_smallk(const bf16_t* __restrict__ 
 #pragma unroll
                 for (int t = 0; t < 8; ++t) w[r][8 * c + t] = f[t];
             }
-        if (m1 - m0 == kSmallKRows && (mode == EPI_STORE || mode == EPI_ROW_ADD)) {
-            // A whole band of a plain or row-add store (the patch embedding, whose row add is the
-            // position table): every A row and every row-add row is loaded before the first store,
-            // one memory round trip for the band instead of one per row.
-            uint4 ar[kSmallKRows][KC], ra[kSmallKRows];
-#pragma unroll
-            for (int i = 0; i < kSmallKRows; ++i) {
-#pragma unroll
-                for (int c = 0; c < KC; ++c)
-                    ar[i][c] = *reinterpret_cast<const uint4*>(A + static_cast<int64_t>(m0 + i) * kK + 8 * c);
-                if (mode == EPI_ROW_ADD) {
-                    const int pr = static_cast<int>((m0 + i) % static_cast<int>(e.row_add_period));
-                    ra[i] = *reinterpret_cast<const uint4*>(e.row_add + static_cast<int64_t>(pr) * N + n0);
-                }
-            }
-            float bias[8];
-            if (e.bias) {
-                unpack8(*reinterpret_cast<const uint4*>(e.bias + n0), bias);
-            } else {
-#pragma unroll
-                for (int r = 0; r < 8; ++r) bias[r] = -0.0f;   // v + (-0.0) is v exactly
-            }
-#pragma unroll
-            for (int i = 0; i < kSmallKRows; ++i) {
-                float a[kK];
-#pragma unroll
-                for (int c = 0; c < KC; ++c) {
-                    float f[8];
-                    unpack8(ar[i][c], f);
-#pragma unroll
-                    for (int t = 0; t < 8; ++t) a[8 * c + t] = f[t];
-                }
-                float v[8];
-#pragma unroll
-                for (int r = 0; r < 8; ++r) {
-                    float acc = 0.f;
-#pragma unroll
-                    for (int t = 0; t < kK; ++t) acc = __fadd_rn(acc, __fmul_rn(a[t], w[r][t]));
-                    v[r] = act_exact(e.act, __fadd_rn(acc, bias[r]));
-                }
-                if (mode == EPI_ROW_ADD) {
-                    float t[8];
-                    if (e.round_mid) {
-#pragma unroll
-                        for (int r = 0; r < 8; ++r) v[r] = round_bf16(v[r]);
-                    }
-                    unpack8(ra[i], t);
-#pragma unroll
-                    for (int r = 0; r < 8; ++r) v[r] = __fadd_rn(v[r], t[r]);
-                }
-                *reinterpret_cast<uint4*>(out + static_cast<int64_t>(m0 + i) * e.ld_out + n0) = pack8(v);
-            }
-            return;
-        }
         for (int m = m0; m < m1; ++m) {
             float a[kK];
 #pragma unroll
@@ -776,6 +783,18 @@ void launch_gemm_bf16(const bf16_t* a, const bf16_t* b, const bf16_t* bias, bf16
     if (k8 && k % BK != 0 && vec && k <= 256 && m * (n / 8) < (int64_t{1} << 31) &&
         e.row_add_period < (int64_t{1} << 31) && e.gate_rows < (int64_t{1} << 31)) {
         ProfileScope ps(K_GEMM, s, flops);
+        if ((k == 8 || k == 16) && (mode == EPI_STORE || mode == EPI_ROW_ADD)) {
+            // rows per wave: many share a wave's weights, while the chip has two waves a SIMD
+            const int64_t chunks = (n + kWaveCols - 1) / kWaveCols;
+            const int64_t band = std::max<int64_t>(kWaveRows, std::min<int64_t>(32, m * chunks / 2048 / kWaveRows * kWaveRows));
+            const int grid = static_cast<int>(((m + band - 1) / band * chunks + 3) / 4);
+            const uint32_t* aw = reinterpret_cast<const uint32_t*>(a);
+            const int mi = static_cast<int>(m), ni = static_cast<int>(n), bi = static_cast<int>(band);
+            if (k == 8) k_gemm_smallk_wave<1><<<grid, 256, 0, s>>>(aw, b, out, mi, ni, bi, e, mode);
+            else k_gemm_smallk_wave<2><<<grid, 256, 0, s>>>(aw, b, out, mi, ni, bi, e, mode);
+            launch_check("gemm (small K)");
+            return;
+        }
         const int64_t threads = (m + kSmallKRows - 1) / kSmallKRows * (n / 8);
         const int blocks = static_cast<int>((threads + 255) / 256);
         const int mi = static_cast<int>(m), ni = static_cast<int>(n), ki = static_cast<int>(k);

@@ -184,6 +184,20 @@ def test_gemm_fused_epilogues(hip):
     assert s1["mismatch_frac"] < 0.01
 
 
+@pytest.mark.parametrize("M,d,K,act", [(9, 8, 16, 0), (2049, 136, 16, 1), (33, 264, 8, 2), (40000, 128, 8, 0)],
+                         ids=lambda v: str(v))
+def test_gemm_small_k_wave_bands(hip, M, d, K, act):
+    # K = 8 and 16 with a plain store: columns in part of a wave's 128, rows in part of its band
+    # (bands of 4, 8 and 16 rows), every activation.
+    rng = np.random.default_rng(41)   # its own: the other tests' inputs stay what they were
+    a, w, bias = randn_bf16(rng, (M, K)), randn_bf16(rng, (d, K), 0.3), randn_bf16(rng, (d,), 0.3)
+    want = np.zeros((M, d), np.uint16)
+    st("stock_gemm", addr(a), addr(w), addr(bias), addr(want), M, d, K, 1, act, BF16, 0)
+    da, dw, db, out = dev(a), dev(w), dev(bias), empty((M, d))
+    call("bh_gemm", P(da), P(dw), P(db), P(out), M, d, K, 1, act, BF16, None)
+    assert_within(from_bf16(host(out, want)), from_bf16(want), "gemm", f"small K {M}x{d}x{K}")
+
+
 @pytest.mark.parametrize("B,N_tok", [(2, 1024), (7, 143)], ids=["whole_bands", "ragged_band"])
 def test_gemm_small_k_fused_epilogues(hip, B, N_tok):
     # K = 16, the patch embedding's in_channels * patch^2: the register-weight kernel. Whole bands
