@@ -389,10 +389,15 @@ int gemm_splitk_choice(int64_t m, int64_t n, int64_t k);
 // launch is chosen per launch and changes no sum.
 int gemm_splits(int64_t m, int64_t n, int64_t k, const GemmEpilogue& ep);
 // out = bf16(residual + bf16(A . B^T)) through `splits` fp32 partials (partial holds
-// splits * m * n floats) summed in slice order; out may alias residual.
-void launch_gemm_splitk_residual(const bf16_t* a, const bf16_t* b, float* partial, int splits,
-                                 const bf16_t* residual, bf16_t* out, int64_t m, int64_t n, int64_t k,
-                                 hipStream_t s);
+// splits * m * n floats) summed in slice order, then normed = the RMSNorm of out (weight w); out may
+// alias residual.
+void launch_gemm_splitk_residual_rms(const bf16_t* a, const bf16_t* b, float* partial, int splits,
+                                     const bf16_t* residual, bf16_t* out, const bf16_t* w, bf16_t* normed,
+                                     float eps, int64_t m, int64_t n, int64_t k, hipStream_t s);
+// Its reduction and norm in one launch (elementwise.hip).
+bool splitk_residual_rms_supported(int64_t m, int64_t n, const void* w, const void* normed);
+void launch_splitk_residual_rms(const float* partial, int splits, const bf16_t* residual, bf16_t* out,
+                                const bf16_t* w, bf16_t* normed, int64_t m, int64_t n, float eps, hipStream_t s);
 // Any dtype / layout, reference summation order: one thread per output (tests, fp32, [K,N] B).
 void launch_gemm_generic(const void* a, const void* b, const void* bias, void* out, int64_t m,
                          int64_t n, int64_t k, bool b_transposed, int act, bool f32,

@@ -196,6 +196,80 @@ __global__ void __launch_bounds__(256) k_norm_rows(const bf16_t* __restrict__ x,
     }
 }
 
+// The split-K reduction with a residual (x = residual + bf16(sum of the S slices, in order)) and the
+// RMSNorm of x that follows it, a row per workgroup: as two launches the row went to memory and back
+// between them, and at the row counts of a text encoder each launch is mostly its own start (T5 XXL:
+// 4.8 + 4.9 us at 120 rows of 4096 and 8 slices, 6.0 + 7.1 at 600 rows and 2). Every slice is requested
+// before the first addition. The arithmetic is that of the two kernels; only the fp64 sum of squares
+// adds its terms in another order. G groups of four columns a thread.
+template <int S, int G>
+__global__ void __launch_bounds__(256) k_splitk_residual_rms(const float* __restrict__ partial, const bf16_t* residual,
+                                                             bf16_t* out, const bf16_t* __restrict__ w,
+                                                             bf16_t* __restrict__ normed, int64_t mn, int cols,
+                                                             float eps) {
+    using f4 = float __attribute__((ext_vector_type(4)));
+    __shared__ double sums[4];
+    const int64_t row0 = static_cast<int64_t>(blockIdx.x) * cols;
+    f4 p[G][S];
+    uint2 res[G], wv[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        // a thread past the row's end reads its last group again and stores nothing
+        const int c = min((g * 256 + static_cast<int>(threadIdx.x)) * 4, cols - 4);
+#pragma unroll
+        for (int sp = 0; sp < S; ++sp) p[g][sp] = *reinterpret_cast<const f4*>(partial + sp * mn + row0 + c);
+        res[g] = *reinterpret_cast<const uint2*>(residual + row0 + c);
+        wv[g] = *reinterpret_cast<const uint2*>(w + c);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    uint2 x[G];
+    double q = 0.0;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        f4 acc = p[g][0];
+#pragma unroll
+        for (int sp = 1; sp < S; ++sp)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc[t] = __fadd_rn(acc[t], p[g][sp][t]);
+        const uint32_t r[2] = {res[g].x, res[g].y};
+        uint32_t o[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+            o[t] = f2bf2(__fadd_rn(__uint_as_float(r[t] << 16), round_bf16(acc[2 * t])),
+                         __fadd_rn(__uint_as_float(r[t] & 0xffff0000u), round_bf16(acc[2 * t + 1])));
+        x[g] = make_uint2(o[0], o[1]);
+        const int c = (g * 256 + static_cast<int>(threadIdx.x)) * 4;
+        if (c < cols) {
+            *reinterpret_cast<uint2*>(out + row0 + c) = x[g];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const double lo = static_cast<double>(__uint_as_float(o[t] << 16));
+                const double hi = static_cast<double>(__uint_as_float(o[t] & 0xffff0000u));
+                q += lo * lo;
+                q += hi * hi;
+            }
+        }
+    }
+    q = wave_sum(q);
+    if (threadIdx.x % kWave == 0) sums[wave_index()] = q;
+    __syncthreads();
+    const double var = (sums[0] + sums[1] + sums[2] + sums[3]) / static_cast<double>(cols);
+    const float inv = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(static_cast<float>(var), eps)));
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const int c = (g * 256 + static_cast<int>(threadIdx.x)) * 4;
+        if (c >= cols) continue;
+        const uint32_t v[2] = {x[g].x, x[g].y}, wr[2] = {wv[g].x, wv[g].y};
+        uint32_t o[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+            o[t] = f2bf2(__fmul_rn(__fmul_rn(__uint_as_float(v[t] << 16), inv), __uint_as_float(wr[t] << 16)),
+                         __fmul_rn(__fmul_rn(__uint_as_float(v[t] & 0xffff0000u), inv),
+                                   __uint_as_float(wr[t] & 0xffff0000u)));
+        *reinterpret_cast<uint2*>(normed + row0 + c) = make_uint2(o[0], o[1]);
+    }
+}
+
 // ---- LayerNorm fused with the adaLN chunk and modulation (the hot row kernel) ---------------
 
 // Row statistics exactly as the oracle forms them: fp64 mean, fp64 sum of squared deviations,
@@ -1279,6 +1353,37 @@ void launch_dit_head(const bf16_t* x, const bf16_t* emb, const bf16_t* table, co
     }
 #undef BH_HEAD
     launch_check("dit_head");
+}
+
+template <int S>
+static void launch_splitk_rms(int g, const float* partial, const bf16_t* residual, bf16_t* out, const bf16_t* w,
+                              bf16_t* normed, int64_t m, int64_t n, float eps, hipStream_t s) {
+    const int grid = static_cast<int>(m), cols = static_cast<int>(n);
+    if (g <= 1) k_splitk_residual_rms<S, 1><<<grid, 256, 0, s>>>(partial, residual, out, w, normed, m * n, cols, eps);
+    else if (g <= 2) k_splitk_residual_rms<S, 2><<<grid, 256, 0, s>>>(partial, residual, out, w, normed, m * n, cols, eps);
+    else k_splitk_residual_rms<S, 4><<<grid, 256, 0, s>>>(partial, residual, out, w, normed, m * n, cols, eps);
+}
+
+// A row of at most 4096 columns stays in registers (four groups of four a thread).
+bool splitk_residual_rms_supported(int64_t m, int64_t n, const void* w, const void* normed) {
+    return n % 4 == 0 && n >= 4 && n <= 4096 && m < (int64_t{1} << 31) && (reinterpret_cast<uintptr_t>(w) & 7) == 0 &&
+           (reinterpret_cast<uintptr_t>(normed) & 7) == 0;
+}
+
+void launch_splitk_residual_rms(const float* partial, int splits, const bf16_t* residual, bf16_t* out,
+                                const bf16_t* w, bf16_t* normed, int64_t m, int64_t n, float eps, hipStream_t s) {
+    ProfileScope ps(K_NORM, s, static_cast<double>(m) * n * (4.0 * splits + 6.0));
+    const int g = static_cast<int>((n + 1023) / 1024);
+    switch (splits) {
+        case 2: launch_splitk_rms<2>(g, partial, residual, out, w, normed, m, n, eps, s); break;
+        case 3: launch_splitk_rms<3>(g, partial, residual, out, w, normed, m, n, eps, s); break;
+        case 4: launch_splitk_rms<4>(g, partial, residual, out, w, normed, m, n, eps, s); break;
+        case 5: launch_splitk_rms<5>(g, partial, residual, out, w, normed, m, n, eps, s); break;
+        case 6: launch_splitk_rms<6>(g, partial, residual, out, w, normed, m, n, eps, s); break;
+        case 7: launch_splitk_rms<7>(g, partial, residual, out, w, normed, m, n, eps, s); break;
+        default: launch_splitk_rms<8>(g, partial, residual, out, w, normed, m, n, eps, s); break;
+    }
+    launch_check("split-K residual and norm");
 }
 
 void launch_scale(const void* in, void* out, int64_t n, float scale, bool f32, hipStream_t s) {

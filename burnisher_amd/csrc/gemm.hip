@@ -904,9 +904,9 @@ int gemm_splits(int64_t m, int64_t n, int64_t k, const GemmEpilogue& ep) {
     return best;
 }
 
-void launch_gemm_splitk_residual(const bf16_t* a, const bf16_t* b, float* partial, int splits,
-                                 const bf16_t* residual, bf16_t* out, int64_t m, int64_t n, int64_t k,
-                                 hipStream_t s) {
+void launch_gemm_splitk_residual_rms(const bf16_t* a, const bf16_t* b, float* partial, int splits,
+                                     const bf16_t* residual, bf16_t* out, const bf16_t* w, bf16_t* normed,
+                                     float eps, int64_t m, int64_t n, int64_t k, hipStream_t s) {
     if (m == 0 || n == 0) return;
     require(splits >= 2 && splits <= 8 && k % (BK * splits) == 0 && n % 8 == 0 && m > kGemvMaxM,
             "gemm split-K: K must split into whole 64-wide k-tiles, N % 8 == 0");
@@ -916,6 +916,10 @@ void launch_gemm_splitk_residual(const bf16_t* a, const bf16_t* b, float* partia
         ProfileScope ps(K_GEMM, s, 2.0 * static_cast<double>(m) * n * k);
         launch_splitk_partials(a, b, partial, m, n, k, splits, s);
         launch_check("gemm (split-K partials)");
+    }
+    if (splitk_residual_rms_supported(m, n, w, normed)) {
+        launch_splitk_residual_rms(partial, splits, residual, out, w, normed, m, n, eps, s);
+        return;
     }
     ProfileScope ps(K_ELEMENTWISE, s, static_cast<double>(m) * n * (4.0 * splits + 4.0));
     const int64_t mn = m * n;
@@ -931,6 +935,7 @@ void launch_gemm_splitk_residual(const bf16_t* a, const bf16_t* b, float* partia
         default: k_splitk_residual<8><<<g, 256, 0, s>>>(partial, residual, out, mn); break;
     }
     launch_check("gemm (split-K reduce)");
+    launch_norm(out, w, nullptr, normed, m, n, eps, true, false, s);
 }
 
 }  // namespace bh

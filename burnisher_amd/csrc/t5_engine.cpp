@@ -130,20 +130,27 @@ void encode(bh_t5* e, const float* ids_in, bf16_t* out, hipStream_t s) {
     residual.round_mid = true;
     residual.residual = e->x;
     const bh::AttnShape sh{e->B, e->H, e->S, e->S, c.d_kv, 3 * inner, 3 * inner, inner, 1.0f};
+    // every norm but the first follows the projection that writes its input
+    const bool any = c.num_layers > 0;
+    bh::launch_norm(e->x, e->at(any ? blk(0, "layer.0.layer_norm.weight") : "encoder.final_layer_norm.weight"),
+                    nullptr, any ? e->normed : out, M, d, eps, true, false, s);
+    // x += A . W^T, then the norm that reads x next, into `normed`
+    auto project = [&](const bf16_t* a, const std::string& w, int64_t k, int splits, const std::string& norm_w,
+                       bf16_t* normed) {
+        if (splits > 1) {
+            bh::launch_gemm_splitk_residual_rms(a, e->at(w), e->partial, splits, e->x, e->x, e->at(norm_w), normed,
+                                                eps, M, d, k, s);
+        } else {
+            bh::launch_gemm_bf16(a, e->at(w), nullptr, e->x, M, d, k, residual, s);
+            bh::launch_norm(e->x, e->at(norm_w), nullptr, normed, M, d, eps, true, false, s);
+        }
+    };
     for (int l = 0; l < c.num_layers; ++l) {
-        bh::launch_norm(e->x, e->at(blk(l, "layer.0.layer_norm.weight")), nullptr, e->normed, M, d, eps,
-                        true, false, s);
         bh::launch_gemm_bf16(e->normed, e->qkv_w[l], nullptr, e->qkv, M, 3 * inner, d, plain, s);
         bh::launch_attention_bf16(e->qkv, e->qkv + inner, e->qkv + 2 * inner, e->ctx, sh, e->mask, false, s,
                                   e->bias);
-        if (e->split_o > 1)
-            bh::launch_gemm_splitk_residual(e->ctx, e->at(blk(l, "layer.0.SelfAttention.o.weight")), e->partial,
-                                            e->split_o, e->x, e->x, M, d, inner, s);
-        else
-            bh::launch_gemm_bf16(e->ctx, e->at(blk(l, "layer.0.SelfAttention.o.weight")), nullptr, e->x, M, d,
-                                 inner, residual, s);
-        bh::launch_norm(e->x, e->at(blk(l, "layer.1.layer_norm.weight")), nullptr, e->normed, M, d, eps,
-                        true, false, s);
+        project(e->ctx, blk(l, "layer.0.SelfAttention.o.weight"), inner, e->split_o,
+                blk(l, "layer.1.layer_norm.weight"), e->normed);
         if (c.gated) {
             bh::launch_gemm_bf16(e->normed, e->wi_w[l], nullptr, e->h01, M, 2 * F, d, plain, s);
             bh::launch_gelu_gated_rows(e->h01, e->hact, M, F, s);
@@ -152,14 +159,11 @@ void encode(bh_t5* e, const float* ids_in, bf16_t* out, hipStream_t s) {
                                  e->h01, M, F, d, plain, s);
             bh::launch_activation(e->h01, e->hact, M * F, BH_EPI_GELU, nullptr, false, s);
         }
-        if (e->split_wo > 1)
-            bh::launch_gemm_splitk_residual(e->hact, e->at(blk(l, "layer.1.DenseReluDense.wo.weight")),
-                                            e->partial, e->split_wo, e->x, e->x, M, d, F, s);
-        else
-            bh::launch_gemm_bf16(e->hact, e->at(blk(l, "layer.1.DenseReluDense.wo.weight")), nullptr, e->x, M, d,
-                                 F, residual, s);
+        const bool last = l + 1 == c.num_layers;
+        project(e->hact, blk(l, "layer.1.DenseReluDense.wo.weight"), F, e->split_wo,
+                last ? std::string("encoder.final_layer_norm.weight") : blk(l + 1, "layer.0.layer_norm.weight"),
+                last ? out : e->normed);
     }
-    bh::launch_norm(e->x, e->at("encoder.final_layer_norm.weight"), nullptr, out, M, d, eps, true, false, s);
 }
 
 }  // namespace

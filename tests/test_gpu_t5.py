@@ -123,7 +123,12 @@ def check(got, want, where):
     (dict(SMALL, gated=0, num_layers=1), 2, 9, [9, 5]),
     (dict(SMALL, d_model=256, d_ff=640, d_kv=64, num_heads=4, vocab_size=1000, num_layers=3), 2, 77, [1, 40]),
     (dict(T5_XXL, num_layers=1), 2, 48, [1, 30]),
-], ids=["small", "small_44", "plain_gelu", "mid", "xxl_widths_1layer"])
+    (dict(SMALL, num_layers=0), 2, 9, [3, 9]),     # the final norm alone
+    # split projections of both kinds (K = 3072 and 4608) whose rows take the reduction's norm with one
+    # group of four columns a thread (part of them idle) and, past 4096 columns, the separate norm
+    (dict(SMALL, d_model=200, d_ff=4608, d_kv=64, num_heads=48, num_layers=1), 1, 33, [20]),
+    (dict(SMALL, d_model=4608, d_ff=3072, d_kv=64, num_heads=48, num_layers=1), 1, 12, [12]),
+], ids=["small", "small_44", "plain_gelu", "mid", "xxl_widths_1layer", "no_layers", "split_200", "split_4608"])
 def test_encoder_matches_oracle(hip, cfg, batch, seq, lengths):
     wl = make_t5_workload(cfg, batch=batch, seq=seq, lengths=lengths, seed=9)
     check(device_encode(wl), stock_encode(wl), f"{cfg['d_model']}x{cfg['num_layers']} B{batch} S{seq}")
