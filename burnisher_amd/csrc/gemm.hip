@@ -444,6 +444,27 @@ void launch_tn(const bf16_t* a, const bf16_t* b, bf16_t* out, int64_t m, int64_t
 struct TileShape {
     int mt, nt;
 };
+// The narrow tiles (48, 80 or 96 columns of 64 or 128 rows), where they divide the width and all `splits`
+// slices' tiles have a CU of their own: few rows leave the 128-wide ones on a part of the chip, and what
+// bounds such a launch is the weights each CU streams. 120 x 20480 x 4096: 160 tiles of 128 columns
+// 51 us, 256 of 80 45; 120 x 12288 x 4096 in two slices: 192 of 128 34, 256 of 96 32.
+template <typename Cost>
+void narrow_tile_shape(int64_t m, int64_t n, int splits, Cost cost, TileShape& best, int64_t& best_cost) {
+    const int64_t cus = device_cus() & ~7;   // launch_tn's grid
+    for (int nt : {6, 5, 3}) {
+        if (n % (16 * nt) != 0) continue;
+        for (int mt : {2, 1}) {
+            const int64_t bm = 64 * mt, bn = 16 * nt, tiles = ((m + bm - 1) / bm) * (n / bn);
+            if (tiles * splits > cus) continue;
+            const int64_t c = cost(bm, bn);
+            if (c < best_cost) {
+                best = {mt, nt};
+                best_cost = c;
+            }
+        }
+    }
+}
+
 TileShape gemm_tile_shape(int64_t m, int64_t n) {
     const int64_t cus = device_cus();
     TileShape best{kMaxMT, kNT};
@@ -465,6 +486,7 @@ TileShape gemm_tile_shape(int64_t m, int64_t n) {
             }
         }
     }
+    narrow_tile_shape(m, n, 1, [](int64_t bm, int64_t bn) { return bm + bn; }, best, best_cost);
     return best;
 }
 
@@ -498,8 +520,9 @@ int64_t splitk_cost(int64_t m, int64_t n, int64_t k, TileShape sh, int splits) {
 // The tile shape of an S-slice launch: the cheapest by splitk_cost (ties keep the taller and the
 // 144-wide tile; 128-wide for widths that are multiples of 128, with the XCD banding's tile count
 // kept whole over several rounds). The shape does not change any sum; the slice count does, and
-// is decided on the full batch.
-TileShape splitk_tile_shape(int64_t m, int64_t n, int64_t k, int splits) {
+// is decided on the full batch and without the narrow tiles (it picks the sums' order, which does not
+// move when a tile is added here).
+TileShape splitk_tile_shape(int64_t m, int64_t n, int64_t k, int splits, bool narrow = true) {
     const int64_t cus = device_cus();
     TileShape best{kMaxMT, kNT};
     int64_t best_cost = -1;
@@ -515,6 +538,10 @@ TileShape splitk_tile_shape(int64_t m, int64_t n, int64_t k, int splits) {
             }
         }
     }
+    if (narrow)
+        narrow_tile_shape(m, n, splits, [&](int64_t bm, int64_t bn) {
+            return splitk_cost(m, n, k, TileShape{static_cast<int>(bm / 64), static_cast<int>(bn / 16)}, splits);
+        }, best, best_cost);
     return best;
 }
 
@@ -542,6 +569,15 @@ void launch_tn_splitk(const bf16_t* a, const bf16_t* b, float* partial, int64_t 
 void launch_splitk_partials(const bf16_t* a, const bf16_t* b, float* partial, int64_t m, int64_t n,
                             int64_t k, int splits, hipStream_t s) {
     const TileShape sh = splitk_tile_shape(m, n, k, splits);
+    switch (sh.mt * 16 + sh.nt) {
+        case 16 + 3: launch_tn_splitk<1, 3>(a, b, partial, m, n, k, splits, s); return;
+        case 16 + 5: launch_tn_splitk<1, 5>(a, b, partial, m, n, k, splits, s); return;
+        case 16 + 6: launch_tn_splitk<1, 6>(a, b, partial, m, n, k, splits, s); return;
+        case 32 + 3: launch_tn_splitk<2, 3>(a, b, partial, m, n, k, splits, s); return;
+        case 32 + 5: launch_tn_splitk<2, 5>(a, b, partial, m, n, k, splits, s); return;
+        case 32 + 6: launch_tn_splitk<2, 6>(a, b, partial, m, n, k, splits, s); return;
+        default: break;
+    }
     if (sh.nt == 8) {
         switch (sh.mt) {
             case 1: launch_tn_splitk<1, 8>(a, b, partial, m, n, k, splits, s); break;
@@ -705,6 +741,15 @@ void launch_tn_mode(int mode, const bf16_t* a, const bf16_t* b, bf16_t* out, int
 template <int ACT>
 void launch_tn_mt(TileShape sh, int mode, const bf16_t* a, const bf16_t* b, bf16_t* out, int64_t m, int64_t n,
                   int64_t k, const Epi& e, hipStream_t s) {
+    switch (sh.mt * 16 + sh.nt) {
+        case 16 + 3: launch_tn_mode<ACT, 1, 3>(mode, a, b, out, m, n, k, e, s); return;
+        case 16 + 5: launch_tn_mode<ACT, 1, 5>(mode, a, b, out, m, n, k, e, s); return;
+        case 16 + 6: launch_tn_mode<ACT, 1, 6>(mode, a, b, out, m, n, k, e, s); return;
+        case 32 + 3: launch_tn_mode<ACT, 2, 3>(mode, a, b, out, m, n, k, e, s); return;
+        case 32 + 5: launch_tn_mode<ACT, 2, 5>(mode, a, b, out, m, n, k, e, s); return;
+        case 32 + 6: launch_tn_mode<ACT, 2, 6>(mode, a, b, out, m, n, k, e, s); return;
+        default: break;
+    }
     if (sh.nt == 8) {
         switch (sh.mt) {
             case 1: launch_tn_mode<ACT, 1, 8>(mode, a, b, out, m, n, k, e, s); break;
@@ -895,7 +940,7 @@ int gemm_splits(int64_t m, int64_t n, int64_t k, const GemmEpilogue& ep) {
     int64_t best_cost = -1;
     for (int sp = 1; sp <= 8; ++sp) {
         if (sp > 1 && (k % (BK * sp) != 0 || k / sp < 4 * BK)) continue;
-        const int64_t c = splitk_cost(m, n, k, splitk_tile_shape(m, n, k, sp), sp);
+        const int64_t c = splitk_cost(m, n, k, splitk_tile_shape(m, n, k, sp, false), sp);
         if (best_cost < 0 || c < best_cost) {
             best = sp;
             best_cost = c;

@@ -232,6 +232,33 @@ def test_gemm_small_k_fused_epilogues(hip, B, N_tok):
     assert_within(from_bf16(host(dx, want_gated)), from_bf16(want_gated), "gemm_fused", f"gated M={M}")
 
 
+@pytest.mark.parametrize("M,N,K", [(120, 12288, 64), (65, 20480, 128), (128, 24576, 64), (9, 48, 64), (64, 80, 320),
+                                   (100, 1152, 3072), (65, 3840, 448)],
+                         ids=["48_cols", "80_cols", "96_cols", "one_tile", "80_one_tile", "split_k", "odd_k_tiles"])
+def test_gemm_narrow_tiles(hip, M, N, K):
+    # Few rows run on tiles of 48, 80 or 96 columns, one a workgroup: ragged heights, fewer k-tiles than
+    # LDS stages, K slices, and every epilogue of the staged store.
+    import burnisher_amd as bh
+    import ctypes
+    rng = np.random.default_rng(43)   # its own: the other tests' inputs stay what they were
+    a, w, bias = randn_bf16(rng, (M, K)), randn_bf16(rng, (N, K), 0.1), randn_bf16(rng, (N,))
+    x, gate = randn_bf16(rng, (M, N)), randn_bf16(rng, (1, N), 0.5)
+    proj, act = np.zeros((M, N), np.uint16), np.zeros((M, N), np.uint16)
+    st("stock_gemm", addr(a), addr(w), addr(bias), addr(proj), M, N, K, 1, 0, BF16, 0)
+    st("stock_gemm", addr(a), addr(w), addr(bias), addr(act), M, N, K, 1, 1, BF16, 0)
+    zero = np.zeros((1, N), np.uint16)
+    want = x.copy()
+    st("stock_modulate", addr(proj), addr(zero), addr(zero), addr(want), 1, M, N, addr(want), addr(gate), BF16)
+    da, dw, db, dx, dg = dev(a), dev(w), dev(bias), dev(x), dev(gate)
+    for kind, ref in ((0, proj), (1, act)):
+        out = empty((M, N))
+        call("bh_gemm", P(da), P(dw), P(db), P(out), M, N, K, 1, kind, BF16, None)
+        assert_within(from_bf16(host(out, ref)), from_bf16(ref), "gemm", f"{M}x{N}x{K} act {kind}")
+    f = bh.GemmFused(epilogue=0, round_mid=1, residual=P(dx), gate=P(dg), gate_rows=M, ld_out=N)
+    call("bh_gemm_fused_run", P(da), P(dw), P(db), P(dx), M, N, K, ctypes.byref(f), None)
+    assert_within(from_bf16(host(dx, want)), from_bf16(want), "gemm_fused", f"gated {M}x{N}x{K}")
+
+
 def test_gemm_split_k_epilogues(hip):
     # A long-K GEMM with few output tiles (the 512px ff2 shape at 300 tokens per row: 24 tiles of
     # 256 x 144, 72 k-tiles) runs as K slices whose fp32 partials are summed in slice order by the
