@@ -23,6 +23,8 @@ pytestmark = pytest.mark.gpu
 @pytest.fixture(scope="module")
 def driver():
     path = oracle.registry_main()
+    if not oracle.REGISTRY_MAIN.parent.exists():
+        pytest.skip("oracle/_ref was not built: the reference's sources were not there at build time")
     assert path is not None, "oracle/_ref/registry_main was not built (build() builds it beside the reference)"
     return path
 
