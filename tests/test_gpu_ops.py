@@ -530,6 +530,19 @@ def test_modulate_matches_oracle(hip, C):
     assert np.array_equal(host(dres, want), want)
 
 
+def test_silu_every_bf16_value(hip):
+    """The 16-byte SiLU against the element-wise kernel (the exact exponential and division, taken where
+    the count is no multiple of eight), on every bf16 bit pattern: the same bits, NaN where that has NaN."""
+    x = np.arange(1 << 16, dtype=np.uint32).astype(np.uint16)
+    got, want = empty((x.size,)), empty((x.size + 1,))
+    call("bh_activation", P(dev(x)), P(got), x.size, 2, None, BF16, None)
+    call("bh_activation", P(dev(np.append(x, x[:1]))), P(want), x.size + 1, 2, None, BF16, None)
+    got, want = host(got, x), host(want, np.append(x, x[:1]))[:-1]
+    nan = np.isnan(from_bf16(want))
+    assert np.array_equal(np.isnan(from_bf16(got)), nan)
+    assert np.array_equal(got[~nan], want[~nan])
+
+
 def test_add_chunk_activation_patch(hip):
     B, T, C = 2, 40, 1152
     a, b, row = randn_bf16(RNG, (B, T * C)), randn_bf16(RNG, (B, T * C)), randn_bf16(RNG, (T * C,))
