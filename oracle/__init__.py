@@ -4,7 +4,7 @@
            graph and DPM-Solver++ sampler (oracle/stock.cpp). Built by `make -C oracle`.
   ref()    oracle/_ref/libref_stock.so, the reference's OWN stock path compiled from
            /root/reference (oracle/ref_shim.cpp + `make -C oracle ref`), or None where it was
-           not built (it needs /root/reference at build time).
+           not built (it needs the reference's sources in /root/reference at build time).
 
 Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may import this package,
 and only as the checker -- never as the thing measured or shipped.
@@ -105,11 +105,16 @@ def _load(path: Path, sigs: dict) -> ctypes.CDLL:
     return lib
 
 
+def reference_sources() -> bool:
+    """Whether the reference's sources are there (its folder may exist and be empty)."""
+    return (REFERENCE_ROOT / "src" / "core" / "tensor.cpp").exists()
+
+
 def build(reference: bool = True) -> None:
-    """make -C oracle (and the `ref` and `registry` targets when /root/reference exists; the
-    registry driver also needs the built burnisher_amd/lib/libburnisher_hip.so)."""
+    """make -C oracle (and the `ref` and `registry` targets when the reference's sources are there;
+    the registry driver also needs the built burnisher_amd/lib/libburnisher_hip.so)."""
     subprocess.run(["make", "-s", "-C", str(HERE)], check=True)
-    if reference and REFERENCE_ROOT.exists():
+    if reference and reference_sources():
         subprocess.run(["make", "-s", "-C", str(HERE), "ref"], check=True)
         if (HERE.parent / "burnisher_amd" / "lib" / "libburnisher_hip.so").exists():
             subprocess.run(["make", "-s", "-C", str(HERE), "registry"], check=True)

@@ -88,3 +88,15 @@ def test_product_never_reaches_the_oracle():
         for pattern in (r"^\s*(import|from)\s+oracle\b", r"libstock|libref_stock",
                         r"\b(stock|ref)_[a-z_]+\s*\(", r"oracle/_(build|ref)"):
             assert not re.search(pattern, text, flags=re.M), f"{p} reaches the oracle ({pattern})"
+
+
+def test_oracle_build_without_the_reference_sources(monkeypatch, tmp_path):
+    # the folder may exist and hold nothing: then only the restatement is built
+    import subprocess
+    import oracle
+    ran = []
+    monkeypatch.setattr(subprocess, "run", lambda cmd, check: ran.append(cmd[4:]))
+    for root in (tmp_path, tmp_path / "absent"):
+        monkeypatch.setattr(oracle, "REFERENCE_ROOT", root)
+        oracle.build()
+    assert ran == [[], []]
