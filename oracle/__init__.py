@@ -19,6 +19,8 @@ HERE = Path(__file__).resolve().parent
 STOCK_PATH = HERE / "_build" / "libstock.so"
 REF_PATH = HERE / "_ref" / "libref_stock.so"
 REFERENCE_ROOT = Path("/root/reference")
+# "present" or "absent": whether the reference's sources were there at the last build()
+REFERENCE_RECORD = HERE / "_build" / "reference_sources"
 
 _V, _I, _I64, _F, _D = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float, ctypes.c_double
 
@@ -114,6 +116,7 @@ def build(reference: bool = True) -> None:
     """make -C oracle (and the `ref` and `registry` targets when the reference's sources are there;
     the registry driver also needs the built burnisher_amd/lib/libburnisher_hip.so)."""
     subprocess.run(["make", "-s", "-C", str(HERE)], check=True)
+    REFERENCE_RECORD.write_text("present" if reference_sources() else "absent")
     if reference and reference_sources():
         subprocess.run(["make", "-s", "-C", str(HERE), "ref"], check=True)
         if (HERE.parent / "burnisher_amd" / "lib" / "libburnisher_hip.so").exists():
@@ -127,6 +130,12 @@ def registry_main() -> Path | None:
     """oracle/_ref/registry_main (the reference runtime with the hip-gfx950 registrations and the
     HIP device layer), or None where it was not built."""
     return REGISTRY_MAIN if REGISTRY_MAIN.exists() else None
+
+
+def built_without_reference() -> bool:
+    """Whether build() ran where the reference's sources were not (only then may what it builds from
+    them be missing)."""
+    return REFERENCE_RECORD.exists() and REFERENCE_RECORD.read_text() == "absent"
 
 
 def stock() -> ctypes.CDLL:

@@ -150,3 +150,15 @@ COEFF_FIELDS = ("order", "sigma_s0", "sigma_t", "sigma_vp_s0", "sigma_vp_t", "al
 
 def coeff_tuple(c) -> tuple:
     return tuple(getattr(c, f) for f in COEFF_FIELDS)
+
+
+def built_driver():
+    """The registry driver, built from the reference's sources. A skip only where build() recorded that
+    they were not there; a driver missing for any other reason is a failure."""
+    import oracle
+    import pytest
+    path = oracle.registry_main()
+    if path is None and oracle.built_without_reference():
+        pytest.skip("oracle/_ref was not built: the reference's sources were not there at build time")
+    assert path is not None, "oracle/_ref/registry_main was not built (build() builds it beside the reference)"
+    return path

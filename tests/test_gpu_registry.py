@@ -15,18 +15,14 @@ import pytest
 
 import oracle
 from burnisher_amd.workload import PIXART_SIGMA, config_struct, make_workload
-from helpers import F32
+from helpers import F32, built_driver
 
 pytestmark = pytest.mark.gpu
 
 
 @pytest.fixture(scope="module")
 def driver():
-    path = oracle.registry_main()
-    if not oracle.REGISTRY_MAIN.parent.exists():
-        pytest.skip("oracle/_ref was not built: the reference's sources were not there at build time")
-    assert path is not None, "oracle/_ref/registry_main was not built (build() builds it beside the reference)"
-    return path
+    return built_driver()
 
 
 def engine_output(wl, mode):

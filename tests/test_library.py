@@ -94,9 +94,29 @@ def test_oracle_build_without_the_reference_sources(monkeypatch, tmp_path):
     # the folder may exist and hold nothing: then only the restatement is built
     import subprocess
     import oracle
+    (tmp_path / "empty").mkdir()
     ran = []
     monkeypatch.setattr(subprocess, "run", lambda cmd, check: ran.append(cmd[4:]))
-    for root in (tmp_path, tmp_path / "absent"):
+    monkeypatch.setattr(oracle, "REFERENCE_RECORD", tmp_path / "record")
+    for root in (tmp_path / "empty", tmp_path / "absent"):
         monkeypatch.setattr(oracle, "REFERENCE_ROOT", root)
         oracle.build()
     assert ran == [[], []]
+
+
+@pytest.mark.parametrize("record,driver,outcome", [("absent", False, "skip"), ("present", False, "fail"),
+                                                   (None, False, "fail"), ("absent", True, "path"),
+                                                   ("present", True, "path")], ids=str)
+def test_a_missing_registry_driver_is_skipped_only_without_sources(monkeypatch, tmp_path, record, driver, outcome):
+    import oracle
+    from helpers import built_driver
+    monkeypatch.setattr(oracle, "REFERENCE_RECORD", tmp_path / "record")
+    monkeypatch.setattr(oracle, "REGISTRY_MAIN", tmp_path / "registry_main")
+    if record:
+        (tmp_path / "record").write_text(record)
+    if driver:
+        (tmp_path / "registry_main").touch()
+        assert built_driver() == tmp_path / "registry_main"
+        return
+    with pytest.raises(pytest.skip.Exception if outcome == "skip" else AssertionError):
+        built_driver()
