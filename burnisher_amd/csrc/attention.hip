@@ -1,8 +1,8 @@
 // Flash attention for the dit-step on gfx950: softmax(scale * Q K^T, key mask) V over
 // head-last [batch, seq, heads, head_dim] operands, bf16 in and out, fp32 scores and softmax.
 //
-// Workgroup = 4 waves = 256 query rows of one (batch, head), each wave 4 tiles of 16, or 64 rows, a
-// tile a wave, where 256-row workgroups would leave the chip idle (flash_query_tiles). K/V stream through LDS in blocks of 64 keys, double-buffered, with the next
+// Workgroup = 4 waves = 64 query rows of one (batch, head), a tile of 16 a wave, or 256 rows, each wave 4
+// tiles, where those fill the CUs in whole rounds (flash_query_tiles). K/V stream through LDS in blocks of 64 keys, double-buffered, with the next
 // block's global loads in flight in registers while the current block is multiplied.
 //
 // Both products run on v_mfma_f32_16x16x32_bf16 and the kernel computes TRANSPOSED tiles:
@@ -24,6 +24,7 @@
 // skipping it changes nothing.
 #include "common.h"
 
+#include <atomic>
 #include <cmath>
 #include <mutex>
 
@@ -59,10 +60,17 @@ __device__ __forceinline__ float mask_at(const void* m, int f32, int64_t i) {
 
 // KS: K=32 steps of the score product (head_dim padded to 32*KS); DT: 16-row tiles of V^T; kQT: 16-row
 // query tiles per wave (64 kQT query rows per workgroup).
-// A one-tile workgroup is a chain of memory latencies, so two or more share a CU.
+// A one-tile workgroup is a chain of memory latencies, so two or more share a CU; its loads are
+// branch-free and its bias is loaded a block ahead. A four-tile wave has a SIMD to itself and no registers to
+// spare: its bias is loaded where it is added (held across the block, its 32 registers made head_dim 96 spill 47:
+// 16 heads of 4096 x 4096 578 us, 425 so), and its loads are branch-free only where a block's chunks fill
+// the threads (head_dim 64: 0.97 of the time with branches; 40: 1.03).
 template <int KS, int DT, bool VEC, int kQT>
 __global__ void __launch_bounds__(kThreads, kQT == 4 ? 1 : 2) k_flash(AttnArgs a) {
+    static_assert(kQT == 1 || kQT == 4, "query tiles per wave");
     constexpr int kQRows = 64 * kQT;
+    constexpr bool kAhead = kQT == 1;                              // the bias a block ahead
+    constexpr bool kClamp = VEC && (kQT == 1 || DT == 2 * KS);     // loads that clamp instead of branching
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     const int stage_elems = kKvBlk * a.k_row + DT * 16 * a.v_row;
     bf16_t* smem = reinterpret_cast<bf16_t*>(smem_raw);
@@ -118,7 +126,7 @@ __global__ void __launch_bounds__(kThreads, kQT == 4 ? 1 : 2) k_flash(AttnArgs a
             bf16x8_t f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) f[e] = static_cast<__bf16>(0.0f);
-            if (VEC) {   // D % 8 == 0; queries past the end read the last one, dims past D are zeroed
+            if (kClamp) {   // D % 8 == 0; queries past the end read the last one, dims past D are zeroed
                 f = *reinterpret_cast<const bf16x8_t*>(a.q + (b * a.Sq + min(qrow, a.Sq - 1)) * a.ld_q + h * D +
                                                        min(d0, D8 - 8));
                 if (d0 >= D8)
@@ -126,7 +134,9 @@ __global__ void __launch_bounds__(kThreads, kQT == 4 ? 1 : 2) k_flash(AttnArgs a
                     for (int e = 0; e < 8; ++e) f[e] = static_cast<__bf16>(0.0f);
             } else if (qrow < a.Sq && d0 < D8) {
                 const bf16_t* src = a.q + (b * a.Sq + qrow) * a.ld_q + h * D + d0;
-                {
+                if (VEC) {
+                    f = *reinterpret_cast<const bf16x8_t*>(src);
+                } else {
                     bf16_t tmp[8];
 #pragma unroll
                     for (int e = 0; e < 8; ++e) tmp[e] = (d0 + e < D) ? src[e] : 0;
@@ -146,7 +156,7 @@ __global__ void __launch_bounds__(kThreads, kQT == 4 ? 1 : 2) k_flash(AttnArgs a
 #pragma unroll
         for (int i = 0; i < kMaxChunks; ++i) {
             const int cidx = tid + i * kThreads;
-            if (VEC) {
+            if (kClamp) {
                 // No branch around a load (each would be waited for by itself): past the last chunk
                 // or key the last one is read again, and only what a key contributes is kept.
                 const int cc = min(cidx, nchunks - 1), row = cc / chunks_per_row, ch = cc % chunks_per_row;
@@ -164,15 +174,20 @@ __global__ void __launch_bounds__(kThreads, kQT == 4 ? 1 : 2) k_flash(AttnArgs a
                 const int64_t kv = static_cast<int64_t>(blk) * kKvBlk + row;
                 if (kv < a.Skv) {
                     const int64_t off = (b * a.Skv + kv) * a.ld_kv + h * D + ch * 8;
-                    bf16_t tk[8], tv[8];
+                    if (VEC) {
+                        rk[i] = *reinterpret_cast<const uint4*>(a.k + off);
+                        rv[i] = *reinterpret_cast<const uint4*>(a.v + off);
+                    } else {
+                        bf16_t tk[8], tv[8];
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const bool in = ch * 8 + e < D;
-                        tk[e] = in ? a.k[off + e] : 0;
-                        tv[e] = in ? a.v[off + e] : 0;
+                        for (int e = 0; e < 8; ++e) {
+                            const bool in = ch * 8 + e < D;
+                            tk[e] = in ? a.k[off + e] : 0;
+                            tv[e] = in ? a.v[off + e] : 0;
+                        }
+                        rk[i] = *reinterpret_cast<const uint4*>(tk);
+                        rv[i] = *reinterpret_cast<const uint4*>(tv);
                     }
-                    rk[i] = *reinterpret_cast<const uint4*>(tk);
-                    rv[i] = *reinterpret_cast<const uint4*>(tv);
                 }
             }
         }
@@ -199,8 +214,7 @@ __global__ void __launch_bounds__(kThreads, kQT == 4 ? 1 : 2) k_flash(AttnArgs a
             mbuf[stage * kKvBlk + tid] = kv < a.Skv ? mask_at(a.mask, a.mask_f32, b * a.Skv + kv) : 1.0f;
         }
     };
-    // The bias of a block as this lane's scores need it (four keys per tile): loaded with the block's
-    // K and V, one 8-byte load per tile where rows are 8-byte aligned. Keys past the end read the
+    // The bias of a block as this lane's scores need it (four keys per tile): one 8-byte load per tile where rows are 8-byte aligned. Keys past the end read the
     // last valid ones; their scores become -inf.
     uint2 braw[kKT][kQT];
     auto load_bias = [&](int blk) {
@@ -248,7 +262,7 @@ __global__ void __launch_bounds__(kThreads, kQT == 4 ? 1 : 2) k_flash(AttnArgs a
     while (blk < nblk && !block_live(blk)) ++blk;
     if (blk < nblk) {
         load_kv(blk);
-        load_bias(blk);
+        if (kAhead) load_bias(blk);
         store_kv(blk, 0);
     }
     __syncthreads();
@@ -286,6 +300,7 @@ __global__ void __launch_bounds__(kThreads, kQT == 4 ? 1 : 2) k_flash(AttnArgs a
 
         float bvals[kKT][kQT][4];
         if (a.bias) {
+            if (!kAhead) load_bias(blk);
 #pragma unroll
             for (int u = 0; u < kQT; ++u)
 #pragma unroll
@@ -295,7 +310,7 @@ __global__ void __launch_bounds__(kThreads, kQT == 4 ? 1 : 2) k_flash(AttnArgs a
                     bvals[t][u][2] = __uint_as_float(braw[t][u].y << 16);
                     bvals[t][u][3] = __uint_as_float(braw[t][u].y & 0xffff0000u);
                 }
-            if (next < nblk) load_bias(next);
+            if (kAhead && next < nblk) load_bias(next);
         }
         // scale, mask, running max, exponentials (base 2 with log2(e) folded into the scale)
         float mvals[kKT][4];
@@ -484,14 +499,43 @@ bf16_t* vt_workspace(size_t elems) {
     return static_cast<bf16_t*>(ptr[dev]);
 }
 
-// Query tiles per wave of the generic flash kernel: 4 (each K/V fragment read feeds four MFMAs) where
-// that makes four workgroups or more per CU; else 1, four times the workgroups and a quarter of the
-// work in each (a workgroup's key blocks run one after another, so its time sets the launch's), and
-// less padding in the last query block. T5 at 64 heads: 120 queries 17 -> 8.6 us, 2 x 300 queries 37 -> 31 us
-// in the encoder (16 us warm).
-int flash_query_tiles(const AttnShape& sh) {
-    const int64_t big = sh.batch * sh.heads * ((sh.q_len + 255) / 256);
-    return big >= 1024 ? 4 : 1;
+int device_cus() {
+    static std::atomic<int> cus[64] = {};
+    int dev = 0;
+    hip_check(hipGetDevice(&dev), "hipGetDevice");
+    require(dev >= 0 && dev < 64, "attention: device index out of range");
+    int n = cus[dev].load(std::memory_order_relaxed);
+    if (n == 0) {
+        hip_check(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev),
+                  "hipDeviceGetAttribute");
+        require(n > 0, "attention: device reports no compute units");
+        cus[dev].store(n, std::memory_order_relaxed);
+    }
+    return n;
+}
+
+// Query tiles per wave of the generic flash kernel: 4 (256 queries a workgroup, one per CU) or 1 (64 queries,
+// two to four of them sharing a CU and hiding each other's latencies). Both give the same bits. The time of
+// either form is its key blocks, one after another, times the workgroups a CU takes in turn, so the rule
+// compares those; the key count is in both alike. Unit: what a CU takes for one four-tile workgroup. Measured
+// at 8 to 128 heads, 77 to 4096 keys (the ends of a range in brackets):
+//  - head_dim <= 32, or above 96 with 16-byte loads: one tile always (0.57 to 0.95 and 0.35 to 0.75 of the time);
+//  - 33 to 64: one-tile workgroups cost 0.49, 0.58, 0.69 for one, two or three on a CU and 0.2 each in long
+//    rows, so they win except where exactly one round of four-tile workgroups is nearly full and the fourth
+//    one-tile workgroup of a CU would wait (16 heads x 4096 queries x 120 keys at 64: 18.0 against 16.5 us);
+//  - 65 to 96: two one-tile workgroups fit a CU and cost 0.6 together (32 x 4096 x 4096 at 96: 955 against
+//    847 us; but 24 x 4096 x 4096, a round and a half: 720 against 845);
+//  - element-wise loads (head_dim not a multiple of 8, or unaligned): a workgroup stages K and V one element
+//    at a time whatever its queries, and a one-tile workgroup costs 0.3 (64 x 2048 x 300 at 50: 105 against 95 us).
+int flash_query_tiles(const AttnShape& sh, bool vec) {
+    const int64_t ks = (sh.head_dim + 31) / 32;
+    if (ks == 1 || (ks == 4 && vec)) return 1;
+    const int64_t cus = device_cus(), groups = sh.batch * sh.heads;
+    const int64_t four = groups * ((sh.q_len + 255) / 256), one = groups * ((sh.q_len + 63) / 64);
+    const int64_t rounds = (four + cus - 1) / cus, per_cu = (one + cus - 1) / cus;
+    if (ks == 3) return 10 * rounds <= 6 * ((per_cu + 1) / 2) ? 4 : 1;
+    if (!vec) return 10 * rounds <= 3 * per_cu ? 4 : 1;
+    return rounds == 1 && per_cu == 4 ? 4 : 1;
 }
 
 // Which kernel launch_attention_bf16 runs for these operands, and the V^T elements it needs.
@@ -602,7 +646,7 @@ void launch_attention_bf16(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf
     // V^T rows of 136 bytes: the transposed 2-byte writes of a wave (8 chunks of 8 rows) then meet
     // two to a bank instead of four, and 16 rows' 8-byte reads touch all banks once.
     a.v_row = kKvBlk + 4;
-    const int qt = flash_query_tiles(sh);
+    const int qt = flash_query_tiles(sh, vec);
     a.qb = static_cast<int>((sh.q_len + 64 * qt - 1) / (64 * qt));
     const int ks = static_cast<int>((sh.head_dim + 31) / 32);
     const int dt = static_cast<int>((sh.head_dim + 15) / 16);
@@ -613,31 +657,29 @@ void launch_attention_bf16(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf
                          sh.head_dim;
     ProfileScope ps(sh.q_len == sh.kv_len ? K_ATTN_SELF : K_ATTN_CROSS, s, flops);
     // Above 64 KiB of dynamic LDS (head_dim > 96) the launch must opt in to the larger size.
-#define BH_FLASH_K(KS_, DT_, VEC_, QT_)                                                    \
-    do {                                                                                   \
-        if (lds > 65536)                                                                   \
-            hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_flash<KS_, DT_, VEC_, QT_>), \
-                                          hipFuncAttributeMaxDynamicSharedMemorySize,      \
-                                          static_cast<int>(lds)), "hipFuncSetAttribute");  \
-        k_flash<KS_, DT_, VEC_, QT_><<<grid, kThreads, lds, s>>>(a);                       \
-    } while (0)
-#define BH_FLASH(KS_, DT_)                                                                 \
-    do {                                                                                   \
-        if (vec && qt == 4) BH_FLASH_K(KS_, DT_, true, 4);                                 \
-        else if (vec) BH_FLASH_K(KS_, DT_, true, 1);                                       \
-        else if (qt == 4) BH_FLASH_K(KS_, DT_, false, 4);                                  \
-        else BH_FLASH_K(KS_, DT_, false, 1);                                               \
-    } while (0)
-    if (ks == 1 && dt == 1) BH_FLASH(1, 1);
-    else if (ks == 1) BH_FLASH(1, 2);
-    else if (ks == 2 && dt == 3) BH_FLASH(2, 3);
-    else if (ks == 2) BH_FLASH(2, 4);
-    else if (ks == 3 && dt == 5) BH_FLASH(3, 5);
-    else if (ks == 3) BH_FLASH(3, 6);
-    else if (dt == 7) BH_FLASH(4, 7);
-    else BH_FLASH(4, 8);
+    auto launch = [&](void (*kernel)(AttnArgs)) {
+        if (lds > 65536)
+            hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)),
+                      "hipFuncSetAttribute");
+        kernel<<<grid, kThreads, lds, s>>>(a);
+    };
+#define BH_FLASH(KS_, DT_, QT_) launch(vec ? &k_flash<KS_, DT_, true, QT_> : &k_flash<KS_, DT_, false, QT_>)
+    if (ks == 1 && dt == 1) BH_FLASH(1, 1, 1);
+    else if (ks == 1) BH_FLASH(1, 2, 1);
+    else if (ks == 2 && dt == 3 && qt == 1) BH_FLASH(2, 3, 1);
+    else if (ks == 2 && dt == 3) BH_FLASH(2, 3, 4);
+    else if (ks == 2 && qt == 1) BH_FLASH(2, 4, 1);
+    else if (ks == 2) BH_FLASH(2, 4, 4);
+    else if (ks == 3 && dt == 5 && qt == 1) BH_FLASH(3, 5, 1);
+    else if (ks == 3 && dt == 5) BH_FLASH(3, 5, 4);
+    else if (ks == 3 && qt == 1) BH_FLASH(3, 6, 1);
+    else if (ks == 3) BH_FLASH(3, 6, 4);
+    else if (dt == 7 && qt == 1) BH_FLASH(4, 7, 1);
+    else if (dt == 7) launch(&k_flash<4, 7, false, 4>);
+    else if (qt == 1) BH_FLASH(4, 8, 1);
+    else launch(&k_flash<4, 8, false, 4>);
 #undef BH_FLASH
-#undef BH_FLASH_K
     launch_check("attention (flash)");
 }
 

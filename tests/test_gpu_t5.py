@@ -189,3 +189,36 @@ def test_t5_weights_from_a_sharded_checkpoint_and_the_encode_stage(hip, tmp_path
     with contextlib.redirect_stdout(io.StringIO()):
         assert stage.main(["t5-encode", "--weights", str(tmp_path / "bad"), "--ids", str(ids), "--out",
                            str(out), "--config", json.dumps(cfg)]) == 1
+
+
+@pytest.mark.parametrize("D,H,S,K", [(64, 128, 512, 70), (40, 120, 500, 33), (80, 192, 250, 70), (96, 256, 200, 130),
+                                     (35, 128, 450, 20), (50, 120, 512, 65), (70, 200, 256, 64), (90, 256, 201, 70),
+                                     (100, 250, 250, 33), (117, 256, 256, 65)], ids=str)
+def test_attention_query_tile_forms_agree(hip, D, H, S, K):
+    """Grids that fill 256 CUs once with workgroups of 256 queries (four query tiles a wave), with 16-byte
+    and element-wise loads, against the first and last heads on their own (a tile a wave), bit for bit, and
+    those against the oracle; ragged query and key blocks, a bias and a mask."""
+    import torch
+    rng = np.random.default_rng(17)
+    q = randn_bf16(rng, (1, S, H, D))
+    k, v = (randn_bf16(rng, (1, K, H, D)) for _ in range(2))
+    bias, mask = randn_bf16(rng, (H, S, K), 2.0), np.ones((1, K), np.float32)
+    mask[0, K // 2::3] = 0
+
+    def run(heads):
+        pick = lambda x: np.ascontiguousarray(x[:, :, heads])  # noqa: E731
+        n = len(range(H)[heads])
+        a, b, c, bi, m = dev(pick(q)), dev(pick(k)), dev(pick(v)), dev(bias[heads]), torch.from_numpy(mask).cuda()
+        out = torch.zeros((1, S, n, D), dtype=torch.bfloat16, device="cuda")
+        bh.call("bh_attention", a.data_ptr(), b.data_ptr(), c.data_ptr(), out.data_ptr(), 1, n, S, K, D, 0.0,
+                bi.data_ptr(), m.data_ptr(), F32, BF16, None)
+        return host(out)
+
+    whole, few = run(slice(0, H)), slice(0, 3)
+    for heads in (few, slice(H - 2, H)):
+        assert np.array_equal(whole[:, :, heads], run(heads))
+    want = np.zeros((1, S, 3, D), np.uint16)
+    args = [np.ascontiguousarray(x[:, :, few]) for x in (q, k, v)] + [want]
+    oracle.call(oracle.stock(), "stock_attention", *(addr(x) for x in args), 1, 3, S, K, D, 0.0,
+                addr(np.ascontiguousarray(bias[few])), addr(mask), F32, BF16, 0, 0)
+    assert_within(from_bf16(np.ascontiguousarray(whole[:, :, few])), from_bf16(want), "attention", f"tiles {D} {H} {S} {K}")

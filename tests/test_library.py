@@ -120,3 +120,35 @@ def test_a_missing_registry_driver_is_skipped_only_without_sources(monkeypatch, 
         return
     with pytest.raises(pytest.skip.Exception if outcome == "skip" else AssertionError):
         built_driver()
+
+
+def kernel_metadata(tmp_path):
+    """name -> (VGPR spills, scratch bytes) of every kernel of the built library."""
+    import shutil
+    import subprocess
+    llvm = Path("/opt/rocm/llvm/bin")
+    lib = tmp_path / "lib.so"
+    shutil.copy(bh.LIB_PATH, lib)   # the code objects are extracted beside it
+    subprocess.run([llvm / "llvm-objdump", "--offloading", lib], check=True, capture_output=True)
+    out = {}
+    for obj in tmp_path.glob("lib.so.*gfx950"):
+        notes = subprocess.run([llvm / "llvm-readelf", "--notes", obj], check=True, capture_output=True,
+                               text=True).stdout
+        for entry in re.split(r"\n\s+- \.agpr_count", notes)[1:]:
+            field = lambda n: re.search(rf"\.{n}:\s+(\S+)", entry).group(1)  # noqa: E731
+            out[field("symbol").removesuffix(".kd")] = (int(field("vgpr_spill_count")),
+                                                       int(field("private_segment_fixed_size")))
+    return out
+
+
+def test_generic_flash_kernels_stay_in_registers(tmp_path):
+    # k_flash<KS, DT, VEC, tiles>: a vector register written to scratch is written and read again for every
+    # key block. Up to head_dim 96 a handful at most (47 there cost a third of the time); one tile
+    # a wave none.
+    flash = {n: v for n, v in kernel_metadata(tmp_path).items() if "7k_flashILi" in n}
+    assert len(flash) >= 24
+    for name, (spills, scratch) in flash.items():
+        ks = int(name.split("7k_flashILi")[1][0])
+        one = "ELi1EEEv" in name
+        if one or ks <= 3:
+            assert spills <= (0 if one else 8), f"{name}: {spills} spills, {scratch} bytes of scratch"
