@@ -279,8 +279,9 @@ __device__ __forceinline__ void smallk_store(const Epi& e, int mode, const float
 // The same for the plain and the row-add store at K = 8 or 16 (a patch embedding of 2 x 2 patches,
 // whose row add is the position table). A wave owns 128 columns, two a lane, their weights in registers, and walks a
 // band of rows: a row's K inputs are the same for all its lanes, so they are scalar loads, four rows in flight, and the
-// lanes read and write whole lines. With eight columns a lane the weights' loads were 256 bytes apart and a
-// wave computed only four rows with them: 10368 x 1152 x 16 took 28.5 us, here 19.
+// lanes read and write whole lines. With eight columns a lane (k_gemm_smallk) the weights' loads are 256 bytes
+// apart and a wave computes only four rows with them: 10368 x 1152 x 16 took 28.5 us, here 19. Where that form
+// is the better one: smallk_banded.
 constexpr int kWaveCols = 128, kWaveRows = 4;
 template <int KC>
 __global__ void __launch_bounds__(256) k_gemm_smallk_wave(const uint32_t* __restrict__ A, const bf16_t* __restrict__ B,
@@ -359,6 +360,60 @@ __global__ void __launch_bounds__(256) k_gemm_smallk(const bf16_t* __restrict__ 
 #pragma unroll
                 for (int t = 0; t < 8; ++t) w[r][8 * c + t] = f[t];
             }
+        if (m1 - m0 == kSmallKRows && (mode == EPI_STORE || mode == EPI_ROW_ADD)) {
+            // A whole band of a plain or row-add store (the patch embedding, whose row add is the
+            // position table): every A row and every row-add row is loaded before the first store,
+            // one memory round trip for the band instead of one per row.
+            uint4 ar[kSmallKRows][KC], ra[kSmallKRows];
+#pragma unroll
+            for (int i = 0; i < kSmallKRows; ++i) {
+#pragma unroll
+                for (int c = 0; c < KC; ++c)
+                    ar[i][c] = *reinterpret_cast<const uint4*>(A + static_cast<int64_t>(m0 + i) * kK + 8 * c);
+                if (mode == EPI_ROW_ADD) {
+                    const int pr = static_cast<int>((m0 + i) % static_cast<int>(e.row_add_period));
+                    ra[i] = *reinterpret_cast<const uint4*>(e.row_add + static_cast<int64_t>(pr) * N + n0);
+                }
+            }
+            float bias[8];
+            if (e.bias) {
+                unpack8(*reinterpret_cast<const uint4*>(e.bias + n0), bias);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 8; ++r) bias[r] = -0.0f;   // v + (-0.0) is v exactly
+            }
+#pragma unroll
+            for (int i = 0; i < kSmallKRows; ++i) {
+                float a[kK];
+#pragma unroll
+                for (int c = 0; c < KC; ++c) {
+                    float f[8];
+                    unpack8(ar[i][c], f);
+#pragma unroll
+                    for (int t = 0; t < 8; ++t) a[8 * c + t] = f[t];
+                }
+                float v[8];
+#pragma unroll
+                for (int r = 0; r < 8; ++r) {
+                    float acc = 0.f;
+#pragma unroll
+                    for (int t = 0; t < kK; ++t) acc = __fadd_rn(acc, __fmul_rn(a[t], w[r][t]));
+                    v[r] = act_exact(e.act, __fadd_rn(acc, bias[r]));
+                }
+                if (mode == EPI_ROW_ADD) {
+                    float t[8];
+                    if (e.round_mid) {
+#pragma unroll
+                        for (int r = 0; r < 8; ++r) v[r] = round_bf16(v[r]);
+                    }
+                    unpack8(ra[i], t);
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) v[r] = __fadd_rn(v[r], t[r]);
+                }
+                *reinterpret_cast<uint4*>(out + static_cast<int64_t>(m0 + i) * e.ld_out + n0) = pack8(v);
+            }
+            return;
+        }
         for (int m = m0; m < m1; ++m) {
             float a[kK];
 #pragma unroll
@@ -396,6 +451,16 @@ __global__ void __launch_bounds__(256) k_gemm_smallk(const bf16_t* __restrict__ 
             smallk_store(e, mode, acc, m, n0, N, out);
         }
     }
+}
+
+// Whether a plain or row-add store at K = 8 or 16 keeps eight columns a thread. A wave of
+// k_gemm_smallk_wave takes its 128 columns' time however few of them exist: about 75 ps a row at K = 8 and 105 at 16,
+// against 0.8 and 1.6 ps a column here (400000 x 8 x 16: 43 against 7.8 us, x 48 43 / 36, x 72 43 / 50; 65536 x 160 x 8
+// 13.4 / 12.5, x 208 13.8 / 16.7). With fewer rows than fill the chip with waves of four the time is latency, and
+// there the wave form is the shorter chain (16384 x 64 x 8: 0.8 of the time, x 16 0.7).
+bool smallk_banded(int64_t m, int64_t n, int64_t k) {
+    const int64_t chunks = (n + kWaveCols - 1) / kWaveCols;
+    return k == 8 ? m >= 24576 && n <= 96 * chunks : m >= 32768 && n <= 64 * chunks;
 }
 
 // Compute units of the current device, looked up once per device.
@@ -828,10 +893,11 @@ void launch_gemm_bf16(const bf16_t* a, const bf16_t* b, const bf16_t* bias, bf16
     if (k8 && k % BK != 0 && vec && k <= 256 && m * (n / 8) < (int64_t{1} << 31) &&
         e.row_add_period < (int64_t{1} << 31) && e.gate_rows < (int64_t{1} << 31)) {
         ProfileScope ps(K_GEMM, s, flops);
-        if ((k == 8 || k == 16) && (mode == EPI_STORE || mode == EPI_ROW_ADD)) {
-            // rows per wave: many share a wave's weights, while the chip has two waves a SIMD
+        if ((k == 8 || k == 16) && (mode == EPI_STORE || mode == EPI_ROW_ADD) && !smallk_banded(m, n, k)) {
+            // rows per wave: many share a wave's weights, while the chip has eight waves a SIMD (with two, a
+            // wave's row loads are waited for: 4096 x 1160 x 8 8.4 us, with eight 6.9)
             const int64_t chunks = (n + kWaveCols - 1) / kWaveCols;
-            const int64_t band = std::max<int64_t>(kWaveRows, std::min<int64_t>(32, m * chunks / 2048 / kWaveRows * kWaveRows));
+            const int64_t band = std::max<int64_t>(kWaveRows, std::min<int64_t>(32, m * chunks / 8192 / kWaveRows * kWaveRows));
             const int grid = static_cast<int>(((m + band - 1) / band * chunks + 3) / 4);
             const uint32_t* aw = reinterpret_cast<const uint32_t*>(a);
             const int mi = static_cast<int>(m), ni = static_cast<int>(n), bi = static_cast<int>(band);

@@ -198,6 +198,49 @@ def test_gemm_small_k_wave_bands(hip, M, d, K, act):
     assert_within(from_bf16(host(out, want)), from_bf16(want), "gemm", f"small K {M}x{d}x{K}")
 
 
+@pytest.mark.parametrize("M,d,K", [(24576, 96, 8), (24575, 96, 8), (24577, 104, 8), (24578, 192, 8), (24576, 200, 8),
+                                   (32768, 64, 16), (32767, 64, 16), (32770, 72, 16), (32769, 8, 16)], ids=str)
+def test_gemm_small_k_narrow_columns(hip, M, d, K):
+    # Both sides of the line between eight columns a thread (whole and ragged last bands) and a wave over
+    # 128: plain stores against the oracle, the row-add store against the plain one and the add.
+    import burnisher_amd as bh
+    import ctypes
+    import torch
+    rng = np.random.default_rng(47)   # its own: the other tests' inputs stay what they were
+    period = 1 + M // 3
+    a, w, bias = randn_bf16(rng, (M, K)), randn_bf16(rng, (d, K), 0.3), randn_bf16(rng, (d,), 0.3)
+    pos = randn_bf16(rng, (period, d))
+    want = np.zeros((M, d), np.uint16)
+    st("stock_gemm", addr(a), addr(w), addr(bias), addr(want), M, d, K, 1, 0, BF16, 0)
+    da, dw, db, dpos, out, added = dev(a), dev(w), dev(bias), dev(pos), empty((M, d)), empty((M, d))
+    call("bh_gemm", P(da), P(dw), P(db), P(out), M, d, K, 1, 0, BF16, None)
+    assert_within(from_bf16(host(out, want)), from_bf16(want), "gemm", f"small K {M}x{d}x{K}")
+    f = bh.GemmFused(epilogue=0, round_mid=1, row_add=P(dpos), row_add_period=period, ld_out=d)
+    call("bh_gemm_fused_run", P(da), P(dw), P(db), P(added), M, d, K, ctypes.byref(f), None)
+    sums = (out.float() + dpos[torch.arange(M, device="cuda") % period].float()).to(torch.bfloat16)
+    assert torch.equal(added, sums)
+
+
+def test_gemm_small_k_few_columns_cost_less(hip):
+    # 8 of a wave's 128 columns once took the time of 128.
+    import torch
+
+    def us(d):
+        a, w, out = (torch.zeros(s, dtype=torch.bfloat16, device="cuda") for s in ((400000, 16), (d, 16), (400000, d)))
+        t = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        best = 1e9
+        for _ in range(6):
+            t[0].record()
+            for _ in range(20):
+                call("bh_gemm", P(a), P(w), None, P(out), 400000, d, 16, 1, 0, BF16, None)
+            t[1].record()
+            torch.cuda.synchronize()
+            best = min(best, t[0].elapsed_time(t[1]) / 20 * 1e3)
+        return best
+    few, all_ = us(8), us(128)
+    assert few < 0.6 * all_, f"8 columns {few:.1f} us, 128 columns {all_:.1f}"
+
+
 @pytest.mark.parametrize("B,N_tok", [(2, 1024), (7, 143)], ids=["whole_bands", "ragged_band"])
 def test_gemm_small_k_fused_epilogues(hip, B, N_tok):
     # K = 16, the patch embedding's in_channels * patch^2: the register-weight kernel. Whole bands
