@@ -81,11 +81,14 @@ constexpr int kGemvMaxM = 8;
 // The dot products of one weight row with M <= MM rows of A, every lane's sums over its octets in
 // order, then over the wave; valid in all lanes. What bounds these launches is the latency of
 // their loads (a wave reads a few KiB), so the octets of four rounds are requested together: with one round trip
-// per round the adaLN projection (6912 x 1152, 16 MB) took three of them.
+// per round the adaLN projection (6912 x 1152, 16 MB) took three of them. Rows past M repeat the last, so
+// that no load waits behind a branch; MM follows M in steps of two, because a repeated row costs what a row
+// does (3 x 20480 x 4096 on MM = 8 50 us, on 4 32; 5 on 8 51, on 6 42). More rows, fewer rounds at once: the
+// registers hold MM + 1 octets of each.
 template <int MM>
 __device__ __forceinline__ void gemv_row(const bf16_t* __restrict__ A, const bf16_t* __restrict__ Bn, int M,
                                          int64_t K, int lane, float (&part)[MM]) {
-    constexpr int U = MM <= 2 ? 4 : 1;
+    constexpr int U = MM <= 2 ? 4 : MM <= 4 ? 2 : 1;
 #pragma unroll
     for (int m = 0; m < MM; ++m) part[m] = 0.f;
     const int64_t chunks = K / 8;
@@ -880,8 +883,8 @@ void launch_gemm_bf16(const bf16_t* a, const bf16_t* b, const bf16_t* bias, bf16
     if (k8 && m <= kGemvMaxM) {
         ProfileScope ps(K_GEMV, s, flops);
         const int grid = static_cast<int>((n + 3) / 4);
-        if (m <= 2) k_gemv<2><<<grid, 256, 0, s>>>(a, b, out, m, n, k, e, mode, ep.silu_out);
-        else k_gemv<kGemvMaxM><<<grid, 256, 0, s>>>(a, b, out, m, n, k, e, mode, ep.silu_out);
+        auto* kernel = m <= 2 ? &k_gemv<2> : m <= 4 ? &k_gemv<4> : m <= 6 ? &k_gemv<6> : &k_gemv<kGemvMaxM>;
+        kernel<<<grid, 256, 0, s>>>(a, b, out, m, n, k, e, mode, ep.silu_out);
         launch_check("gemm (small M)");
         return;
     }
@@ -971,10 +974,9 @@ void launch_adaln_chunks(const bf16_t* a, const bf16_t* w, const bf16_t* bias, c
                          hipStream_t s) {
     ProfileScope ps(K_GEMV, s, 2.0 * batch * 6 * channels * channels);
     const int grid = static_cast<int>(6 * channels / 8), m = static_cast<int>(batch);
-    if (m <= 2)
-        k_adaln_chunks<2><<<grid, 512, 0, s>>>(a, w, bias, tables_dev, out, out_f32, layers, m, channels);
-    else
-        k_adaln_chunks<kGemvMaxM><<<grid, 512, 0, s>>>(a, w, bias, tables_dev, out, out_f32, layers, m, channels);
+    auto* kernel = m <= 2 ? &k_adaln_chunks<2> : m <= 4 ? &k_adaln_chunks<4> : m <= 6 ? &k_adaln_chunks<6>
+                                                                                     : &k_adaln_chunks<kGemvMaxM>;
+    kernel<<<grid, 512, 0, s>>>(a, w, bias, tables_dev, out, out_f32, layers, m, channels);
     launch_check("adaln_chunks");
 }
 

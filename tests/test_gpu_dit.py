@@ -211,6 +211,17 @@ def test_first_and_last_launches_equal_the_ops(hip, heads, dim, out, batch, hw, 
         b.close()
 
 
+@pytest.mark.parametrize("batch", [2, 4, 5, 6, 7, 8])
+def test_adaln_projection_of_every_batch_equals_the_ops(hip, batch):
+    wl = make_workload(dict(SMALL, num_layers=2), batch=batch, latent_hw=8, caption_len=4)
+    a, b = Engine(wl, 0), Engine(wl, 1)
+    try:
+        assert np.array_equal(a.forward(), b.forward())
+    finally:
+        a.close()
+        b.close()
+
+
 @pytest.mark.parametrize("cfg,batch,hw,cap,layers", [
     (PIXART_SIGMA, 2, 64, 300, 2),   # the CFG pair at 512px: one row per stream, head_dim 72
     (SMALL, 3, 8, 5, None),          # groups of two rows and one, the generic attention

@@ -57,6 +57,21 @@ def call(name, *args):
     bh.call(name, *args)
 
 
+def best_us(a, w, out, m, n, k):
+    """The shortest of six runs of 20 plain GEMM calls, microseconds a call."""
+    import torch
+    t = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    best = 1e9
+    for _ in range(6):
+        t[0].record()
+        for _ in range(20):
+            call("bh_gemm", P(a), P(w), None, P(out), m, n, k, 1, 0, BF16, None)
+        t[1].record()
+        torch.cuda.synchronize()
+        best = min(best, t[0].elapsed_time(t[1]) / 20 * 1e3)
+    return best
+
+
 def st(name, *args):
     oracle.call(oracle.stock(), name, *args)
 
@@ -128,6 +143,39 @@ def test_gemm_tile_heights_agree_gated_residual(hip):
         results[rows] = host(dx, x[:rows])
     for rows in (4608, 2048):
         assert np.array_equal(results[rows], results[M][:rows]), f"{rows} rows differ from {M}"
+
+
+@pytest.mark.parametrize("K", [72, 512, 1160, 4104])
+def test_gemm_few_rows_agree_with_each_alone(hip, K):
+    # One to eight rows: a wave per column, rows in pairs past the last one, one, two or four rounds of
+    # octets at once. Every row has the bits it has alone, and those are the oracle's within the gate.
+    rng = np.random.default_rng(53)   # its own: the other tests' inputs stay what they were
+    N = 100
+    a, w, bias = randn_bf16(rng, (8, K)), randn_bf16(rng, (N, K), 0.1), randn_bf16(rng, (N,), 0.1)
+    want = np.zeros((8, N), np.uint16)
+    st("stock_gemm", addr(a), addr(w), addr(bias), addr(want), 8, N, K, 1, 2, BF16, 0)
+    alone = []
+    for m in range(8):
+        out = empty((1, N))
+        call("bh_gemm", P(dev(a[m])), P(dev(w)), P(dev(bias)), P(out), 1, N, K, 1, 2, BF16, None)
+        alone.append(host(out, want[:1])[0])
+    assert_within(from_bf16(np.stack(alone)), from_bf16(want), "gemm", f"rows alone K {K}")
+    for M in range(2, 9):
+        out = empty((M, N))
+        call("bh_gemm", P(dev(a[:M])), P(dev(w)), P(dev(bias)), P(out), M, N, K, 1, 2, BF16, None)
+        assert np.array_equal(host(out, want[:M]), np.stack(alone[:M])), f"{M} rows"
+
+
+def test_gemm_three_rows_cost_less_than_eight(hip):
+    # Three rows once took what eight do.
+    import torch
+
+    def us(m):
+        return best_us(*(torch.zeros(s, dtype=torch.bfloat16, device="cuda")
+                         for s in ((m, 4096), (20480, 4096), (m, 20480))), m, 20480, 4096)
+
+    three, eight = us(3), us(8)
+    assert three < 0.8 * eight, f"three rows {three:.1f} us, eight {eight:.1f}"
 
 
 def test_gemm_unaligned_k_and_plain_layouts(hip):
@@ -226,17 +274,9 @@ def test_gemm_small_k_few_columns_cost_less(hip):
     import torch
 
     def us(d):
-        a, w, out = (torch.zeros(s, dtype=torch.bfloat16, device="cuda") for s in ((400000, 16), (d, 16), (400000, d)))
-        t = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
-        best = 1e9
-        for _ in range(6):
-            t[0].record()
-            for _ in range(20):
-                call("bh_gemm", P(a), P(w), None, P(out), 400000, d, 16, 1, 0, BF16, None)
-            t[1].record()
-            torch.cuda.synchronize()
-            best = min(best, t[0].elapsed_time(t[1]) / 20 * 1e3)
-        return best
+        return best_us(*(torch.zeros(s, dtype=torch.bfloat16, device="cuda")
+                         for s in ((400000, 16), (d, 16), (400000, d))), 400000, d, 16)
+
     few, all_ = us(8), us(128)
     assert few < 0.6 * all_, f"8 columns {few:.1f} us, 128 columns {all_:.1f}"
 
