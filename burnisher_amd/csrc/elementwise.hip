@@ -719,6 +719,11 @@ __device__ __forceinline__ float silu_from_bf16(float x) {
     return __fmul_rn(0.25f * x, r);
 }
 
+// From how many values on a GELU goes eight a thread. Below, one thread's eight in turn are the launch's time
+// (4096 values 2.1 us, one a thread 1.8; 524288 2.37 / 2.22; 1048576 2.7 / 3.0); SiLU and the copy are as
+// short either way (1.8).
+constexpr int64_t kGeluVector = int64_t{1} << 20;
+
 // The same, eight bf16 values per access (n8 octets). SiLU is bound by memory: 15.4 -> 10.5 us a call on
 // average over 18.9M and 9.4M values (5.4 TB/s); before, by the exact exponential and division, as GELU is.
 template <int KIND>
@@ -1224,7 +1229,8 @@ void launch_activation(const void* x, void* out, int64_t numel, int kind, const 
         k_activation<float><<<grid_for(numel), 256, 0, s>>>(
             static_cast<const float*>(x), static_cast<float*>(out), numel, kind,
             static_cast<const float*>(gate));
-    } else if (numel % 8 == 0 && aligned16(x) && aligned16(out) && (!gate || aligned16(gate))) {
+    } else if (numel % 8 == 0 && aligned16(x) && aligned16(out) && (!gate || aligned16(gate)) &&
+               (kind == 0 || kind == 2 || numel >= kGeluVector)) {
         auto* k = kind == 0 ? k_activation_v8<0> : kind == 2 ? k_activation_v8<2> : kind == 3 ? k_activation_v8<3>
                                                                                             : k_activation_v8<1>;
         k<<<grid_for(numel / 8), 256, 0, s>>>(static_cast<const bf16_t*>(x), static_cast<bf16_t*>(out), numel / 8,

@@ -43,6 +43,12 @@ def host(t, like):
     return t.cpu().numpy().reshape(like.shape)
 
 
+def torch_equal(a, b):
+    """The same bits (NaN included)."""
+    import torch
+    return torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
 def empty(shape, bf16=True):
     import torch
     return torch.zeros(shape, dtype=torch.bfloat16 if bf16 else torch.float32, device="cuda")
@@ -624,6 +630,45 @@ def test_silu_every_bf16_value(hip):
     nan = np.isnan(from_bf16(want))
     assert np.array_equal(np.isnan(from_bf16(got)), nan)
     assert np.array_equal(got[~nan], want[~nan])
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2, 3])
+def test_activation_vectors_equal_single_values(hip, kind):
+    """Eight values a thread (GELU from 2^20 on) against one (a count that is no multiple of eight), bit for bit."""
+    rng = np.random.default_rng(59)   # its own: the other tests' inputs stay what they were
+    n = 1 << 20
+    x, g = randn_bf16(rng, (n + 1,), 3.0), randn_bf16(rng, (n + 1,))
+    dx, dg = dev(x), dev(g)
+    want = empty((n + 1,))
+    call("bh_activation", P(dx), P(want), n + 1, kind, P(dg) if kind == 3 else None, BF16, None)
+    for count in (8, 4096, n - 8, n):
+        got = empty((count,))
+        call("bh_activation", P(dx), P(got), count, kind, P(dg) if kind == 3 else None, BF16, None)
+        assert torch_equal(got, want[:count]), f"kind {kind}, {count} values"
+
+
+def test_gelu_of_few_values_goes_one_a_thread(hip):
+    # Eight in turn on one thread were the launch's time at a few thousand values (1.19 of it).
+    import torch
+    x, out = (torch.ones(4104, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    t = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+
+    def us(n):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(100):
+                call("bh_activation", P(x), P(out), n, 1, None, BF16, torch.cuda.current_stream().cuda_stream)
+        best = 1e9
+        for _ in range(8):
+            t[0].record()
+            graph.replay()
+            t[1].record()
+            torch.cuda.synchronize()
+            best = min(best, t[0].elapsed_time(t[1]) * 10)
+        return best
+
+    whole, ragged = us(4096), us(4097)
+    assert whole < 1.1 * ragged, f"4096 values {whole:.2f} us, 4097 {ragged:.2f}"
 
 
 def test_add_chunk_activation_patch(hip):
