@@ -498,6 +498,13 @@ void launch_tn(const bf16_t* a, const bf16_t* b, bf16_t* out, int64_t m, int64_t
     // 16 / MT M-tiles (1024 rows; 960 at the 192-row tile) at a time whatever the tile height.
     int grid = min(tiles, device_cus() & ~7);
     if (grid < 8) grid = min(tiles, device_cus());
+    // Only the staged epilogue of a workgroup's last tile knows the narrow widths and a V^T store of short
+    // tiles: a second tile would be lost.
+    if constexpr (NT < 8) require(grid == tiles, "gemm: a tile narrower than 128 columns is its workgroup's only one");
+    if constexpr (MT < kMaxMT)
+        if (e.vt)
+            require(MT <= 2 && NT == kNT && grid == tiles,
+                    "gemm: a transposed V store takes 144-wide tiles of 256 rows, or of 64 or 128 one to a workgroup");
     k_gemm_tn<ACT, MODE, MT, NT><<<grid, kWgThreads, 0, s>>>(a, b, out, m, n, k, e, tiles_m, tiles_n, 16 / MT);
 }
 
@@ -623,6 +630,8 @@ void launch_tn_splitk(const bf16_t* a, const bf16_t* b, float* partial, int64_t 
     const int tiles_n = static_cast<int>((n + kBN<NT> - 1) / kBN<NT>);
     const int tiles = tiles_m * tiles_n;
     const int grid = max(1, min(tiles, device_cus() / splits));
+    if constexpr (NT < 8)
+        require(grid == tiles, "gemm split-K: a tile narrower than 128 columns is its workgroup's only one");
     Epi e{};
     e.row_add_period = 1;
     e.gate_rows = 1;
