@@ -78,8 +78,6 @@ Plan plan_of(const bh_vae_config& c) {
     return p;
 }
 
-bool mfma_conv(int64_t ci, int64_t co) { return ci % 64 == 0 && co % 8 == 0; }
-
 }  // namespace
 
 // Every tensor the decoder reads with its checkpoint shape (the VAE part of declare_pixart_shapes,
@@ -183,13 +181,13 @@ struct Run {
         ep.residual = residual;
         ep.round_mid = residual != nullptr;
         const int64_t rows = (co / e.cfg.norm_num_groups) % 4 == 0 ? conv3x3_stats_rows(g, co) : 0;
-        const bool fits = rows > 0 && rows * (co / 4) * 16 <= e.gn_part_bytes;
+        require(rows * (co / 4) * 16 <= e.gn_part_bytes, "vae: the GroupNorm sums do not fit their buffer");
         const auto padded = e.rw.find(n + ".bias");
         const bf16_t* bias = padded != e.rw.end() ? padded->second : e.at(n + ".bias");
         launch_conv3x3_bf16(g, e.rw.at(n + ".weight"), bias, out, co, ep, s,
-                            fits ? e.gn.part : nullptr, fused ? e.gn.channels : nullptr);
-        summed = fits ? out : nullptr;
-        sum_rows = fits ? rows : 0;
+                            rows > 0 ? e.gn.part : nullptr, fused ? e.gn.channels : nullptr);
+        summed = rows > 0 ? out : nullptr;
+        sum_rows = rows;
     }
 
     // out = x . W^T + bias over [h*h, ci] (a 1x1 conv or a linear layer), optionally + residual
@@ -367,9 +365,8 @@ int bh_vae_create(const bh_vae_config* cfg, const bh_vae_weights* w, int64_t lat
             e->gn_part_bytes = bytes;
         }
         e->gn.channels = static_cast<bh::NormChannel*>(e->alloc(2048 * sizeof(bh::NormChannel)));
-        // repack every 3x3 weight the MFMA conv reads
+        // every 3x3 weight in the order the convolution reads
         auto repack = [&](const std::string& n, int64_t ci, int64_t co) {
-            if (!bh::mfma_conv(ci, co) || e->rw.count(n + ".weight")) return;
             bf16_t* r = static_cast<bf16_t*>(e->alloc(co * ci * 9 * 2));
             bh::launch_repack3x3(e->at(n + ".weight"), r, co, ci, nullptr);
             e->rw[n + ".weight"] = r;
