@@ -310,8 +310,9 @@ struct ConvGeom {
     int up = 0;
 };
 // With `norm` the input is normalised on the way in: every value becomes norm_silu8's of its channel,
-// as launch_group_norm_apply would have stored it. With `stats` it also writes, for every run of four output channels, conv3x3_stats_rows pairs (sum,
-// sum of squares) in fp64 over disjoint sets of the stored pixels: stats[(run * rows + r) * 2 + {0, 1}].
+// as launch_group_norm_apply would have stored it. With `stats` it also writes, for every run of four output
+// channels, conv3x3_stats_rows pairs (sum, sum of squares) in fp64 over disjoint sets of the stored pixels:
+// stats[(run * rows + r) * 2 + {0, 1}].
 // 0 rows: the shape has no such sums.
 int64_t conv3x3_stats_rows(const ConvGeom& cv, int64_t c_out);
 void launch_conv3x3_bf16(const ConvGeom& cv, const bf16_t* wr, const bf16_t* bias, bf16_t* out,
@@ -335,8 +336,8 @@ bool gn_nhwc_supported(int64_t C, int64_t G);
 void launch_group_norm_channels(const bf16_t* x, int64_t S, int64_t C, int64_t G, float eps,
                                 const bf16_t* w, const bf16_t* b, GroupNormScratch& sc, hipStream_t s,
                                 int64_t stats_rows = 0);
-// The GroupNorm of x with them, then optionally SiLU, each rounded to bf16 as the reference stores
-// it. out may alias x.
+// The GroupNorm of x with them, rounded to bf16 as the reference stores it (norm8), or followed by SiLU, each
+// rounded to bf16, in the folded form of norm_silu8. out may alias x.
 void launch_group_norm_apply(const bf16_t* x, bf16_t* out, int64_t S, int64_t C, bool silu,
                              const GroupNormScratch& sc, hipStream_t s);
 // Stride-1 "same" convolution, channels-last, w in the checkpoint layout [co][ci][k][k], in the

@@ -26,7 +26,8 @@
 // With NORM the convolution reads the raw tensor and applies its GroupNorm and SiLU itself: each
 // producer wave normalises the patch rows it loaded, in LDS, as soon as they have landed, so the
 // normalised tensor is never written to or read from memory. A pixel is normalised once per patch
-// and chunk (1.27 times on average, once per 128 output channels) on waves that otherwise only issue
+// and chunk and 128 output channels, border included (1.27 times each on average with patches of 16 rows, 1.41
+// with 8, 1.69 with 4), on waves that otherwise only issue
 // loads, under the consumers' MFMAs; the ~10 vector instructions per value take issue slots from
 // them (512 -> 512 at 128 x 128: 57 -> 75 us with the raw tensor read in place of the normalised
 // one), less than the pass they replace as a whole: decode at 512px 3.32 -> 2.84 ms, at 1024px
@@ -527,7 +528,10 @@ void launch_conv(const ConvGeom& cv, const bf16_t* w, bf16_t* out, int64_t c_out
     a.tiles = patches(cv, MT) * a.tiles_n;
     int grid = min(a.tiles, device_cus() & ~7);
     if (grid < 8) grid = min(a.tiles, device_cus());
-    // The combinations the decoder and the single op use; null sums are skipped.
+    // The combinations the decoder and the single op use; null sums are skipped. Above 32 channels a tile is 128
+    // wide whatever the width: 136 or 144 channels multiply 256 columns, where tiles of 144 multiplied 144, and the op
+    // is still the shorter one (256 channels to 144 at 256 x 256: 92 -> 75 us; 512 to 144 at 192 x 192: 108 -> 97,
+    // the least gain of 77 such sizes; 512 to 288 at 256 x 256: 237 -> 185).
     if constexpr (NT == 8) {
         if (x.norm) {
             if (e.residual) k_conv3x3<MT, EPI_RESIDUAL, NT, true, true><<<grid, kWgThreads, 0, s>>>(a, e);

@@ -5,11 +5,12 @@
 //   - k_transpose       [R, C] -> [C, R] per batch: NCHW <-> NHWC at the stage's two ends, and
 //                       the reference's TransposeArgs op (ops.h:184-191);
 //   - GroupNorm         fp64 sums and sums of squares in a fixed order (from the convolution that
-//                       wrote the tensor, or one pass over it), applied with its SiLU (each
-//                       rounded to bf16 as the reference stores them, ops_cpu.cpp:186-224,
-//                       265-274) by a pass, or by the convolution that reads the tensor;
-//   - k_conv_direct     a convolution in the reference's summation order, for the layers too thin
-//                       for the MFMA tile (conv_in: 4 input channels; conv_out: 3 outputs);
+//                       wrote the tensor, or one pass over it), applied by a pass, or by the
+//                       convolution that reads the tensor; rounded to bf16 as the reference stores
+//                       it (ops_cpu.cpp:186-224), and with its SiLU both rounded, in the folded form
+//                       of norm_silu8 (common.h);
+//   - k_conv_direct     a convolution in the reference's summation order, for the single op where
+//                       the MFMA tile does not apply (the engine pads its two thin convolutions);
 //   - k_upsample_nchw   the reference's UpsampleArgs op (the engine fuses the upsample into the
 //                       next convolution's gather instead).
 // The convolutions are in conv.hip, the mid-block's attention in flash512.hip.

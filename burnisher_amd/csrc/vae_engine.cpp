@@ -3,9 +3,9 @@
 //
 // The reference runs the decoder NCHW and transposes around the mid-block attention. Here the
 // activation between ops is [pixels, channels] bf16 (NHWC, batch 1), chosen for gfx950:
-//   - a 3x3 convolution is an implicit GEMM on the MFMA tile kernel (gemm.hip): a k-tile is one
-//     tap x 64 input channels, i.e. 128 contiguous bytes of one neighbouring pixel;
-//   - the upsampler's nearest 2x upsample is folded into that gather (the conv reads pixel
+//   - a 3x3 convolution is an implicit GEMM over patches of the image on the MFMA cores (conv.hip),
+//     which normalises the tensor it reads and sums the one it writes for the next GroupNorm;
+//   - the upsampler's nearest 2x upsample is folded into its patch loads (the conv reads pixel
 //     (y/2, x/2)), so the 4x-larger upsampled tensor is never written (at 1024px it would be
 //     0.5 GB written and read back);
 //   - the resnet's "skip + conv2" is the residual epilogue of conv2, and the shortcut 1x1 conv
@@ -13,8 +13,9 @@
 //   - the mid-block attention reads its tokens in place: the reference's two transposes vanish.
 // Only the latent (4 channels) and the image (3 channels) change layout, at the two ends.
 //
-// Rounding follows the reference's graph: every op's output is stored in bf16, including
-// conv2 before its residual add (round_mid) and the GroupNorm output before its SiLU.
+// Rounding follows the reference's graph: every op's output is rounded to bf16, including
+// conv2 before its residual add (round_mid) and the GroupNorm output before its SiLU. Inside that
+// GroupNorm the multiplications are folded (norm_silu8, common.h), not the reference's sequence.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
