@@ -325,7 +325,7 @@ void launch_transpose_bf16(const bf16_t* in, bf16_t* out, int64_t batch, int64_t
                            hipStream_t s);
 // Device scratch of a GroupNorm: fp64 partial sums and the channels' statistics and affine.
 struct GroupNormScratch {
-    double* part = nullptr;           // 2 * 64 * max_chunks, or what conv3x3_stats_rows asks for
+    double* part = nullptr;           // 2 * groups * max_chunks, or what conv3x3_stats_rows asks for
     NormChannel* channels = nullptr;  // 2048 (the widest supported norm)
     int64_t max_chunks = 0;
 };

@@ -314,3 +314,35 @@ def test_vae_weights_from_a_checkpoint_and_the_decode_stage(hip, tmp_path):
     check_decode(to_bf16(img), want, "vae-decode stage")
     # loaded weights == host-rounded upload, byte for byte
     assert np.array_equal(to_bf16(img), decode(wl))
+
+
+def test_decoder_creation_time_beside_another(hip):
+    """A decoder's creation where one is alive (its buffers come from the runtime's allocator, which once
+    made an allocation of 2 MiB take four times the whole creation): a small latent against a large one."""
+    import time
+    import torch
+    import burnisher_amd as bh
+    wl = make_vae_workload(SDXL_VAE, latent_hw=16, seed=5)
+    tensors, _ = wl.to_device()
+    cfg = config_struct(wl.cfg)
+    w, keep = wl.table(tensors)
+
+    def create(hw):
+        h = ctypes.c_void_p()
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        bh.call("bh_vae_create", ctypes.byref(cfg), ctypes.byref(w), hw, ctypes.byref(h))
+        return h, time.perf_counter() - t
+
+    def median_ms(hw):
+        alive, _ = create(hw)
+        ms = []
+        for _ in range(7):
+            h, s = create(hw)
+            ms.append(s * 1e3)
+            bh.lib().bh_vae_destroy(h)
+        bh.lib().bh_vae_destroy(alive)
+        return float(np.median(ms))
+
+    small, large = median_ms(16), median_ms(64)
+    assert small < 1.6 * large, f"latent 16: {small:.2f} ms, 64: {large:.2f}"
