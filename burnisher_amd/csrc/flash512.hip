@@ -150,7 +150,7 @@ __global__ void __launch_bounds__(256, 1) k_flash512(Args a) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         dma_v(smem + 2 * kStage, a, b0, i, wave, lane);
-        dma_k(smem + kStage, a, min(b0 + 1, nblk_all - 1), i, wave, lane);
+        if (b0 + 1 < b1) dma_k(smem + kStage, a, b0 + 1, i, wave, lane);
     }
     bf16x8_t qf[2][16];
 #pragma unroll
@@ -236,10 +236,8 @@ __global__ void __launch_bounds__(256, 1) k_flash512(Args a) {
         }
 #pragma unroll
         for (int e = 0; e < 16; ++e) scale(s, e, b0);
-        {
-            const float mx[2] = {block_max(s, 0), block_max(s, 1)};
-            rescale(mx);
-        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) m[u] = fmaxf(m[u], block_max(s, u));   // no sums to rescale yet
         for (int j = b0; j + 1 < b1; ++j) {
             const int x = (j - b0) & 1;
             join();   // K of block j + 1 and V^T of block j are complete; K of j and V^T of j - 1 are free
@@ -328,26 +326,43 @@ __global__ void __launch_bounds__(256, 1) k_flash512(Args a) {
 }
 
 // out[q] = sum_s 2^(m_s - M) o_s[q] / sum_s 2^(m_s - M) l_s over the splits in order. A wave per
-// query, eight dims a lane; bound by the partials it reads.
+// query, eight dims a lane; bound by the partials it reads, or by the latency of its loads where there are few: lane s
+// holds split s's maximum and denominator (one load for all of them), and kAtOnce splits' sums are requested at once.
+template <int kAtOnce>
 __global__ void __launch_bounds__(256) k_flash512_combine(const float* __restrict__ part, bf16_t* __restrict__ out,
                                                           int S, int splits) {
     const int q = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (q >= S) return;
     const float* ml = part + static_cast<int64_t>(splits) * S * kD;
-    float top = -INFINITY;
-    for (int s = 0; s < splits; ++s) top = fmaxf(top, ml[(static_cast<int64_t>(s) * S + q) * 2]);
+    const float2 mine = *reinterpret_cast<const float2*>(ml + (static_cast<int64_t>(min(lane, splits - 1)) * S + q) * 2);
+    f32x4_t x[kAtOnce], y[kAtOnce];
+    auto request = [&](int s0) {   // splits past the last are read again, unused
+#pragma unroll
+        for (int i = 0; i < kAtOnce; ++i) {
+            const float* row = part + (static_cast<int64_t>(min(s0 + i, splits - 1)) * S + q) * kD + lane * 8;
+            x[i] = *reinterpret_cast<const f32x4_t*>(row);
+            y[i] = *reinterpret_cast<const f32x4_t*>(row + 4);
+        }
+    };
+    request(0);
+    float top = mine.x;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) top = fmaxf(top, __shfl_xor(top, o, 64));
+    const float weight = exp2f(mine.x - top);
     f32x4_t lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
     float den = 0.f;
-    for (int s = 0; s < splits; ++s) {
-        const int64_t row = static_cast<int64_t>(s) * S + q;
-        const float w = exp2f(ml[row * 2] - top);
-        const f32x4_t x = *reinterpret_cast<const f32x4_t*>(part + row * kD + lane * 8);
-        const f32x4_t y = *reinterpret_cast<const f32x4_t*>(part + row * kD + lane * 8 + 4);
-        den += w * ml[row * 2 + 1];
+    for (int s0 = 0; s0 < splits; s0 += kAtOnce) {
+        if (s0 > 0) request(s0);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            lo[t] += w * x[t];
-            hi[t] += w * y[t];
+        for (int i = 0; i < kAtOnce; ++i) {
+            if (s0 + i >= splits) break;
+            const float w = __shfl(weight, s0 + i, 64);
+            den += w * __shfl(mine.y, s0 + i, 64);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                lo[t] += w * x[i][t];
+                hi[t] += w * y[i][t];
+            }
         }
     }
     const float r = __frcp_rn(den);
@@ -404,8 +419,9 @@ int64_t flash512_scratch_elems(int64_t S, int splits) {
 }
 
 // The key splits of S tokens, at most what `scratch_bytes` holds beside V^T: the least estimated
-// time. A workgroup takes about 1.3 us per block and ~4 us at its ends; the partials of one split
-// are S x 2 KiB written and read at ~4.5 TB/s.
+// time. A workgroup takes about 1.7 us per block (4096 tokens in 1, 2 and 4 splits: 224, 128 and 79 us) and
+// ~4 us at its ends; the combine ~3 us, and the partials of one split are S x 2 KiB written and read at
+// ~4.5 TB/s. Few tokens: 64 in 1 and 2 splits 14.5 and 15.1 us, 100 in 1 and 4 20.7 and 18.4.
 int flash512_splits(int64_t S, int64_t scratch_bytes) {
     const int64_t cus = device_cus(), qb = (S + kQ - 1) / kQ, nblk = (S + kKv - 1) / kKv;
     int best = 1;
@@ -413,8 +429,8 @@ int flash512_splits(int64_t S, int64_t scratch_bytes) {
     for (int sp = 1; sp <= kMaxSplits && sp <= nblk; ++sp) {
         if (sp > 1 && flash512_scratch_elems(S, sp) * 2 > scratch_bytes) break;
         const int64_t rounds = (qb * sp + cus - 1) / cus;
-        const double cost = rounds * (((nblk + sp - 1) / sp) * 1.3 + 4.0) +
-                            (sp > 1 ? 4.0 + sp * static_cast<double>(S) * 4096.0 / 4.5e6 : 0.0);
+        const double cost = rounds * (((nblk + sp - 1) / sp) * 1.7 + 4.0) +
+                            (sp > 1 ? 3.0 + sp * static_cast<double>(S) * 4096.0 / 4.5e6 : 0.0);
         if (best_cost < 0 || cost < best_cost) {
             best = sp;
             best_cost = cost;
@@ -438,7 +454,10 @@ void launch_attention512(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16
            (scale > 0.0f ? scale : 1.0f / std::sqrt(static_cast<float>(kD))) * 1.4426950408889634f};
     ProfileScope ps(K_ATTN_SELF, s, 4.0 * static_cast<double>(S) * S * kD);
     k_flash512<<<static_cast<unsigned>(a.qblocks) * splits, 256, 0, s>>>(a);
-    if (splits > 1) k_flash512_combine<<<static_cast<unsigned>((S + 3) / 4), 256, 0, s>>>(a.part, out, n, splits);
+    if (splits > 1) {
+        auto* combine = splits == 2 ? &k_flash512_combine<2> : splits <= 4 ? &k_flash512_combine<4> : &k_flash512_combine<8>;
+        combine<<<static_cast<unsigned>((S + 3) / 4), 256, 0, s>>>(a.part, out, n, splits);
+    }
     launch_check("attention (head_dim 512)");
 }
 

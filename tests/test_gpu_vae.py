@@ -346,3 +346,51 @@ def test_decoder_creation_time_beside_another(hip):
 
     small, large = median_ms(16), median_ms(64)
     assert small < 1.6 * large, f"latent 16: {small:.2f} ms, 64: {large:.2f}"
+
+
+@pytest.mark.parametrize("S", [64, 81, 100, 128, 144, 289])
+def test_attention_head_dim_512_few_tokens(hip, S):
+    """Two to ten blocks of keys, in one, three, four and more splits (every count of sums that the combine
+    requests at once), against the oracle and, for a constant V, exactly V."""
+    rng = np.random.default_rng(61)
+    q, k, v = (randn_bf16(rng, (1, S, 1, 512), sc) for sc in (4.0, 1.0, 1.0))
+    want = np.zeros_like(q)
+    st("stock_attention", addr(q), addr(k), addr(v), addr(want), 1, 1, S, S, 512, 0.0, None, None, F32,
+       BF16, 0, 0)
+    dq, dk, dv, out = dev(q), dev(k), dev(v), empty((1, S, 1, 512))
+    call("bh_attention", dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), out.data_ptr(), 1, 1,
+         S, S, 512, 0.0, None, None, F32, BF16, None)
+    assert_within(from_bf16(host(out)), from_bf16(want), "attention", f"head_dim 512 S={S}")
+    dv.fill_(1.5)
+    call("bh_attention", dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), out.data_ptr(), 1, 1,
+         S, S, 512, 0.0, None, None, F32, BF16, None)
+    assert np.all(from_bf16(host(out)) == 1.5)
+
+
+def test_attention_head_dim_512_of_one_block_has_no_rescale(hip):
+    # Rescaling the sums that are still zero at the first block cost a quarter of the call at few tokens: one
+    # token against sixteen at head_dim 128, whose kernel is a chain of the same length.
+    import torch
+
+    def us(heads, D, S):
+        q, k, v, out = (torch.zeros((1, S, heads, D), dtype=torch.bfloat16, device="cuda") for _ in range(4))
+        graph = torch.cuda.CUDAGraph()
+        args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), 1, heads, S, S, D, 0.0, None, None, F32, BF16)
+        call("bh_attention", *args, None)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph):
+            for _ in range(100):
+                call("bh_attention", *args, torch.cuda.current_stream().cuda_stream)
+        t = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        best = 1e9
+        for _ in range(8):
+            t[0].record()
+            graph.replay()
+            t[1].record()
+            torch.cuda.synchronize()
+            best = min(best, t[0].elapsed_time(t[1]) * 10)
+        return best
+
+    one, block = us(1, 512, 1), us(4, 128, 16)
+    print(f"head_dim 512, one token {one:.2f} us; head_dim 128, 16 tokens {block:.2f}")
+    assert one < 1.12 * block
