@@ -501,10 +501,8 @@ void launch_tn(const bf16_t* a, const bf16_t* b, bf16_t* out, int64_t m, int64_t
     // Only the staged epilogue of a workgroup's last tile knows the narrow widths and a V^T store of short
     // tiles: a second tile would be lost.
     if constexpr (NT < 8) require(grid == tiles, "gemm: a tile narrower than 128 columns is its workgroup's only one");
-    if constexpr (MT < kMaxMT)
-        if (e.vt)
-            require(MT <= 2 && NT == kNT && grid == tiles,
-                    "gemm: a transposed V store takes 144-wide tiles of 256 rows, or of 64 or 128 one to a workgroup");
+    if constexpr (MODE == EPI_VT && MT < kMaxMT)
+        require(grid == tiles, "gemm: a transposed V store of short tiles takes one tile to a workgroup");
     k_gemm_tn<ACT, MODE, MT, NT><<<grid, kWgThreads, 0, s>>>(a, b, out, m, n, k, e, tiles_m, tiles_n, 16 / MT);
 }
 
@@ -873,8 +871,8 @@ void launch_gemm_bf16(const bf16_t* a, const bf16_t* b, const bf16_t* bias, bf16
           ep.residual, ep.gate, ep.gate_rows > 0 ? ep.gate_rows : 1, ep.ld_out > 0 ? ep.ld_out : n, 0,
           ep.vt, ep.vt_period, ep.vt_col0, ep.vt_seq, ep.vt_ld, ep.vt_heads, ep.vt_dim};
     if (ep.vt) {
-        require(!ep.residual && !ep.row_add && !ep.round_mid,
-                "gemm: the transposed V store has no residual or row-add epilogue");
+        require(!ep.residual && !ep.row_add && !ep.round_mid && ep.act == 0,
+                "gemm: the transposed V store has no activation, residual or row-add epilogue");
         require(ep.vt_period > 0 && ep.vt_period % BN == 0 && ep.vt_col0 % BN == 0 &&
                     ep.vt_col0 < ep.vt_period && ep.vt_seq > 0 && m % ep.vt_seq == 0 &&
                     ep.vt_ld >= ep.vt_seq && ep.vt_heads > 0 && ep.vt_dim > 0 &&
@@ -965,7 +963,16 @@ void launch_gemm_bf16(const bf16_t* a, const bf16_t* b, const bf16_t* bias, bf16
         return;
     }
     ProfileScope ps(K_GEMM, s, flops, gemm_subclass());
-    const TileShape mt = ep.vt ? vt_tile_shape(m, n) : gemm_tile_shape(m, n);
+    if (ep.vt) {
+        switch (vt_tile_shape(m, n).mt) {
+            case 1: launch_tn<0, EPI_VT, 1>(a, b, out, m, n, k, e, s); break;
+            case 2: launch_tn<0, EPI_VT, 2>(a, b, out, m, n, k, e, s); break;
+            default: launch_tn<0, EPI_VT>(a, b, out, m, n, k, e, s); break;
+        }
+        launch_check("gemm (mfma, transposed V)");
+        return;
+    }
+    const TileShape mt = gemm_tile_shape(m, n);
     switch (ep.act) {
         case 1: launch_tn_mt<1>(mt, mode, a, b, out, m, n, k, e, s); break;
         case 2: launch_tn_mt<2>(mt, mode, a, b, out, m, n, k, e, s); break;
