@@ -24,6 +24,7 @@
 // skipping it changes nothing.
 #include "common.h"
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <mutex>
@@ -608,7 +609,11 @@ void launch_attention_bf16(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf
         return vt_buf;
     };
     if (plan.kind == AttnPlan::FLASH512) {
-        bf16_t* vt = vt_for(plan.vt_elems);
+        // The partials of few tokens can need more than those of many (16384 tokens split in one, 4096 in seven),
+        // so the shared workspace takes the limit of the splits at once: a call after one of more tokens
+        // never grows it, nor frees it under a captured graph.
+        bf16_t* vt = vt_buf ? vt_for(plan.vt_elems)
+                            : vt_for(std::max<int64_t>(plan.vt_elems, kNoAllocScratchBytes / sizeof(bf16_t)));
         const int sp = flash512_splits(sh.q_len, kNoAllocScratchBytes);
         for (int64_t b = 0; b < sh.batch; ++b) {
             const int64_t off = b * sh.q_len * 512;

@@ -394,3 +394,35 @@ def test_attention_head_dim_512_of_one_block_has_no_rescale(hip):
     one, block = us(1, 512, 1), us(4, 128, 16)
     print(f"head_dim 512, one token {one:.2f} us; head_dim 128, 16 tokens {block:.2f}")
     assert one < 1.12 * block
+
+
+def test_attention_head_dim_512_captures_fewer_tokens_after_more(hip):
+    """A graph of a call whose key splits need more scratch than the warmed-up call of more tokens did: the
+    shared workspace must not grow during the capture, and every replay equals the eager call."""
+    import torch
+
+    def operands(S):
+        q, k, v = (torch.randn((1, S, 1, 512), device="cuda").to(torch.bfloat16) for _ in range(3))
+        return q, k, v, torch.empty_like(q)
+
+    def attend(t, stream):
+        S = t[0].shape[1]
+        call("bh_attention", *(x.data_ptr() for x in t), 1, 1, S, S, 512, 0.0, None, None, F32, BF16, stream)
+
+    many, few = operands(16384), operands(4096)
+    attend(many, None)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        attend(few, torch.cuda.current_stream().cuda_stream)
+    got = []
+    for _ in range(3):
+        few[3].zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        got.append(host(few[3]))
+        attend(many, None)   # the program's own eager work between the replays
+        torch.cuda.synchronize()
+    attend(few, None)
+    want = host(few[3])
+    assert all(np.array_equal(g, want) for g in got)
