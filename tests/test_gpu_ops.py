@@ -289,10 +289,9 @@ def test_gemm_small_k_few_columns_cost_less(hip):
 
 @pytest.mark.parametrize("B,N_tok", [(2, 1024), (7, 143)], ids=["whole_bands", "ragged_band"])
 def test_gemm_small_k_fused_epilogues(hip, B, N_tok):
-    # K = 16, the patch embedding's in_channels * patch^2: the register-weight kernel. Whole bands
-    # of rows take the path that issues every load of the band before its first store (plain and
-    # row-add stores); M = 1001 leaves a ragged last band, which walks its rows one at a time, as
-    # do the residual epilogues.
+    # K = 16, the patch embedding's in_channels * patch^2: the plain and row-add stores on a wave over 128
+    # columns, in whole bands of rows and with a ragged last one (M = 1001), and the residual epilogues on
+    # the register-weight kernel, a row at a time.
     import burnisher_amd as bh
     import ctypes
     d, K = 1152, 16

@@ -190,7 +190,7 @@ def test_attention_head_dim_512_matches_oracle(hip, S):
 @pytest.mark.parametrize("S,spread", [(1, 1.0), (33, 8.0), (128, 8.0), (129, 1.0), (1055, 8.0), (2048, 1.0)])
 def test_attention_head_dim_512_splits_and_rescales(hip, S, spread):
     """One key to 64 blocks of 32: a single block, ragged last blocks and query blocks, key splits
-    (from a few hundred tokens on), and scores spread wide enough (standard deviation 8) that the
+    (from eighty tokens on), and scores spread wide enough (standard deviation 8) that the
     running maximum moves in most blocks and splits carry very different maxima."""
     q, k, v = (randn_bf16(RNG, (1, S, 1, 512), sc) for sc in (spread, 1.0, 1.0))
     want = np.zeros_like(q)
@@ -393,7 +393,7 @@ def test_attention_head_dim_512_of_one_block_has_no_rescale(hip):
 
     one, block = us(1, 512, 1), us(4, 128, 16)
     print(f"head_dim 512, one token {one:.2f} us; head_dim 128, 16 tokens {block:.2f}")
-    assert one < 1.12 * block
+    assert one < 1.17 * block
 
 
 def test_attention_head_dim_512_captures_fewer_tokens_after_more(hip):
